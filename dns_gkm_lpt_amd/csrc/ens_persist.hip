@@ -137,7 +137,7 @@ __device__ __forceinline__ void zpass_item(const PersistStep& a, int i)
 template <bool MIX>
 __global__ __launch_bounds__(256, 2) void ens_step_kernel(PersistStep a)
 {
-    __shared__ double lds[kSweepLdsMax];
+    __shared__ double lds[kSweepLdsMax<MIX>];
     __shared__ int failed, slot;
     // a launch after a timed-out one (same run, flag not yet cleared by the
     // host) does nothing; thread 0 reads the flag for the whole workgroup

@@ -112,9 +112,11 @@ gkm::SweepArgs sweep_args(const gkm_ctx* c, int dir, int mode)
     a.nc = c->nc;
     a.dx = c->dx;
     a.inv_dx = 1.0 / c->dx;
-    a.g = c->gas;
+    a.two_idx = 2.0 * a.inv_dx;
+    a.half_idx = 0.5 * a.inv_dx;
+    a.g = gkm::gas_const(c->gas);
     a.tile = c->tile[dir];
-    a.seg = gkm::sweep_seg_len(dir, c->nc, a.tile, c->slots);
+    a.seg = gkm::sweep_seg_len(dir, c->nc, a.tile, c->slots, c->cfg.precision == GKM_MIXED);
     a.nseg = gkm::sweep_nseg(c->nc, a.seg);
     a.mode = mode;
     return a;
@@ -558,7 +560,7 @@ int gkm_autotune(gkm_ctx* c, int reps, int tile[3], double ms[9])
             }
             gkm::SweepArgs a = sweep_args(c, dir, dir);
             a.tile = v;
-            a.seg = gkm::sweep_seg_len(dir, c->nc, v, c->slots);
+            a.seg = gkm::sweep_seg_len(dir, c->nc, v, c->slots, mixed);
             a.nseg = gkm::sweep_nseg(c->nc, a.seg);
             // dW is scratch and Wout is the next state's buffer: the resident state is not changed
             hipError_t e = gkm::launch_sweep(dir, a, mixed, c->stream);  // warm-up
@@ -1108,9 +1110,11 @@ gkm::SweepArgs ens_sweep_args(const gkm_ctx* c, int p, int d, int v)
     a.nc = c->nc;
     a.dx = c->dx;
     a.inv_dx = 1.0 / c->dx;
-    a.g = c->gas;
+    a.two_idx = 2.0 * a.inv_dx;
+    a.half_idx = 0.5 * a.inv_dx;
+    a.g = gkm::gas_const(c->gas);
     a.tile = v;
-    a.seg = gkm::sweep_seg_len(d, c->nc, v, 0);
+    a.seg = gkm::sweep_seg_len(d, c->nc, v, 0, c->cfg.precision == GKM_MIXED);
     a.nseg = gkm::sweep_nseg(c->nc, a.seg);
     a.mode = d;
     return a;
@@ -1136,6 +1140,7 @@ int ens_build(gkm_ensemble* e, const int t[3])
         // instead of the long ones trailing it: the persistent step hands the
         // pencils out in this order (64-member workload: 6.62 -> 6.42 ms per
         // step); the per-phase launches measured the same either way
+        const bool mixed = e->mem[0]->cfg.precision == GKM_MIXED;  // members share the precision
         std::vector<int> order(n);
         std::vector<int> seg(n);
         for (int m = 0; m < n; m++) {
@@ -1148,8 +1153,8 @@ int ens_build(gkm_ensemble* e, const int t[3])
             first[(size_t)d * (n + 1) + k] = acc;
             for (int p = 0; p < 2; p++) args[((size_t)p * 3 + d) * n + k] = ens_sweep_args(e->mem[m], p, d, t[d]);
             const gkm::SweepArgs& a = args[(size_t)d * n + k];
-            acc += gkm::sweep_blocks(d, a.nc, t[d], a.seg);
-            exact = exact && gkm::sweep_exact(d, t[d], a.nc, a.seg);
+            acc += gkm::sweep_blocks(d, a.nc, t[d], a.seg, mixed);
+            exact = exact && gkm::sweep_exact(d, t[d], a.nc, a.seg, mixed);
         }
         first[(size_t)d * (n + 1) + n] = acc;
         e->nblk[d] = acc;

@@ -123,14 +123,13 @@ __host__ __device__ __forceinline__ void slope_from_lab(TE b0, TE b1, TE b2, TE 
 // Each value is fetched where it is used, so a caller that keeps them in LDS or
 // cache does not hold them in registers across the whole flux.
 // tau: collision time of the left cell; the pressure-jump term is added here.
-template <typename TE, typename TS, typename IN>
-__host__ __device__ __forceinline__ void gks_flux_tf(const IN& in, TE tau, TE dt, TE dx, const Gas<TE>& g, TE F[5])
+template <typename TE, typename TS, typename IN, typename G>
+__host__ __device__ __forceinline__ void gks_flux_tf(const IN& in, TE tau, TE dt, TE dx, const G& g, TE F[5])
 {
     const TE isqpi = TE(0.5641895835477562869480794515607726);  // 1/sqrt(pi)
-    const TE kp2e = TE(g.K + 2);
-    const TS kp2 = TS(g.K + 2), kp3 = TS(g.K + 3), kp4 = TS(g.K + 4);
-    const TS ikp3 = TS(1) / kp3;
-    const TS inv_prn = (TS)g.inv_prn;
+    const TE kp2e = gas_k<TE>(g).kp2;
+    const KConst<TS> kc = gas_k<TS>(g);
+    const TS kp2 = kc.kp2, kp3 = kc.kp3, kp4 = kc.kp4, ikp3 = kc.ikp3, inv_prn = kc.inv_prn;
 
     Maxw<TE> L, R;
     {

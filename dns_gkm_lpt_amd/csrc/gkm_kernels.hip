@@ -7,6 +7,7 @@
 // flux differences are formed in LDS and accumulated per cell.  Interface
 // states and fluxes never round-trip HBM.
 #include "gkm_kernels.hpp"
+#include "gkm_pair.hpp"
 #include "gkm_sweep.hpp"
 
 namespace gkm {
@@ -65,12 +66,15 @@ bool sweep_grid_ok(int nc)
     return nc >= 16 && sweep_first_tile(0, nc) >= 0 && sweep_first_tile(1, nc) >= 0 && sweep_first_tile(2, nc) >= 0;
 }
 
-int sweep_seg_len(int dir, int nc, int tile, int slots)
+static const int* tile_shape(int dir, int tile, bool mixed) { return mixed ? kTiles[dir][tile] : kTilesPair[dir][tile]; }
+
+int sweep_seg_len(int dir, int nc, int tile, int slots, bool mixed)
 {
     // faces per workgroup along the sweep axis (a multiple of CN); a segment
     // costs seg/CN chunks plus one lead-in chunk (the face before the segment).
     if (!sweep_tile_ok(dir, tile, nc)) return 0;
-    const int CN = kTiles[dir][tile][0], CA = kTiles[dir][tile][1], CB = kTiles[dir][tile][2];
+    const int* t = tile_shape(dir, tile, mixed);
+    const int CN = t[0], CA = t[1], CB = t[2];
     const long pencils = (long)cdiv(nc, CA) * cdiv(nc, CB);
     const int lchunks = cdiv(nc, CN);  // chunks of a whole line
     if (slots > 0) {
@@ -106,15 +110,16 @@ int sweep_seg_len(int dir, int nc, int tile, int slots)
 template <int DIR, int V>
 static hipError_t launch_tile(const SweepArgs& a, bool mixed, hipStream_t s)
 {
-    constexpr int CN = Tile<DIR, V>::CN, CA = Tile<DIR, V>::CA, CB = Tile<DIR, V>::CB;
+    const int* t = tile_shape(DIR, V, mixed);
+    const int CN = t[0], CA = t[1], CB = t[2];
     if (!sweep_tile_ok(DIR, V, a.nc) || a.seg <= 0 || a.seg % CN || a.nseg != cdiv(a.nc, a.seg))
         return hipErrorInvalidValue;
     const long nblk = (long)cdiv(a.nc, CA) * cdiv(a.nc, CB) * a.nseg;
     // the compensated update is the mixed z sweep's (an FP64 context has no carry)
     if ((a.cmp_out != nullptr) != (a.cmp_in != nullptr) || (a.cmp_out && !mixed)) return hipErrorInvalidValue;
-    const bool gen = !sweep_exact(DIR, V, a.nc, a.seg);  // some workgroup reaches past the grid
+    const bool gen = !sweep_exact(DIR, V, a.nc, a.seg, mixed);  // some workgroup reaches past the grid
     const bool cmp = a.cmp_out && a.mode == 2;
-    const dim3 grid((unsigned)nblk), block(CN * CA * CB);
+    const dim3 grid((unsigned)nblk), block(256);
     if (mixed) {
         if constexpr (DIR == 2) {
             if (cmp) {
@@ -152,17 +157,18 @@ hipError_t launch_sweep(int dir, const SweepArgs& a, bool mixed, hipStream_t s)
     return hipErrorInvalidValue;
 }
 
-int sweep_blocks(int dir, int nc, int tile, int seg)
+int sweep_blocks(int dir, int nc, int tile, int seg, bool mixed)
 {
     if (!sweep_tile_ok(dir, tile, nc) || seg <= 0) return 0;
-    const int CA = kTiles[dir][tile][1], CB = kTiles[dir][tile][2];
-    return cdiv(nc, CA) * cdiv(nc, CB) * cdiv(nc, seg);
+    const int* t = tile_shape(dir, tile, mixed);
+    return cdiv(nc, t[1]) * cdiv(nc, t[2]) * cdiv(nc, seg);
 }
 
-bool sweep_exact(int dir, int tile, int nc, int seg)
+bool sweep_exact(int dir, int tile, int nc, int seg, bool mixed)
 {
     if (!sweep_tile_ok(dir, tile, nc) || seg <= 0) return false;
-    return nc % kTiles[dir][tile][1] == 0 && nc % kTiles[dir][tile][2] == 0 && nc % seg == 0;
+    const int* t = tile_shape(dir, tile, mixed);
+    return nc % t[1] == 0 && nc % t[2] == 0 && nc % seg == 0;
 }
 
 template <int DIR, int V>
@@ -343,6 +349,43 @@ __global__ __launch_bounds__(64) void flux_batch_kernel(long n, const double* __
     for (int q = 0; q < 5; q++) F[5 * i + q] = (double)Fo[q];
 }
 
+// FP64: two threads per face, the sweeps' flux (gkm_pair.hpp)
+struct BatchSide {
+    double s[5], c[5], n[5], t[2][5];
+    __device__ double S(int q) const { return s[q]; }
+    __device__ double C(int q) const { return c[q]; }
+    __device__ double N(int q) const { return n[q]; }
+    __device__ double T(int k, int q) const { return t[k][q]; }
+};
+__global__ __launch_bounds__(64) void flux_batch_pair_kernel(long n, const double* __restrict__ in,
+                                                             const double* __restrict__ tau, double dt, double dx,
+                                                             GasK g, double* __restrict__ F)
+{
+    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const int side = (int)(t & 1);
+    const bool live = (t >> 1) < n;
+    const long i = live ? t >> 1 : n - 1;  // lanes past the end repeat the last face: the pair exchange needs them
+    const double* v = in + 50 * i;
+    BatchSide b;
+#pragma unroll
+    for (int q = 0; q < 5; q++) {
+        // side 1 in its mirrored frame: slots 2 and 3 and the tangential
+        // directions change places, slot 1 and the normal direction their sign
+        const int p = side && (q == 2 || q == 3) ? 5 - q : q;
+        const double m = side && q == 1 ? -1.0 : 1.0;
+        b.c[q] = m * v[5 * side + p];
+        b.s[q] = m * v[10 + 5 * side + p];
+        b.n[q] = (side ? -m : m) * v[20 + 5 * side + p];
+        b.t[0][q] = m * v[(side ? 45 : 30) + p];
+        b.t[1][q] = m * v[(side ? 35 : 40) + p];
+    }
+    double Fo[5];
+    gks_flux_pair(b, tau[i], dt, dx, g, PairSwap{}, Fo);
+    if (live && side == 0)
+#pragma unroll
+        for (int q = 0; q < 5; q++) F[5 * i + q] = Fo[q];
+}
+
 __global__ __launch_bounds__(64) void flux_batch_mixed_kernel(long n, const double* __restrict__ in,
                                                               const double* __restrict__ tau, double dt, double dx,
                                                               Gas<double> g, double* __restrict__ F)
@@ -408,7 +451,8 @@ hipError_t launch_flux_batch(long n, const double* in, const double* tau, double
     if (n <= 0) return hipSuccess;
     const unsigned blocks = (unsigned)((n + 63) / 64);
     if (precision == 0)
-        hipLaunchKernelGGL(flux_batch_kernel<double>, dim3(blocks), dim3(64), 0, s, n, in, tau, dt, dx, g, F);
+        hipLaunchKernelGGL(flux_batch_pair_kernel, dim3((unsigned)((2 * n + 63) / 64)), dim3(64), 0, s, n, in, tau, dt,
+                           dx, gas_const(g), F);
     else if (precision == 1)
         hipLaunchKernelGGL(flux_batch_mixed_kernel, dim3(blocks), dim3(64), 0, s, n, in, tau, dt, dx, g, F);
     else

@@ -26,8 +26,8 @@ struct SweepArgs {
     int nseg;            // nc / seg
     int mode;            // 0: dW = dF   1: dW += dF   2: Wout = W - (dW + dF)/dx
     int tile;            // tile shape variant, 0 .. kTileVariants-1
-    double dx, inv_dx;
-    Gas<double> g;
+    double dx, inv_dx, two_idx, half_idx;  // cell width, 1/dx, 2/dx, 1/(2 dx)
+    GasK g;
 };
 
 // Layout of the compensated update's FP32 carry, which only the z sweep's
@@ -54,14 +54,23 @@ constexpr int kTiles[3][kTileVariants][3] = {
     {{4, 4, 16}, {1, 16, 16}, {2, 8, 16}},
     {{16, 4, 4}, {4, 8, 8}, {8, 8, 4}},
 };
-template <int DIR, int V>
+// FP64 shapes: 128 faces, two threads each (gkm_pair.hpp).  The first of each
+// direction is the fastest or within 1 % of it at 64^3 and 256^3 (256^3: x 1.92-
+// 1.97, y 1.96-2.02, z 2.05-2.21 ms over the three).
+constexpr int kTilesPair[3][kTileVariants][3] = {
+    {{2, 8, 8}, {1, 8, 16}, {2, 4, 16}},
+    {{2, 8, 8}, {1, 8, 16}, {2, 4, 16}},
+    {{8, 4, 4}, {4, 4, 8}, {4, 8, 4}},
+};
+template <int DIR, int V, bool MIX>
 struct Tile {
-    static constexpr int CN = kTiles[DIR][V][0], CA = kTiles[DIR][V][1], CB = kTiles[DIR][V][2];
+    static constexpr const int* t = MIX ? kTiles[DIR][V] : kTilesPair[DIR][V];
+    static constexpr int CN = t[0], CA = t[1], CB = t[2];
 };
 
 hipError_t launch_sweep(int dir, const SweepArgs& a, bool mixed, hipStream_t s);
 // blocks of one grid's sweep launch for a tile variant and segment length
-int sweep_blocks(int dir, int nc, int tile, int seg);
+int sweep_blocks(int dir, int nc, int tile, int seg, bool mixed);
 // one launch sweeping every member of an ensemble: members[m] (device array) with
 // blocks [first[m], first[m+1]) of nblk = first[nmem]; one tile variant for all.
 // exact: the tile and segment divide every member's grid (sweep_exact);
@@ -70,10 +79,10 @@ int sweep_blocks(int dir, int nc, int tile, int seg);
 hipError_t launch_ens_sweep(int dir, int tile, const SweepArgs* members, const int* first, int nmem, int nblk,
                             bool mixed, bool exact, bool compensated, hipStream_t s);
 // the tile variant and the segment length divide nc: no workgroup reaches past the grid
-bool sweep_exact(int dir, int tile, int nc, int seg);
+bool sweep_exact(int dir, int tile, int nc, int seg, bool mixed);
 // faces per workgroup chosen for a grid: slots = concurrent workgroups of the
 // device for a single grid, 0 for the members of an ensemble
-int sweep_seg_len(int dir, int nc, int tile, int slots);
+int sweep_seg_len(int dir, int nc, int tile, int slots, bool mixed);
 // any nc in [16, 1024] has a tile variant per direction; a variant fits nc when
 // CN + 3 <= nc and CA, CB <= nc
 bool sweep_grid_ok(int nc);

@@ -29,6 +29,68 @@ struct Gas {
     int K;      // internal degrees of freedom (FlowField.cpp:42)
 };
 
+// Gas with the constants the sweeps form from it, computed once on the host: a
+// kernel then reads them as scalar arguments.  Formed in a kernel they are
+// uniform FP64 values, which gfx950 can only compute and keep in vector
+// registers (24 of the 256 a lane has, through the whole sweep).  The values
+// are those the expressions below give from a plain Gas.
+struct GasK : Gas<double> {
+    double gam1, gR, Rg, T110;    // gam - 1, (gam - 1)/R, R/(gam - 1), T0 + 110.4
+    double iT0, muT;              // 1/T0, mu0 (T0 + 110.4)
+    double kp2, kp3, kp4, ikp3;   // K + 2, K + 3, K + 4, 1/(K + 3)
+    float fkp2, fkp3, fkp4, fikp3, finv_prn;
+    float feps;
+};
+inline GasK gas_const(const Gas<double>& g)
+{
+    GasK k;
+    static_cast<Gas<double>&>(k) = g;
+    k.gam1 = g.gam - 1.0;
+    k.gR = (g.gam - 1.0) / g.R;
+    k.Rg = g.R / (g.gam - 1.0);
+    k.T110 = g.T0 + 110.4;
+    k.iT0 = 1.0 / g.T0;
+    k.muT = g.mu0 * k.T110;
+    k.kp2 = g.K + 2;
+    k.kp3 = g.K + 3;
+    k.kp4 = g.K + 4;
+    k.ikp3 = 1.0 / k.kp3;
+    k.fkp2 = (float)k.kp2;
+    k.fkp3 = (float)k.kp3;
+    k.fkp4 = (float)k.kp4;
+    k.fikp3 = 1.0f / k.fkp3;
+    k.finv_prn = (float)g.inv_prn;
+    k.feps = (float)g.eps;
+    return k;
+}
+template <typename T> __host__ __device__ __forceinline__ T gas_gam1(const Gas<T>& g) { return g.gam - T(1); }
+template <typename T> __host__ __device__ __forceinline__ T gas_gR(const Gas<T>& g) { return (g.gam - T(1)) / g.R; }
+template <typename T> __host__ __device__ __forceinline__ T gas_Rg(const Gas<T>& g) { return g.R / (g.gam - T(1)); }
+template <typename T> __host__ __device__ __forceinline__ T gas_T110(const Gas<T>& g) { return g.T0 + T(110.4); }
+template <typename T> __host__ __device__ __forceinline__ float gas_feps(const Gas<T>& g) { return (float)g.eps; }
+__host__ __device__ __forceinline__ double gas_gam1(const GasK& g) { return g.gam1; }
+__host__ __device__ __forceinline__ double gas_gR(const GasK& g) { return g.gR; }
+__host__ __device__ __forceinline__ double gas_Rg(const GasK& g) { return g.Rg; }
+__host__ __device__ __forceinline__ double gas_T110(const GasK& g) { return g.T110; }
+__host__ __device__ __forceinline__ float gas_feps(const GasK& g) { return g.feps; }
+// the flux's K + n constants in type T
+template <typename T>
+struct KConst {
+    T kp2, kp3, kp4, ikp3, inv_prn;
+};
+template <typename TS, typename T>
+__host__ __device__ __forceinline__ KConst<TS> gas_k(const Gas<T>& g)
+{
+    const TS kp3 = TS(g.K + 3);
+    return KConst<TS>{TS(g.K + 2), kp3, TS(g.K + 4), TS(1) / kp3, (TS)g.inv_prn};
+}
+template <typename TS>
+__host__ __device__ __forceinline__ KConst<TS> gas_k(const GasK& g)
+{
+    if constexpr (sizeof(TS) == 4) return KConst<TS>{g.fkp2, g.fkp3, g.fkp4, g.fikp3, g.finv_prn};
+    else return KConst<TS>{g.kp2, g.kp3, g.kp4, g.ikp3, g.inv_prn};
+}
+
 template <typename T>
 __host__ __device__ __forceinline__ T sq(T a) { return a * a; }
 
@@ -73,6 +135,59 @@ __host__ __device__ __forceinline__ double g_div<double>(double a, double b)
 #else
     return a / b;
 #endif
+}
+
+// The FP64 path's square root and exponential (gkm_pair.hpp).  The mixed path
+// keeps sqrt() and exp(): its FP32 terms turn a last-bit change of an FP64 input
+// into an FP32 rounding, and its results stay what they were.
+//
+// f_sqrt_inv: square root and its inverse together (the flux needs both): the
+// hardware's reciprocal root y, s = x y and h = y/2 refined by one coupled Newton
+// step (both errors squared), s by its residual x - s^2, 1/s by the residual of
+// s (1/s) = 1: 11 VALU instructions (8 for the root alone, 22 for sqrt() with its
+// scaling and special cases) within 1 ulp for normal x > 0; zero, negative,
+// infinite and NaN x give NaN (a state's lambda and temperature are positive
+// and finite, as for g_rcp).
+// f_exp: exp of the flux's arguments -z^2 and -dt/tau.  x = n ln 2 + r,
+// |r| <= ln 2 / 2 (ln 2 in two parts, n times the first exact), e^r =
+// 1 + r + r^2 q(r) with q of degree 9 interpolating (e^r - 1 - r)/r^2 on
+// Chebyshev points (dns_gkm_lpt_amd/erfcx_fit.py prints the coefficients;
+// 1.7e-17 relative), scaled by 2^n: 19 VALU instructions against 42, 1.4e-16
+// relative.  Arguments below -1000 give 0 as e^-1000 does.
+__host__ __device__ __forceinline__ void f_sqrt_inv(double x, double& s, double& is)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    const double y = __builtin_amdgcn_rsq(x);
+    s = x * y;
+    double h = 0.5 * y;
+    const double e = fma(-h, s, 0.5);
+    s = fma(s, e, s);
+    h = fma(h, e, h);
+    s = fma(fma(-s, s, x), h, s);
+    h += h;
+    is = fma(fma(-s, h, 1.0), h, h);
+#else
+    s = sqrt(x);
+    is = 1.0 / s;
+#endif
+}
+__host__ __device__ __forceinline__ double f_exp(double x)
+{
+    x = fmax(x, -1000.0);
+    const double n = rint(x * 1.4426950408889634);
+    double r = fma(-n, 0.6931471806019545, x);
+    r = fma(n, 4.2009150726810846e-11, r);
+    double q = 2.510038549551032e-08;
+    q = fma(q, r, 2.7620088445409746e-07);
+    q = fma(q, r, 2.7557268459997064e-06);
+    q = fma(q, r, 2.4801521295954376e-05);
+    q = fma(q, r, 0.00019841269863053618);
+    q = fma(q, r, 0.0013888888917213717);
+    q = fma(q, r, 0.008333333333330062);
+    q = fma(q, r, 0.04166666666662413);
+    q = fma(q, r, 0.16666666666666669);
+    q = fma(q, r, 0.5000000000000001);
+    return ldexp(fma(q * r, r, r) + 1.0, (int)n);
 }
 
 // 0.5 erfc(x) given E = exp(-x^2), which the half-space moments of a
@@ -225,6 +340,51 @@ __host__ __device__ __forceinline__ void weno_pair(T a, T b, T c, T d, T e, T f,
     }
 }
 
+// FP64: the same reconstructions from the cells' differences d_k, which both
+// sides of the face (and the next face of the line) share.  With u_k = t_k/3 of
+// the second differences t_k the four candidates are the base cell (c for the
+// left side, d for the right) plus d2/2 + u0, d2/2 + u1, (d3 - u2)/2,
+// d3 - d4/2 + u3, and the indicators' first-difference parts d2 + t0/2,
+// d2 + t1/2, d3 - t2/2, d4 - 3 t3/2; the right side is the mirror image (-d4,
+// -d3, -d2 for d2, d3, d4, t and u in reverse).  The weights are taken times 20
+// (1, 9, 9, 1), and eps joins the indicators' shared second-difference parts:
+// 95 operations for both sides of a variable instead of 134.  Every fused
+// multiply-add is written out and no other is formed: what two faces of a
+// thread share is then the same whichever of the two comes first.
+__host__ __device__ __forceinline__ double weno_offset(double D0, double D1, double D2, double D3, double q0, double q1,
+                                                       double q2, double q3)
+{
+#pragma clang fp contract(off)
+    // sum of d_k q_k/D_k over the sum of d_k/D_k, over common denominators
+    D3 = wmax(wmax(wmax(D0, D1), D2), D3);  // update.cpp:577-584
+    const double p01 = D0 * D1, p23 = D2 * D3;
+    const double w1 = 9.0 * D0, w2 = 9.0 * D3;
+    const double m = fma(w1, q1, D1 * q0), n = fma(w2, q2, D2 * q3);
+    return fma(p23, m, p01 * n) * g_rcp(fma(p23, D1 + w1, p01 * (w2 + D2)));
+}
+template <>
+__host__ __device__ __forceinline__ void weno_pair<double>(double a, double b, double c, double d, double e, double f,
+                                                           double eps, double& wl, double& wr)
+{
+#pragma clang fp contract(off)
+    const double d1 = b - a, d2 = c - b, d3 = d - c, d4 = e - d, d5 = f - e;
+    const double t0 = d2 - d1, t1 = d3 - d2, t2 = d4 - d3, t3 = d5 - d4;
+    const double k3 = 1.0 / 3.0, k13 = 13.0 / 12.0;
+    const double u0 = k3 * t0, u1 = k3 * t1, u2 = k3 * t2, u3 = k3 * t3;
+    const double K0 = fma(k13 * t0, t0, eps), K1 = fma(k13 * t1, t1, eps);
+    const double K2 = fma(k13 * t2, t2, eps), K3 = fma(k13 * t3, t3, eps);
+    {
+        const double h0 = fma(0.5, t0, d2), h1 = fma(0.5, t1, d2), h2 = fma(-0.5, t2, d3), h3 = fma(-1.5, t3, d4);
+        wl = c + weno_offset(fma(h0, h0, K0), fma(h1, h1, K1), fma(h2, h2, K2), fma(h3, h3, K3), fma(0.5, d2, u0),
+                             fma(0.5, d2, u1), 0.5 * (d3 - u2), fma(-0.5, d4, d3) + u3);
+    }
+    {
+        const double h0 = fma(-0.5, t3, d4), h1 = fma(-0.5, t2, d4), h2 = fma(0.5, t1, d3), h3 = fma(1.5, t0, d2);
+        wr = d + weno_offset(fma(h0, h0, K3), fma(h1, h1, K2), fma(h2, h2, K1), fma(h3, h3, K0), fma(-0.5, d4, u3),
+                             fma(-0.5, d4, u2), -0.5 * (d3 + u1), fma(0.5, d2, u0 - d3));
+    }
+}
+
 // temperature with (gam - 1)/R given (one division)
 template <typename T>
 __host__ __device__ __forceinline__ T temp_gr(const T W[5], T gR)
@@ -246,45 +406,54 @@ __host__ __device__ __forceinline__ T temp_of(const T W[5], T gam, T R)
 // R/(gam-1); both equal the reference's expressions up to rounding.
 // weno5 with the six cells' temperatures given (Tc[s] = temp_gr(S[s], (gam - 1)/R)):
 // two neighbouring faces of a line share five cells and their temperatures
-template <typename T>
-__host__ __device__ __forceinline__ void weno5_t(const T S[6][5], const T Tc[6], const Gas<T>& g, T Wl[5], T Wr[5])
+template <typename T, typename G>
+__host__ __device__ __forceinline__ void weno5_t(const T S[6][5], const T Tc[6], const G& g, T Wl[5], T Wr[5])
 {
 #pragma unroll
     for (int q = 0; q < 4; q++) weno_pair(S[0][q], S[1][q], S[2][q], S[3][q], S[4][q], S[5][q], g.eps, Wl[q], Wr[q]);
     T Tl, Tr;
     weno_pair(Tc[0], Tc[1], Tc[2], Tc[3], Tc[4], Tc[5], g.eps, Tl, Tr);
-    const T Rg = g.R / (g.gam - T(1));
+    const T Rg = gas_Rg(g);
     Wl[4] = Wl[0] * Rg * Tl + g_div(T(0.5) * (Wl[1] * Wl[1] + Wl[2] * Wl[2] + Wl[3] * Wl[3]), Wl[0]);
     Wr[4] = Wr[0] * Rg * Tr + g_div(T(0.5) * (Wr[1] * Wr[1] + Wr[2] * Wr[2] + Wr[3] * Wr[3]), Wr[0]);
 }
 
-template <typename T>
-__host__ __device__ __forceinline__ void weno5(const T S[6][5], const Gas<T>& g, T Wl[5], T Wr[5])
+template <typename T, typename G>
+__host__ __device__ __forceinline__ void weno5(const T S[6][5], const G& g, T Wl[5], T Wr[5])
 {
 #pragma unroll
     for (int q = 0; q < 4; q++) weno_pair(S[0][q], S[1][q], S[2][q], S[3][q], S[4][q], S[5][q], g.eps, Wl[q], Wr[q]);
-    const T gR = (g.gam - T(1)) / g.R;
+    const T gR = gas_gR(g);
     T Tc[6];
 #pragma unroll
     for (int s = 0; s < 6; s++) Tc[s] = temp_gr(S[s], gR);
     T Tl, Tr;
     weno_pair(Tc[0], Tc[1], Tc[2], Tc[3], Tc[4], Tc[5], g.eps, Tl, Tr);
-    const T Rg = g.R / (g.gam - T(1));
+    const T Rg = gas_Rg(g);
     Wl[4] = Wl[0] * Rg * Tl + g_div(T(0.5) * (Wl[1] * Wl[1] + Wl[2] * Wl[2] + Wl[3] * Wl[3]), Wl[0]);
     Wr[4] = Wr[0] * Rg * Tr + g_div(T(0.5) * (Wr[1] * Wr[1] + Wr[2] * Wr[2] + Wr[3] * Wr[3]), Wr[0]);
 }
 
 // collision time mu(T)/p of the face's left cell, Sutherland law (update.cpp:276-278)
-template <typename T>
-__host__ __device__ __forceinline__ T collision_time(const T W[5], const Gas<T>& g)
+template <typename T, typename G>
+__host__ __device__ __forceinline__ T collision_time(const T W[5], const G& g)
 {
     T ir = g_rcp(W[0]);
     T u = W[1] * ir, v = W[2] * ir, w = W[3] * ir;
-    T P = (W[0] * (g.gam - T(1))) * (W[4] * ir - T(0.5) * (u * u + v * v + w * w));
+    T P = (W[0] * gas_gam1(g)) * (W[4] * ir - T(0.5) * (u * u + v * v + w * w));
     T Tt = g_div(P, g.R * W[0]);
     T x = g_div(Tt, g.T0);
-    T mu = g_div(g.mu0 * (x * g_sqrt(x)) * (g.T0 + T(110.4)), Tt + T(110.4));
+    T mu = g_div(g.mu0 * (x * g_sqrt(x)) * gas_T110(g), Tt + T(110.4));
     return g_div(mu, P);
+}
+
+// the same from the cell's density and temperature: mu(T)/(rho R T), one division
+__host__ __device__ __forceinline__ double collision_time_t(double den, double T, const GasK& g)
+{
+    const double x = T * g.iT0;
+    double s, is;
+    f_sqrt_inv(x, s, is);
+    return g_div(g.muT * (x * s), (T + 110.4) * (den * g.R * T));
 }
 
 // ---------------------------------------------------------------------------
@@ -300,15 +469,15 @@ struct Maxw {
     T den, u, v, w, lam, i2l, e2, e4;
 };
 
-template <typename T>
-__host__ __device__ __forceinline__ void maxw_init(Maxw<T>& s, const T W[5], const Gas<T>& g)
+template <typename T, typename G>
+__host__ __device__ __forceinline__ void maxw_init(Maxw<T>& s, const T W[5], const G& g)
 {
     s.den = W[0];
     T ir = g_rcp(W[0]);
     s.u = W[1] * ir;
     s.v = W[2] * ir;
     s.w = W[3] * ir;
-    T P = (s.den * (g.gam - T(1))) * (W[4] * ir - T(0.5) * (s.u * s.u + s.v * s.v + s.w * s.w));
+    T P = (s.den * gas_gam1(g)) * (W[4] * ir - T(0.5) * (s.u * s.u + s.v * s.v + s.w * s.w));
     s.i2l = P * ir;  // 1/(2 lambda) = p/rho
     s.lam = T(0.5) * g_rcp(s.i2l);
     s.e2 = T(g.K) * s.i2l;
@@ -348,10 +517,11 @@ __host__ __device__ __forceinline__ void half_tab(T m, T i2l, T h0, T h1, T* h)
 // of both sides (the reconstruction is shift invariant: candidates are affine
 // with unit coefficient sum and the indicators see differences only).
 // weno5_mixed with the six cells' temperatures given (as weno5_t)
-__host__ __device__ __forceinline__ void weno5_mixed_t(const double S[6][5], const double Tc[6], const Gas<double>& g,
+template <typename G>
+__host__ __device__ __forceinline__ void weno5_mixed_t(const double S[6][5], const double Tc[6], const G& g,
                                                        double Wl[5], double Wr[5])
 {
-    const float eps = (float)g.eps;
+    const float eps = gas_feps(g);
 #pragma unroll
     for (int q = 0; q < 4; q++) {
         const double c = S[2][q];
@@ -365,15 +535,15 @@ __host__ __device__ __forceinline__ void weno5_mixed_t(const double S[6][5], con
     weno_pair<float>((float)(Tc[0] - Tc[2]), (float)(Tc[1] - Tc[2]), 0.f, (float)(Tc[3] - Tc[2]),
                      (float)(Tc[4] - Tc[2]), (float)(Tc[5] - Tc[2]), eps, l, r);
     const double Tl = Tc[2] + (double)l, Tr = Tc[2] + (double)r;
-    const double Rg = g.R / (g.gam - 1.0);
+    const double Rg = gas_Rg(g);
     Wl[4] = Wl[0] * Rg * Tl + g_div(0.5 * (Wl[1] * Wl[1] + Wl[2] * Wl[2] + Wl[3] * Wl[3]), Wl[0]);
     Wr[4] = Wr[0] * Rg * Tr + g_div(0.5 * (Wr[1] * Wr[1] + Wr[2] * Wr[2] + Wr[3] * Wr[3]), Wr[0]);
 }
 
-__host__ __device__ __forceinline__ void weno5_mixed(const double S[6][5], const Gas<double>& g, double Wl[5],
-                                                     double Wr[5])
+template <typename G>
+__host__ __device__ __forceinline__ void weno5_mixed(const double S[6][5], const G& g, double Wl[5], double Wr[5])
 {
-    const float eps = (float)g.eps;
+    const float eps = gas_feps(g);
 #pragma unroll
     for (int q = 0; q < 4; q++) {
         const double c = S[2][q];
@@ -383,7 +553,7 @@ __host__ __device__ __forceinline__ void weno5_mixed(const double S[6][5], const
         Wl[q] = c + (double)l;
         Wr[q] = c + (double)r;
     }
-    const double gR = (g.gam - 1.0) / g.R;
+    const double gR = gas_gR(g);
     double Tc[6];
 #pragma unroll
     for (int s = 0; s < 6; s++) Tc[s] = temp_gr<double>(S[s], gR);
@@ -391,7 +561,7 @@ __host__ __device__ __forceinline__ void weno5_mixed(const double S[6][5], const
     weno_pair<float>((float)(Tc[0] - Tc[2]), (float)(Tc[1] - Tc[2]), 0.f, (float)(Tc[3] - Tc[2]),
                      (float)(Tc[4] - Tc[2]), (float)(Tc[5] - Tc[2]), eps, l, r);
     const double Tl = Tc[2] + (double)l, Tr = Tc[2] + (double)r;
-    const double Rg = g.R / (g.gam - 1.0);
+    const double Rg = gas_Rg(g);
     Wl[4] = Wl[0] * Rg * Tl + g_div(0.5 * (Wl[1] * Wl[1] + Wl[2] * Wl[2] + Wl[3] * Wl[3]), Wl[0]);
     Wr[4] = Wr[0] * Rg * Tr + g_div(0.5 * (Wr[1] * Wr[1] + Wr[2] * Wr[2] + Wr[3] * Wr[3]), Wr[0]);
 }

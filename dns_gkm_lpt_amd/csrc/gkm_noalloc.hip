@@ -109,9 +109,11 @@ extern "C" int gkm_step_noalloc(const gkm_config* cfg, const double* W, double* 
         a.nc = nc;
         a.dx = gkm::config_dx(*cfg);
         a.inv_dx = 1.0 / a.dx;
-        a.g = gkm::config_gas(*cfg);
+        a.two_idx = 2.0 * a.inv_dx;
+        a.half_idx = 0.5 * a.inv_dx;
+        a.g = gkm::gas_const(gkm::config_gas(*cfg));
         a.tile = gkm::sweep_first_tile(dir, nc);  // a new context's tiles
-        a.seg = gkm::sweep_seg_len(dir, nc, a.tile, slots);
+        a.seg = gkm::sweep_seg_len(dir, nc, a.tile, slots, mixed);
         a.nseg = gkm::sweep_nseg(nc, a.seg);
         a.mode = dir;  // x: dW = dF, y: dW += dF, z: Wout = W - (dW + dF)/dx
         e = gkm::launch_sweep(dir, a, mixed, s);

@@ -47,6 +47,23 @@ def coefficients():
     return np.polynomial.chebyshev.cheb2poly(c)
 
 
+def exp_coefficients(degree=11):
+    """q of e^r = 1 + r + r^2 q(r), |r| <= ln 2 / 2, by interpolation on Chebyshev
+    points (kept in csrc/gkm_math.hpp's f_exp, lowest power first)."""
+    import mpmath as mp
+
+    mp.mp.dps = 50
+    n = degree - 1
+    h = mp.log(2) / 2 * mp.mpf("1.0001")
+    xs = [h * mp.cos(mp.pi * (j + mp.mpf(1) / 2) / n) for j in range(n)]
+    A, b = mp.matrix(n, n), mp.matrix(n, 1)
+    for i, x in enumerate(xs):
+        b[i] = (mp.exp(x) - 1 - x) / x ** 2
+        for k in range(n):
+            A[i, k] = x ** k
+    return [float(c) for c in mp.lu_solve(A, b)]
+
+
 def half_erfc(x, p):
     """0.5 erfc(x) in double precision, the device code's operation order."""
     t = abs(x)
@@ -68,6 +85,7 @@ def main(argv=None):
     for a in p:
         print(f"    {float(a)!r},")
     print("};")
+    print("exp:", ", ".join(repr(c) for c in exp_coefficients()))
     if "--check" in argv:
         import mpmath as mp
 
