@@ -19,6 +19,7 @@
 #include "adj_kernels.hpp"
 #include "gkm_config.hpp"
 #include "ens_persist.hpp"
+#include "host_copy.hpp"
 #include "gkm_kernels.hpp"
 #include "lpt_kernels.hpp"
 
@@ -47,6 +48,7 @@ struct gkm_ctx {
     int tile[3] = {0, 0, 0};       // sweep tile variant per direction
     int slots = 512;               // concurrent sweep workgroups: 2 per CU
     std::string err;
+    gkm::HostPipe pipe;            // copies of whole states and tracer arrays to and from the caller's memory
     // per-kernel timing
     bool timing = false;
     hipEvent_t ev[2] = {nullptr, nullptr};
@@ -209,6 +211,7 @@ void gkm_destroy(gkm_ctx* c)
     if (!c) return;
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     lpt::release(c->lpt);
+    c->pipe.release();
     (void)hipFree(c->adj_scratch);
     (void)hipFree(c->adj_vec[0]);
     (void)hipFree(c->adj_vec[1]);
@@ -275,11 +278,12 @@ int gkm_download_carry(gkm_ctx* c, float* out)
 int gkm_upload_state(gkm_ctx* c, const double* const W[5])
 {
     if (!c || !W) return fail(c, GKM_EINVAL, "null argument");
+    gkm::CopySeg seg[5];
     for (int q = 0; q < 5; q++) {
         if (!W[q]) return fail(c, GKM_EINVAL, "null state plane");
-        HIPCHK(c, hipMemcpyAsync(c->stage + q * c->padded, W[q], sizeof(double) * c->padded, hipMemcpyHostToDevice,
-                                 c->stream));
+        seg[q] = {const_cast<double*>(W[q]), c->stage + q * c->padded, sizeof(double) * c->padded};
     }
+    HIPCHK(c, c->pipe.to_device(seg, 5, c->stream));
     int rc = timed(c, 7, [&] { return gkm::launch_unpack(c->stage, c->W[c->cur], c->nc, c->stream); });
     if (rc) return rc;
     if (c->cmp[c->cur])  // a new state carries no rounding error
@@ -302,14 +306,14 @@ int gkm_download_state(gkm_ctx* c, double* const W[5])
 {
     if (!c || !W) return fail(c, GKM_EINVAL, "null argument");
     if (!c->have_state) return fail(c, GKM_ENOTREADY, "no state uploaded");
-    int rc = timed(c, 7, [&] { return gkm::launch_pack(c->W[c->cur], c->stage, c->nc, c->stream); });
-    if (rc) return rc;
+    gkm::CopySeg seg[5];
     for (int q = 0; q < 5; q++) {
         if (!W[q]) return fail(c, GKM_EINVAL, "null state plane");
-        HIPCHK(c, hipMemcpyAsync(W[q], c->stage + q * c->padded, sizeof(double) * c->padded, hipMemcpyDeviceToHost,
-                                 c->stream));
+        seg[q] = {W[q], c->stage + q * c->padded, sizeof(double) * c->padded};
     }
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    int rc = timed(c, 7, [&] { return gkm::launch_pack(c->W[c->cur], c->stage, c->nc, c->stream); });
+    if (rc) return rc;
+    HIPCHK(c, c->pipe.to_host(seg, 5, c->stream));
     return GKM_OK;
 }
 
@@ -380,8 +384,8 @@ int gkm_sweep_flux_diff(gkm_ctx* c, int dir, double dt, double* out)
     const gkm::SweepArgs a = sweep_args(c, dir, 0);
     int rc = timed(c, dir, [&] { return gkm::launch_sweep(dir, a, c->cfg.precision == GKM_MIXED, c->stream); });
     if (rc) return rc;
-    HIPCHK(c, hipMemcpyAsync(out, c->dW, sizeof(double) * 5 * c->plane, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    const gkm::CopySeg seg{out, c->dW, sizeof(double) * 5 * c->plane};
+    HIPCHK(c, c->pipe.to_host(&seg, 1, c->stream));
     return GKM_OK;
 }
 
@@ -410,7 +414,8 @@ int adj_prepare(gkm_ctx* c, double dt, int nstates)
 
 int vec_upload(gkm_ctx* c, const double* host_padded, double* dev)
 {
-    HIPCHK(c, hipMemcpyAsync(c->stage, host_padded, sizeof(double) * 5 * c->padded, hipMemcpyHostToDevice, c->stream));
+    const gkm::CopySeg seg{const_cast<double*>(host_padded), c->stage, sizeof(double) * 5 * c->padded};
+    HIPCHK(c, c->pipe.to_device(&seg, 1, c->stream));
     HIPCHK(c, gkm::launch_unpack(c->stage, dev, c->nc, c->stream));
     return GKM_OK;
 }
@@ -418,8 +423,8 @@ int vec_upload(gkm_ctx* c, const double* host_padded, double* dev)
 int vec_download(gkm_ctx* c, const double* dev, double* host_padded)
 {
     HIPCHK(c, gkm::launch_pack(dev, c->stage, c->nc, c->stream));
-    HIPCHK(c, hipMemcpyAsync(host_padded, c->stage, sizeof(double) * 5 * c->padded, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    const gkm::CopySeg seg{host_padded, c->stage, sizeof(double) * 5 * c->padded};
+    HIPCHK(c, c->pipe.to_host(&seg, 1, c->stream));
     return GKM_OK;
 }
 }  // namespace
@@ -823,7 +828,8 @@ int lpt_upload(gkm_ctx* c, long np, const double* pos)
         }
         pos = kept.data();
     }
-    HIPCHK(c, hipMemcpyAsync(L.pos, pos, sizeof(double) * 3 * np, hipMemcpyHostToDevice, c->stream));
+    const gkm::CopySeg seg{const_cast<double*>(pos), L.pos, sizeof(double) * 3 * np};
+    HIPCHK(c, c->pipe.to_device(&seg, 1, c->stream));
     HIPCHK(c, hipMemcpyAsync(L.tag, tags.data(), sizeof(int) * np, hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, lpt::sort_by_cell(L, geom_of(c), c->dx, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -834,9 +840,9 @@ int lpt_upload(gkm_ctx* c, long np, const double* pos)
 static int download_tag_order(gkm_ctx* c, const double* src, int width, double* host)
 {
     lpt::State& L = c->lpt;
-    HIPCHK(c, lpt::scatter_to_tags(L.np, L.tag, src, width, L.pos2, c->stream));
-    HIPCHK(c, hipMemcpyAsync(host, L.pos2, sizeof(double) * width * L.np, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    HIPCHK(c, lpt::scatter_to_tags(L.np, L.tag, src, width, width, L.pos2, c->stream));
+    const gkm::CopySeg seg{host, L.pos2, sizeof(double) * width * L.np};
+    HIPCHK(c, c->pipe.to_host(&seg, 1, c->stream));
     return GKM_OK;
 }
 
@@ -899,15 +905,14 @@ int lpt_sample(gkm_ctx* c, double* U, double* gU, double* gV, double* gW)
         rc = download_tag_order(c, L.U, 3, U);
         if (rc) return rc;
     }
-    if (gU || gV || gW) {
-        std::vector<double> G((size_t)9 * L.np);
-        rc = download_tag_order(c, L.G, 9, G.data());
-        if (rc) return rc;
+    if (gU || gV || gW) {  // the 9 gradient values of a tracer split into the caller's three arrays on the device
+        HIPCHK(c, lpt::scatter_to_tags(L.np, L.tag, L.G, 9, 3, L.pos2, c->stream));
         double* outs[3] = {gU, gV, gW};
+        gkm::CopySeg seg[3];
+        int n = 0;
         for (int f = 0; f < 3; f++)
-            if (outs[f])
-                for (long p = 0; p < L.np; p++)
-                    for (int a = 0; a < 3; a++) outs[f][3 * p + a] = G[(size_t)9 * p + 3 * f + a];
+            if (outs[f]) seg[n++] = {outs[f], L.pos2 + (size_t)3 * f * L.np, sizeof(double) * 3 * L.np};
+        HIPCHK(c, c->pipe.to_host(seg, n, c->stream));
     }
     return GKM_OK;
 }
@@ -949,9 +954,8 @@ int lpt_properties(gkm_ctx* c, double* out)
         return fail(c, GKM_ENOMEM, "hipMalloc particle properties");
     const lpt::Geom g = geom_of(c);
     HIPCHK(c, lpt::launch_props(L.np, L.pos, L.tag, L.pcs, g, L.props, c->stream));
-    HIPCHK(c, hipMemcpyAsync(out, L.props, sizeof(double) * lpt::kPropWidth * L.np, hipMemcpyDeviceToHost,
-                             c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    const gkm::CopySeg seg{out, L.props, sizeof(double) * lpt::kPropWidth * L.np};
+    HIPCHK(c, c->pipe.to_host(&seg, 1, c->stream));
     return GKM_OK;
 }
 

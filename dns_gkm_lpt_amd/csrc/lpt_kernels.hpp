@@ -73,8 +73,10 @@ hipError_t launch_heun(long np, double* pos, const double* U, const double* cons
 // Reorder the particles by cell index (y, x, z cell of dx) with a radix sort;
 // pos and tag follow, U and G are resampled after a sort.
 hipError_t sort_by_cell(State& s, const Geom& g, double dx, hipStream_t st);
-// dst[tag[i]] = src[i] for rows of `width` doubles (slot order -> tag order)
-hipError_t scatter_to_tags(long np, const int* tag, const double* src, int width, double* dst, hipStream_t st);
+// dst[tag[i]] = src[i] for rows of `width` doubles (slot order -> tag order); with
+// part < width the rows' parts of `part` values go to arrays of their own, np x
+// part each, one after the other
+hipError_t scatter_to_tags(long np, const int* tag, const double* src, int width, int part, double* dst, hipStream_t st);
 
 // ---- batched over the members of an ensemble (no reference counterpart) ----
 // One launch covers every entry; entry e owns blocks [first[e], first[e+1]),

@@ -52,13 +52,17 @@ __global__ void gather_kernel(long np, const int* __restrict__ perm, const doubl
     tag_out[p] = tag[q];
 }
 
-__global__ void scatter_kernel(long np, const int* __restrict__ tag, const double* __restrict__ src, int width,
+// one thread per value: reads run along the rows, and a row's `width` values
+// (or its parts of `part` values, each part an array of its own) are written by
+// neighbouring threads
+__global__ void scatter_kernel(long np, const int* __restrict__ tag, const double* __restrict__ src, int width, int part,
                                double* __restrict__ dst)
 {
-    const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= np) return;
-    const long t = tag[p];
-    for (int c = 0; c < width; c++) dst[t * width + c] = src[p * width + c];
+    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= np * width) return;
+    const long p = i / width;
+    const int c = (int)(i - p * width);
+    dst[(c / part) * np * part + (long)tag[p] * part + c % part] = src[i];
 }
 
 static unsigned nblocks(long n) { return (unsigned)((n + 255) / 256); }
@@ -97,10 +101,11 @@ hipError_t sort_by_cell(State& s, const Geom& g, double dx, hipStream_t st)
     return e;
 }
 
-hipError_t scatter_to_tags(long np, const int* tag, const double* src, int width, double* dst, hipStream_t st)
+hipError_t scatter_to_tags(long np, const int* tag, const double* src, int width, int part, double* dst, hipStream_t st)
 {
     if (np <= 0) return hipSuccess;
-    hipLaunchKernelGGL(scatter_kernel, dim3(nblocks(np)), dim3(256), 0, st, np, tag, src, width, dst);
+    if (width < 1 || part < 1 || width % part) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(scatter_kernel, dim3(nblocks(np * width)), dim3(256), 0, st, np, tag, src, width, part, dst);
     return hipGetLastError();
 }
 
