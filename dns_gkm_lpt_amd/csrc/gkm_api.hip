@@ -31,6 +31,7 @@ struct gkm_ctx {
     double dx = 0.0;
     gkm::Gas<double> gas{};
     hipStream_t stream = nullptr;
+    double* slab = nullptr;  // holds W, dW, faces, stage, dscal, hist, partial and a mixed context's cmp
     double* W[2] = {nullptr, nullptr};
     int cur = 0;
     double* dW = nullptr;
@@ -38,12 +39,16 @@ struct gkm_ctx {
     // and variable (5 x plane floats) of W[0] and W[1]; on by default for
     // GKM_MIXED (allocated at create), off for GKM_FP64
     float* cmp[2] = {nullptr, nullptr};
+    float* cmp_own = nullptr;      // cmp[] of an FP64 context, allocated when switched on
     bool compensate = false;
     bool member = false;           // owned by an ensemble (its tables hold the carry pointers)
     double* stage = nullptr;       // 5 * padded
-    double* dscal = nullptr;       // [0] dt, [1] vmax
-    int* dflag = nullptr;          // non-physical-state flag
+    double* dscal = nullptr;       // [0] dt, [1] vmax, [2] dt of lpt_heun, [3] the two ints of dflag
+    int* dflag = nullptr;          // in dscal[3]: non-physical-state flag, ticket of the step's CFL
+    double* hscal = nullptr;       // pinned copy of dscal
     double* partial = nullptr;     // CFL block maxima
+    double* faces = nullptr;       // face fluxes of the three directions (small FP64 grids)
+    double* hist = nullptr;        // behind dscal: dt of the last kHist steps of gkm_run
     bool have_state = false;
     int tile[3] = {0, 0, 0};       // sweep tile variant per direction
     int slots = 512;               // concurrent sweep workgroups: 2 per CU
@@ -59,7 +64,8 @@ struct gkm_ctx {
     // tangent-linear / adjoint (allocated on first use)
     double* adj_scratch = nullptr;
     double* adj_vec[2] = {nullptr, nullptr};  // tangent or adjoint vectors, 5 x plane each
-    std::vector<double*> adj_states;          // checkpoints and segment states
+    std::vector<double*> adj_states;          // checkpoints and segment states, parts of adj_slabs
+    std::vector<double*> adj_slabs;
     // the trajectory recorded by the last gkm_adjoint_forward (adj_n < 0: none)
     int adj_n = -1, adj_every = 1;
     double adj_dt = 0.0;
@@ -79,6 +85,8 @@ int fail(gkm_ctx* c, int code, const std::string& msg)
         if (e_ != hipSuccess)                                                                        \
             return fail((ctx), GKM_EHIP, std::string(#call) + ": " + hipGetErrorString(e_));          \
     } while (0)
+
+constexpr int kScal = 4, kHist = 4096;
 
 // run f() bracketed by timing events when enabled; accumulates into slot
 template <typename Fn>
@@ -124,8 +132,18 @@ gkm::SweepArgs sweep_args(const gkm_ctx* c, int dir, int mode)
     return a;
 }
 
+// Two launches instead of three sweeps (gkm::launch_small_step) where the grid
+// is small and nothing asks for the sweeps one by one; the results are the same.
+bool small_step(const gkm_ctx* c) { return c->faces && !c->timing && !c->compensate; }
+
 int eulerian_step(gkm_ctx* c)
 {
+    if (small_step(c)) {
+        HIPCHK(c, gkm::launch_small_step(sweep_args(c, 0, 0), c->faces, nullptr, c->stream));
+        c->cur = 1 - c->cur;
+        c->lpt.valid = false;
+        return GKM_OK;
+    }
     for (int dir = 0; dir < 3; dir++) {
         // x: dW = dF, y: dW += dF, z: Wout = W - (dW + dF)/dx
         const gkm::SweepArgs a = sweep_args(c, dir, dir);
@@ -137,11 +155,26 @@ int eulerian_step(gkm_ctx* c)
     return GKM_OK;
 }
 
-int cfl_on_device(gkm_ctx* c)
+// dscal into hscal once the stream's work is done; an error if the CFL pass saw
+// a non-physical state
+int read_scalars(gkm_ctx* c)
+{
+    if (!c->hscal && hipHostMalloc(reinterpret_cast<void**>(&c->hscal), sizeof(double) * kScal, hipHostMallocDefault) != hipSuccess) {
+        c->hscal = nullptr;
+        return fail(c, GKM_ENOMEM, "hipHostMalloc scalars");
+    }
+    HIPCHK(c, hipMemcpyAsync(c->hscal, c->dscal, sizeof(double) * kScal, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    if (*reinterpret_cast<const int*>(c->hscal + 3) && c->cfg.check_state)
+        return fail(c, GKM_ESTATE, "non-physical state (rho <= 0, p <= 0 or NaN)");
+    return GKM_OK;
+}
+
+int cfl_on_device(gkm_ctx* c, double* hist = nullptr)
 {
     return timed(c, 3, [&] {
         return gkm::launch_cfl(c->W[c->cur], c->plane, c->gas.gam, c->cfg.cfl, c->dx, c->partial, c->dscal,
-                               c->dscal + 1, c->dflag, c->stream);
+                               c->dscal + 1, c->dflag, hist, c->stream);
     });
 }
 
@@ -185,24 +218,42 @@ int gkm_create(const gkm_config* cfg, gkm_ctx** out)
     }
     HIPCHK(c, hipEventCreate(&c->ev[0]));
     HIPCHK(c, hipEventCreate(&c->ev[1]));
-    const size_t sbytes = sizeof(double) * 5 * (size_t)c->plane;
-    for (int b = 0; b < 2; b++)
-        if (hipMalloc(&c->W[b], sbytes) != hipSuccess) return fail(c, GKM_ENOMEM, "hipMalloc state");
-    if (hipMalloc(&c->dW, sbytes) != hipSuccess) return fail(c, GKM_ENOMEM, "hipMalloc dW");
-    if (cfg->precision == GKM_MIXED) {
-        const size_t cbytes = sizeof(float) * 5 * (size_t)gkm::carry_plane(c->nc);
+    // one allocation for everything the context always holds (a gradient makes a
+    // context per call; create at 128^3 0.6-1.2 -> 0.3 ms, at 512^3 1.6 -> 0.7)
+    const bool mixed = cfg->precision == GKM_MIXED;
+    const size_t state = 5 * (size_t)c->plane, staged = 5 * (size_t)c->padded;
+    // face fluxes of the two-launch step: the y and z directions' behind dW's 5 planes
+    const size_t faces = !mixed && gkm::small_step_ok(nc) ? 2 * state : 0;
+    const size_t carry = mixed ? (5 * (size_t)gkm::carry_plane(nc) + 1) / 2 : 0;  // floats, in doubles
+    auto even = [](size_t n) { return (n + 31) & ~size_t(31); };               // 256 B
+    const size_t sizes[] = {even(state), even(state), even(state + faces), even(staged), even(kScal + kHist),
+                            even(gkm::kCflBlocks), even(carry), even(carry)};
+    size_t total = 0;
+    for (size_t n : sizes) total += n;
+    if (hipMalloc(&c->slab, sizeof(double) * total) != hipSuccess) return fail(c, GKM_ENOMEM, "hipMalloc state");
+    double* at = c->slab;
+    auto take = [&](int k) {
+        double* p = at;
+        at += sizes[k];
+        return p;
+    };
+    c->W[0] = take(0);
+    c->W[1] = take(1);
+    c->dW = take(2);
+    if (faces) c->faces = c->dW;
+    c->stage = take(3);
+    c->dscal = take(4);
+    c->dflag = reinterpret_cast<int*>(c->dscal + 3);
+    c->hist = c->dscal + kScal;
+    c->partial = take(5);
+    HIPCHK(c, hipMemsetAsync(c->dscal, 0, sizeof(double) * kScal, c->stream));
+    if (mixed) {
         for (int b = 0; b < 2; b++) {
-            if (hipMalloc(&c->cmp[b], cbytes) != hipSuccess) return fail(c, GKM_ENOMEM, "hipMalloc carry");
-            HIPCHK(c, hipMemsetAsync(c->cmp[b], 0, cbytes, c->stream));
+            c->cmp[b] = reinterpret_cast<float*>(take(6 + b));
+            HIPCHK(c, hipMemsetAsync(c->cmp[b], 0, sizeof(float) * 5 * (size_t)gkm::carry_plane(nc), c->stream));
         }
         c->compensate = true;
     }
-    if (hipMalloc(&c->stage, sizeof(double) * 5 * (size_t)c->padded) != hipSuccess)
-        return fail(c, GKM_ENOMEM, "hipMalloc staging");
-    if (hipMalloc(&c->dscal, sizeof(double) * 4) != hipSuccess) return fail(c, GKM_ENOMEM, "hipMalloc scalars");
-    if (hipMalloc(&c->dflag, sizeof(int) * 4) != hipSuccess) return fail(c, GKM_ENOMEM, "hipMalloc flag");
-    if (hipMalloc(&c->partial, sizeof(double) * gkm::kCflBlocks) != hipSuccess)
-        return fail(c, GKM_ENOMEM, "hipMalloc partial");
     return GKM_OK;
 }
 
@@ -215,16 +266,10 @@ void gkm_destroy(gkm_ctx* c)
     (void)hipFree(c->adj_scratch);
     (void)hipFree(c->adj_vec[0]);
     (void)hipFree(c->adj_vec[1]);
-    for (double* p : c->adj_states) (void)hipFree(p);
-    (void)hipFree(c->W[0]);
-    (void)hipFree(c->W[1]);
-    (void)hipFree(c->dW);
-    (void)hipFree(c->cmp[0]);
-    (void)hipFree(c->cmp[1]);
-    (void)hipFree(c->stage);
-    (void)hipFree(c->dscal);
-    (void)hipFree(c->dflag);
-    (void)hipFree(c->partial);
+    for (double* p : c->adj_slabs) (void)hipFree(p);
+    (void)hipFree(c->slab);
+    (void)hipFree(c->cmp_own);
+    (void)hipHostFree(c->hscal);
     if (c->ev[0]) (void)hipEventDestroy(c->ev[0]);
     if (c->ev[1]) (void)hipEventDestroy(c->ev[1]);
     if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -240,9 +285,10 @@ int gkm_set_compensation(gkm_ctx* c, int on)
     if (!c) return GKM_EINVAL;
     if (c->member) return fail(c, GKM_EINVAL, "an ensemble member keeps its precision's compensation setting");
     if (on && !c->cmp[0]) {
-        const size_t cbytes = sizeof(float) * 5 * (size_t)gkm::carry_plane(c->nc);
-        for (int b = 0; b < 2; b++)
-            if (hipMalloc(&c->cmp[b], cbytes) != hipSuccess) return fail(c, GKM_ENOMEM, "hipMalloc carry");
+        const size_t n = 5 * (size_t)gkm::carry_plane(c->nc);
+        if (hipMalloc(&c->cmp_own, 2 * sizeof(float) * n) != hipSuccess) return fail(c, GKM_ENOMEM, "hipMalloc carry");
+        c->cmp[0] = c->cmp_own;
+        c->cmp[1] = c->cmp_own + n;
     }
     if (on && !c->compensate) {
         // the resident state starts with no carried error
@@ -330,8 +376,7 @@ int gkm_step(gkm_ctx* c, double dt)
     if (!c) return GKM_EINVAL;
     if (!c->have_state) return fail(c, GKM_ENOTREADY, "no state uploaded");
     if (!(dt > 0.0) || !std::isfinite(dt)) return fail(c, GKM_EINVAL, "dt must be positive and finite");
-    HIPCHK(c, hipMemcpyAsync(c->dscal, &dt, sizeof(double), hipMemcpyHostToDevice, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));  // dt lives on the host stack
+    HIPCHK(c, gkm::launch_set_scalar(c->dscal, dt, c->stream));
     return eulerian_step(c);
 }
 
@@ -341,13 +386,9 @@ int gkm_cfl_dt(gkm_ctx* c, double* dt)
     if (!c->have_state) return fail(c, GKM_ENOTREADY, "no state uploaded");
     int rc = cfl_on_device(c);
     if (rc) return rc;
-    double s[2];
-    int flag = 0;
-    HIPCHK(c, hipMemcpyAsync(s, c->dscal, sizeof(double) * 2, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipMemcpyAsync(&flag, c->dflag, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    if (flag && c->cfg.check_state) return fail(c, GKM_ESTATE, "non-physical state (rho <= 0, p <= 0 or NaN)");
-    *dt = s[0];
+    rc = read_scalars(c);
+    if (rc) return rc;
+    *dt = c->hscal[0];
     return GKM_OK;
 }
 
@@ -355,23 +396,40 @@ int gkm_run(gkm_ctx* c, int nsteps, double* dt_hist)
 {
     if (!c || nsteps < 0) return fail(c, GKM_EINVAL, "bad argument");
     if (!c->have_state) return fail(c, GKM_ENOTREADY, "no state uploaded");
-    for (int n = 0; n < nsteps; n++) {
-        int rc = cfl_on_device(c);  // dt of this step from W^n (update.cpp:115, 167)
-        if (rc) return rc;
-        if (dt_hist) HIPCHK(c, hipMemcpyAsync(dt_hist + n, c->dscal, sizeof(double), hipMemcpyDeviceToHost, c->stream));
-        rc = eulerian_step(c);
+    // dt of step n from W^n (update.cpp:115, 167), kept on the device: hist[n mod kHist]
+    const bool small = small_step(c);
+    auto hist = [&](int n) { return dt_hist && n < nsteps ? c->hist + n % kHist : nullptr; };
+    auto fetch = [&](int n) {  // the dts of the history's part that ends with step n - 1
+        const int m = (n - 1) % kHist + 1;
+        return hipMemcpyAsync(dt_hist + n - m, c->hist, sizeof(double) * m, hipMemcpyDeviceToHost, c->stream);
+    };
+    if (small && nsteps > 0) {
+        int rc = cfl_on_device(c, hist(0));
         if (rc) return rc;
     }
+    for (int n = 0; n < nsteps; n++) {
+        if (small) {
+            // the history's slot of step n + 1 may be one not yet fetched: fetch first
+            if (dt_hist && (n + 1) % kHist == 0 && n + 1 < nsteps) HIPCHK(c, fetch(n + 1));
+            const gkm::StepCfl next{c->gas.gam, c->cfg.cfl, c->partial, c->dscal, c->dscal + 1, hist(n + 1), c->dflag, c->dflag + 1};
+            HIPCHK(c, gkm::launch_small_step(sweep_args(c, 0, 0), c->faces, &next, c->stream));
+            c->cur = 1 - c->cur;
+            c->lpt.valid = false;
+        } else {
+            if (dt_hist && n % kHist == 0 && n > 0) HIPCHK(c, fetch(n));
+            int rc = cfl_on_device(c, hist(n));
+            if (rc) return rc;
+            rc = eulerian_step(c);
+            if (rc) return rc;
+        }
+    }
+    if (dt_hist && nsteps > 0) HIPCHK(c, fetch(nsteps));
     // the flag so far describes W^0 .. W^{n-1}; check the state the last step produced
-    if (nsteps > 0) {
+    if (nsteps > 0 && !small) {
         int rc = cfl_on_device(c);
         if (rc) return rc;
     }
-    int flag = 0;
-    HIPCHK(c, hipMemcpyAsync(&flag, c->dflag, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    if (flag && c->cfg.check_state) return fail(c, GKM_ESTATE, "non-physical state (rho <= 0, p <= 0 or NaN)");
-    return GKM_OK;
+    return read_scalars(c);
 }
 
 int gkm_sweep_flux_diff(gkm_ctx* c, int dir, double dt, double* out)
@@ -379,8 +437,7 @@ int gkm_sweep_flux_diff(gkm_ctx* c, int dir, double dt, double* out)
     if (!c || !out || dir < 0 || dir > 2) return fail(c, GKM_EINVAL, "bad argument");
     if (!c->have_state) return fail(c, GKM_ENOTREADY, "no state uploaded");
     if (!(dt > 0.0) || !std::isfinite(dt)) return fail(c, GKM_EINVAL, "dt must be positive and finite");
-    HIPCHK(c, hipMemcpyAsync(c->dscal, &dt, sizeof(double), hipMemcpyHostToDevice, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    HIPCHK(c, gkm::launch_set_scalar(c->dscal, dt, c->stream));
     const gkm::SweepArgs a = sweep_args(c, dir, 0);
     int rc = timed(c, dir, [&] { return gkm::launch_sweep(dir, a, c->cfg.precision == GKM_MIXED, c->stream); });
     if (rc) return rc;
@@ -402,13 +459,14 @@ int adj_prepare(gkm_ctx* c, double dt, int nstates)
         return fail(c, GKM_ENOMEM, "hipMalloc adjoint scratch");
     for (auto& v : c->adj_vec)
         if (!v && hipMalloc(&v, sb) != hipSuccess) return fail(c, GKM_ENOMEM, "hipMalloc adjoint vectors");
-    while ((int)c->adj_states.size() < nstates) {
+    const int more = nstates - (int)c->adj_states.size();
+    if (more > 0) {  // the missing states in one allocation
         double* p = nullptr;
-        if (hipMalloc(&p, sb) != hipSuccess) return fail(c, GKM_ENOMEM, "hipMalloc checkpoints");
-        c->adj_states.push_back(p);
+        if (hipMalloc(&p, sb * more) != hipSuccess) return fail(c, GKM_ENOMEM, "hipMalloc checkpoints");
+        c->adj_slabs.push_back(p);
+        for (int k = 0; k < more; k++) c->adj_states.push_back(p + (size_t)k * 5 * c->plane);
     }
-    HIPCHK(c, hipMemcpyAsync(c->dscal, &dt, sizeof(double), hipMemcpyHostToDevice, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));  // dt lives on the host stack
+    HIPCHK(c, gkm::launch_set_scalar(c->dscal, dt, c->stream));
     return GKM_OK;
 }
 
@@ -987,8 +1045,7 @@ int lpt_heun(gkm_ctx* c, double dt)
     if (!(dt > 0.0) || !std::isfinite(dt)) return fail(c, GKM_EINVAL, "dt must be positive and finite");
     int rc = ensure_spline(c);
     if (rc) return rc;
-    HIPCHK(c, hipMemcpyAsync(c->dscal + 2, &dt, sizeof(double), hipMemcpyHostToDevice, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    HIPCHK(c, gkm::launch_set_scalar(c->dscal + 2, dt, c->stream));
     const lpt::Geom g = geom_of(c);
     const double* cn[3] = {L.coef[L.cur][0], L.coef[L.cur][1], L.coef[L.cur][2]};
     rc = timed(c, 5, [&] { return lpt::launch_heun(L.np, L.pos, L.U, cn, g, c->dscal + 2, c->stream); });
@@ -997,7 +1054,6 @@ int lpt_heun(gkm_ctx* c, double dt)
         rc = timed(c, 6, [&] { return lpt::sort_by_cell(L, g, c->dx, c->stream); });
         if (rc) return rc;
     }
-    HIPCHK(c, hipStreamSynchronize(c->stream));
     return GKM_OK;
 }
 
@@ -1024,7 +1080,6 @@ int lpt_coupled_step(gkm_ctx* c, double dt)
         rc = timed(c, 6, [&] { return lpt::sort_by_cell(L, g, c->dx, c->stream); });
         if (rc) return rc;
     }
-    HIPCHK(c, hipStreamSynchronize(c->stream));
     return GKM_OK;
 }
 

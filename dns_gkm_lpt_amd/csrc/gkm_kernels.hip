@@ -42,6 +42,128 @@ __global__ __launch_bounds__(256, 2) void ens_sweep_kernel(const SweepArgs* __re
 
 static int cdiv(int a, int b) { return (a + b - 1) / b; }
 
+// ---------------------------------------------------------------------------
+// FP64 step of a small grid in two launches.  A 32^3 sweep is 256 workgroups of
+// two chunks, one of them the lead-in: three sweeps in turn leave half the chip
+// idle, do every face twice and pay three launches.  Here one launch computes
+// the face fluxes of all three directions (independent of each other), one chunk
+// per workgroup and no lead-in, and a second one the update (the sweeps'
+// expressions in their order: equal to them bit for bit) and, in a free-running
+// loop, the CFL maximum of the new state; its last workgroup forms the next dt.
+// ---------------------------------------------------------------------------
+struct FaceArgs {
+    SweepArgs dir[3];
+    int first[4];  // blocks [first[d], first[d+1]) sweep direction d
+};
+template <bool GEN>
+__global__ __launch_bounds__(256, 2) void faces_kernel(FaceArgs a)
+{
+    __shared__ double lds[max3(sweep_lds_doubles<0, 0, false>(), sweep_lds_doubles<1, 0, false>(), sweep_lds_doubles<2, 0, false>())];
+    const int b = blockIdx.x;
+    if (b < a.first[1]) sweep_body_pair<0, 0, true, GEN, true>(a.dir[0], b, a.first[1], true, lds);
+    else if (b < a.first[2]) sweep_body_pair<1, 0, true, GEN, true>(a.dir[1], b - a.first[1], a.first[2] - a.first[1], true, lds);
+    else sweep_body_pair<2, 0, true, GEN, true>(a.dir[2], b - a.first[2], a.first[3] - a.first[2], true, lds);
+}
+
+struct UpdateArgs {
+    const double* W;
+    double* Wout;
+    const double* F;  // 3 directions x 5 planes
+    long plane;
+    int nc;
+    double inv_dx, gam, cfl, dx;
+    double *partial, *dt, *vmax, *hist;  // partial = nullptr: no CFL
+    int *bad, *ticket;
+};
+__global__ __launch_bounds__(256) void step_update_kernel(UpdateArgs a)
+{
+    const int nc = a.nc;
+    double m = 0.0;
+    bool bad = false;
+    for (long c = (long)blockIdx.x * 256 + threadIdx.x; c < a.plane; c += (long)gridDim.x * 256) {
+        const int z = (int)(c % nc), x = (int)((c / nc) % nc), y = (int)(c / ((long)nc * nc));
+        const long cx = x ? c - nc : c + (long)(nc - 1) * nc;
+        const long cy = y ? c - (long)nc * nc : c + (long)(nc - 1) * nc * nc;
+        const long cz = z ? c - 1 : c + nc - 1;
+        double t[5];
+#pragma unroll
+        for (int q = 0; q < 5; q++) {
+            const double *Fx = a.F + q * a.plane, *Fy = Fx + 5 * a.plane, *Fz = Fy + 5 * a.plane;
+            const double dW = (Fx[c] - Fx[cx]) + (Fy[c] - Fy[cy]);
+            const double dF = Fz[c] - Fz[cz];
+            t[q] = a.W[q * a.plane + c] - a.inv_dx * (dW + dF);
+            a.Wout[q * a.plane + c] = t[q];
+        }
+        if (a.partial) cfl_cell(t[0], t[1], t[2], t[3], t[4], a.gam, m, bad);
+    }
+    if (!a.partial) return;
+    __shared__ int last;
+    __shared__ double mine;
+    cfl_block(m, bad, &mine);
+    if (threadIdx.x == 0) {
+        // the block's maximum is written through to where every XCD sees it, and
+        // there before the ticket: a release fence would write the whole L2 back,
+        // once per block (64^3: 30 us a step)
+        __hip_atomic_store(a.partial + blockIdx.x, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        const int k = __hip_atomic_fetch_add(a.ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        last = k == (int)gridDim.x - 1;
+        if (last) __hip_atomic_store(a.ticket, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch
+    }
+    __syncthreads();
+    if (!last) return;
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    cfl_reduce(a.partial, gridDim.x, a.cfl, a.dx, a.dt, a.vmax, a.bad, a.hist);
+}
+
+bool small_step_ok(int nc)
+{
+    bool ok = nc >= 16 && nc <= kSmallNc;
+    for (int d = 0; d < 3; d++) {
+        const int* t = kTilesPair[d][0];
+        ok = ok && t[0] + 3 <= nc && t[1] <= nc && t[2] <= nc;
+    }
+    return ok;
+}
+
+hipError_t launch_small_step(const SweepArgs& a, double* F, const StepCfl* cfl, hipStream_t s)
+{
+    if (!small_step_ok(a.nc) || !F || a.cmp_out) return hipErrorInvalidValue;
+    FaceArgs f{};
+    bool gen = false;
+    for (int d = 0; d < 3; d++) {
+        f.dir[d] = a;
+        f.dir[d].tile = 0;
+        f.dir[d].mode = 0;
+        f.dir[d].dW = F + (long)d * 5 * a.plane;
+        const int* t = kTilesPair[d][0];
+        f.dir[d].seg = t[0];  // one chunk per workgroup
+        f.dir[d].nseg = sweep_nseg(a.nc, t[0]);
+        f.first[d + 1] = f.first[d] + cdiv(a.nc, t[1]) * cdiv(a.nc, t[2]) * f.dir[d].nseg;
+        gen = gen || a.nc % t[0] || a.nc % t[1] || a.nc % t[2];
+    }
+    if (gen) hipLaunchKernelGGL(faces_kernel<true>, dim3(f.first[3]), dim3(256), 0, s, f);
+    else hipLaunchKernelGGL(faces_kernel<false>, dim3(f.first[3]), dim3(256), 0, s, f);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    UpdateArgs u{a.W, a.Wout, F, a.plane, a.nc, a.inv_dx, 0.0, 0.0, a.dx, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
+    if (cfl) {
+        u.gam = cfl->gam;
+        u.cfl = cfl->cfl;
+        u.partial = cfl->partial;
+        u.dt = cfl->dt;
+        u.vmax = cfl->vmax;
+        u.hist = cfl->hist;
+        u.bad = cfl->bad;
+        u.ticket = cfl->ticket;
+    }
+    // with the CFL one maximum and one ticket per block: two blocks per CU
+    const long all = (a.plane + 255) / 256, blocks = cfl && all > 512 ? 512 : all;
+    static_assert(512 <= kCflBlocks, "a partial maximum per block");
+    hipLaunchKernelGGL(step_update_kernel, dim3((unsigned)blocks), dim3(256), 0, s, u);
+    return hipGetLastError();
+}
+
 bool sweep_tile_ok(int dir, int tile, int nc)
 {
     // Any grid size: the pencils and segments of the last tiles reach past nc
@@ -227,18 +349,28 @@ __global__ __launch_bounds__(256) void cfl_partial_kernel(const double* __restri
 }
 
 __global__ __launch_bounds__(256) void cfl_final_kernel(const double* partial, int n, double cfl, double dx,
-                                                        double* dt, double* vmax, int* bad)
+                                                        double* dt, double* vmax, int* bad, double* hist)
 {
-    cfl_reduce(partial, n, cfl, dx, dt, vmax, bad);
+    cfl_reduce(partial, n, cfl, dx, dt, vmax, bad, hist);
+}
+
+__global__ void set_scalar_kernel(double* p, double v)
+{
+    if (threadIdx.x == 0) *p = v;
+}
+hipError_t launch_set_scalar(double* p, double v, hipStream_t s)
+{
+    hipLaunchKernelGGL(set_scalar_kernel, dim3(1), dim3(64), 0, s, p, v);
+    return hipGetLastError();
 }
 
 hipError_t launch_cfl(const double* W, long plane, double gam, double cfl, double dx, double* partial, double* dt,
-                      double* vmax, int* bad, hipStream_t s)
+                      double* vmax, int* bad, double* hist, hipStream_t s)
 {
     hipLaunchKernelGGL(cfl_partial_kernel, dim3(kCflBlocks), dim3(256), 0, s, W, plane, gam, partial);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(cfl_final_kernel, dim3(1), dim3(256), 0, s, partial, kCflBlocks, cfl, dx, dt, vmax, bad);
+    hipLaunchKernelGGL(cfl_final_kernel, dim3(1), dim3(256), 0, s, partial, kCflBlocks, cfl, dx, dt, vmax, bad, hist);
     return hipGetLastError();
 }
 

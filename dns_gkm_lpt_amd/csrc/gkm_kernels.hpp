@@ -93,9 +93,27 @@ inline int sweep_nseg(int nc, int seg) { return seg > 0 ? (nc + seg - 1) / seg :
 
 // CFL: partial maxima (one per block) then a one-block final pass writing
 // dt = cfl*dx/max and a non-physical-state flag.
+// hist (may be nullptr) receives a copy of dt.
 constexpr int kCflBlocks = 1024;
 hipError_t launch_cfl(const double* W, long plane, double gam, double cfl, double dx, double* partial, double* dt,
-                      double* vmax, int* bad, hipStream_t s);
+                      double* vmax, int* bad, double* hist, hipStream_t s);
+// *p = v in stream order (a scalar the caller need not keep)
+hipError_t launch_set_scalar(double* p, double v, hipStream_t s);
+
+// FP64 step of a small grid in two launches: the face fluxes of the three
+// directions, then the update and, with cfl, the dt of the new state.  F holds
+// 15 plane doubles.  Equal to the three sweeps bit for bit.  us per step with
+// dt, this / the sweeps and the CFL pass: 16^3 16 / 44, 32^3 29 / 57, 64^3 123 /
+// 160, 80^3 229 / 266, 96^3 381 / 411, 128^3 907 / 764 (the fluxes' round trip
+// through memory outweighs the lead-in chunks).
+constexpr int kSmallNc = 96;
+bool small_step_ok(int nc);
+struct StepCfl {
+    double gam, cfl;
+    double *partial, *dt, *vmax, *hist;  // hist may be nullptr
+    int *bad, *ticket;                   // ticket: 0 before the first launch, left 0
+};
+hipError_t launch_small_step(const SweepArgs& a, double* F, const StepCfl* cfl, hipStream_t s);
 // ensemble CFL: one dt per member (partial holds nmem * kEnsCflBlocks doubles)
 struct CflArgs {
     const double* W;

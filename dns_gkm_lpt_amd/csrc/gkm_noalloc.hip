@@ -1,8 +1,9 @@
 // gkm_noalloc.hip -- gkm_step_noalloc: one Eulerian step on caller-owned device
 // buffers with no device allocation (declared in include/dnsgkm.h).
 //
-// The step's scratch -- the flux-difference accumulator dW of the x and y
-// sweeps (5 nc^3 doubles) and the device dt the sweeps read -- lives in the
+// The step's scratch -- the face fluxes of the three directions (FP64, 15 nc^3
+// doubles; gkm::launch_small_step) or the flux-difference accumulator of the x
+// and y sweeps (5 nc^3), and the device dt they read -- lives in the
 // file-scope array `scratch` below, sized for nc <= kNoallocMaxNc.  Each GPU
 // the library runs on holds its own copy until the process ends; its address
 // on a device is taken once, with that device current, by hipGetSymbolAddress
@@ -25,7 +26,7 @@
 namespace {
 
 constexpr int kNoallocMaxNc = 64;
-constexpr long kNoallocDW = 5L * kNoallocMaxNc * kNoallocMaxNc * kNoallocMaxNc;  // dW doubles
+constexpr long kNoallocDW = 15L * kNoallocMaxNc * kNoallocMaxNc * kNoallocMaxNc;  // flux doubles
 constexpr long kNoallocDoubles = kNoallocDW + 32;                                // + dt (aligned)
 
 __device__ __align__(256) double scratch[kNoallocDoubles];
@@ -34,11 +35,6 @@ constexpr int kMaxDevices = 64;
 std::mutex g_mutex;
 double* g_scratch[kMaxDevices] = {};  // device address of `scratch` per device
 int g_slots[kMaxDevices] = {};        // concurrent sweep workgroups per device
-
-__global__ void set_dt_kernel(double* p, double dt)
-{
-    if (threadIdx.x == 0) *p = dt;
-}
 
 int put_msg(char* msg, int len, int code, const std::string& m)
 {
@@ -80,7 +76,7 @@ extern "C" int gkm_step_noalloc(const gkm_config* cfg, const double* W, double* 
     if (cfg->nc > kNoallocMaxNc)
         return put_msg(msg, msglen, GKM_EINVAL,
                        "nc = " + std::to_string(cfg->nc) + " exceeds the no-allocation maximum of " +
-                           std::to_string(kNoallocMaxNc) + " (scratch of 5 x 64^3 doubles per GPU)");
+                           std::to_string(kNoallocMaxNc) + " (scratch sized for 64^3 cells per GPU)");
     if (!(dt > 0.0) || !std::isfinite(dt)) return put_msg(msg, msglen, GKM_EINVAL, "dt must be positive and finite");
     if (cfg->device < 0 || cfg->device >= kMaxDevices) return put_msg(msg, msglen, GKM_EINVAL, "device out of range");
     hipError_t e = hipSetDevice(cfg->device);
@@ -93,8 +89,7 @@ extern "C" int gkm_step_noalloc(const gkm_config* cfg, const double* W, double* 
     const hipStream_t s = static_cast<hipStream_t>(stream);
     const bool mixed = cfg->precision == GKM_MIXED;
     double* ddt = sc + kNoallocDW;
-    hipLaunchKernelGGL(set_dt_kernel, dim3(1), dim3(64), 0, s, ddt, dt);
-    e = hipGetLastError();
+    e = gkm::launch_set_scalar(ddt, dt, s);
     if (e != hipSuccess) return put_msg(msg, msglen, GKM_EHIP, std::string("dt kernel: ") + hipGetErrorString(e));
     const int nc = cfg->nc;
     for (int dir = 0; dir < 3; dir++) {
@@ -116,6 +111,11 @@ extern "C" int gkm_step_noalloc(const gkm_config* cfg, const double* W, double* 
         a.seg = gkm::sweep_seg_len(dir, nc, a.tile, slots, mixed);
         a.nseg = gkm::sweep_nseg(nc, a.seg);
         a.mode = dir;  // x: dW = dF, y: dW += dF, z: Wout = W - (dW + dF)/dx
+        if (dir == 0 && !mixed && gkm::small_step_ok(nc)) {
+            e = gkm::launch_small_step(a, sc, nullptr, s);
+            if (e != hipSuccess) return put_msg(msg, msglen, GKM_EHIP, std::string("step launch: ") + hipGetErrorString(e));
+            break;
+        }
         e = gkm::launch_sweep(dir, a, mixed, s);
         if (e != hipSuccess) return put_msg(msg, msglen, GKM_EHIP, std::string("sweep launch: ") + hipGetErrorString(e));
     }

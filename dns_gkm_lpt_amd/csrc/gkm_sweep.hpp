@@ -304,7 +304,10 @@ struct PairIn {
 // The FP64 sweep: a workgroup of 256 threads walks a pencil of CA x CB lines in
 // chunks of CN faces, CN CA CB = 128, two threads per face (gks_flux_pair).
 // Otherwise as sweep_body below.
-template <int DIR, int V, bool EXT = false, bool GEN = true>
+// FACES = true: the fluxes of the faces i+1/2 of cells i go to p.dW (5 planes)
+// instead of the flux differences, and there is no lead-in chunk (step_update
+// forms the differences of all three directions).
+template <int DIR, int V, bool EXT = false, bool GEN = true, bool FACES = false>
 __device__ __forceinline__ void sweep_body_pair(const SweepArgs& p, int bid, int nblk, bool remap, double* lds = nullptr)
 {
     constexpr int CN = Tile<DIR, V, false>::CN, CA = Tile<DIR, V, false>::CA, CB = Tile<DIR, V, false>::CB;
@@ -352,9 +355,10 @@ __device__ __forceinline__ void sweep_body_pair(const SweepArgs& p, int bid, int
         for (int q = 0; q < 5; q++) r[q * st] = c[q];
         r[5 * st] = temp_gr<double>(c, gas_gR(p.g));
     };
-    // window of the lead-in chunk: cells seg0 - CN - 2 ... seg0 + 2
+    // window of the first chunk (the lead-in): cells n - 2 ... n + CN + 2
+    constexpr int c0 = FACES ? 0 : -1;
     for (int j = itn; has && j < RC; j += CN) {
-        const long idx = cell_index<DIR>(wrapi(seg0 - CN - 2 + j, nc), lca, lcb, nc);
+        const long idx = cell_index<DIR>(wrapi(seg0 + c0 * CN - 2 + j, nc), lca, lcb, nc);
         double c[5];
 #pragma unroll
         for (int q = 0; q < 5; q++) c[q] = W[q * plane + idx];
@@ -374,7 +378,7 @@ __device__ __forceinline__ void sweep_body_pair(const SweepArgs& p, int bid, int
     const int q0 = tid < NF ? 0 : 3;
 
     int h = 0;  // ring slot of cell n0 - 2
-    for (int c = -1; c < nchunk; ++c) {
+    for (int c = c0; c < nchunk; ++c) {
         const int n0 = seg0 + c * CN;  // first face of the chunk (may be < 0 for the lead-in)
 
         // ---- WENO states of every (face, line) of the chunk, one variable at a
@@ -414,13 +418,13 @@ __device__ __forceinline__ void sweep_body_pair(const SweepArgs& p, int bid, int
         }
         const bool live = c >= 0 && (!GEN || (a0 + ua < nc && b0 + ub < nc && n0 + un < seg_end));
         double old[3] = {0.0, 0.0, 0.0}, was[3] = {0.0, 0.0, 0.0};
-        if (DIR != 0 && live && p.mode != 0) {
+        if (!FACES && DIR != 0 && live && p.mode != 0) {
             const long idx = cell_index<DIR>(n0 + un, a0 + ua, b0 + ub, nc);
 #pragma unroll
             for (int k = 0; k < 3; k++)
                 if (q0 + k < 5) old[k] = p.dW[(q0 + k) * plane + idx];
         }
-        if (DIR == 2) {
+        if (!FACES && DIR == 2) {
             // the cells themselves: after the flux their ring slots may be rewritten
             const double* const w = sC + ring_at<DIR, CN, L>(0, ring_slot<CN>(h, un + 2), uc);
 #pragma unroll
@@ -467,8 +471,12 @@ __device__ __forceinline__ void sweep_body_pair(const SweepArgs& p, int bid, int
             for (int k = 0; k < 3; k++) {
                 const int q = q0 + k;
                 if (q >= 5) break;
-                const double dF = f1[q * NF] - f0[q * NF];
                 const long o = q * plane + idx;
+                if (FACES) {
+                    p.dW[o] = f1[q * NF];
+                    continue;
+                }
+                const double dF = f1[q * NF] - f0[q * NF];
                 if (DIR == 0 || p.mode == 0) p.dW[o] = dF;
                 else if (DIR == 1) p.dW[o] = old[k] + dF;
                 else p.Wout[o] = was[k] - p.inv_dx * (old[k] + dF);
@@ -643,23 +651,22 @@ __device__ __forceinline__ double wave_max(double v)
     return v;
 }
 
-// maximum of |U| + c over cells c0, c0 + stride, ... of one state; thread 0
-// writes it (or -1) to *out
-__device__ __forceinline__ void cfl_cells(const double* __restrict__ W, long plane, double gam, long c0, long stride,
-                                          double* out)
+// |U| + c of one cell into m; bad: the cell is non-physical
+__device__ __forceinline__ void cfl_cell(double den, double m1, double m2, double m3, double e, double gam, double& m,
+                                         bool& bad)
 {
-    double m = 0.0;
-    bool bad = false;
-    for (long c = c0 + threadIdx.x; c < plane; c += stride) {
-        const double den = W[c];
-        const double ir = 1.0 / den;
-        const double u = W[plane + c] * ir, v = W[2 * plane + c] * ir, w = W[3 * plane + c] * ir;
-        const double Vsqr = u * u + v * v + w * w;
-        const double P = (den * (gam - 1)) * (W[4 * plane + c] * ir - 0.5 * Vsqr);
-        const double val = sqrt(Vsqr) + sqrt(gam * P * ir);
-        if (!(den > 0.0) || !(P > 0.0) || !isfinite(val)) bad = true;
-        else m = fmax(m, val);
-    }
+    const double ir = 1.0 / den;
+    const double u = m1 * ir, v = m2 * ir, w = m3 * ir;
+    const double Vsqr = u * u + v * v + w * w;
+    const double P = (den * (gam - 1)) * (e * ir - 0.5 * Vsqr);
+    const double val = sqrt(Vsqr) + sqrt(gam * P * ir);
+    if (!(den > 0.0) || !(P > 0.0) || !isfinite(val)) bad = true;
+    else m = fmax(m, val);
+}
+
+// block maximum m (or -1 where a thread saw a bad cell), written by thread 0 to *out
+__device__ __forceinline__ void cfl_block(double m, bool bad, double* out)
+{
     __shared__ double sm[4];
     __shared__ int sbad;
     if (threadIdx.x == 0) sbad = 0;
@@ -675,9 +682,21 @@ __device__ __forceinline__ void cfl_cells(const double* __restrict__ W, long pla
     __syncthreads();  // sm, sbad are reused by the block's next call
 }
 
+// maximum of |U| + c over cells c0, c0 + stride, ... of one state; thread 0
+// writes it (or -1) to *out
+__device__ __forceinline__ void cfl_cells(const double* __restrict__ W, long plane, double gam, long c0, long stride,
+                                          double* out)
+{
+    double m = 0.0;
+    bool bad = false;
+    for (long c = c0 + threadIdx.x; c < plane; c += stride)
+        cfl_cell(W[c], W[plane + c], W[2 * plane + c], W[3 * plane + c], W[4 * plane + c], gam, m, bad);
+    cfl_block(m, bad, out);
+}
+
 // block reduction of n partial maxima (-1 = non-physical state seen) -> dt
 __device__ __forceinline__ void cfl_reduce(const double* partial, int n, double cfl, double dx, double* dt, double* vmax,
-                                           int* bad)
+                                           int* bad, double* hist = nullptr)
 {
     double m = 0.0;
     int b = 0;
@@ -701,7 +720,9 @@ __device__ __forceinline__ void cfl_reduce(const double* partial, int n, double 
         const int anyb = sb[0] | sb[1] | sb[2] | sb[3];
         *vmax = r;
         *bad = anyb;
-        *dt = (anyb || !(r > 0.0)) ? 0.0 : cfl * dx / r;
+        const double d = (anyb || !(r > 0.0)) ? 0.0 : cfl * dx / r;
+        *dt = d;
+        if (hist) *hist = d;
     }
     __syncthreads();  // sm, sb are reused by the block's next call
 }
