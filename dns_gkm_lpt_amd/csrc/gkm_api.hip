@@ -11,6 +11,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <map>
 #include <new>
 #include <string>
 #include <vector>
@@ -1156,7 +1157,7 @@ void drop_graphs(gkm_ensemble* e)
 }
 
 // sweep arguments of member m for parity p (state in W[p], next state W[1-p]), direction d, tile v
-gkm::SweepArgs ens_sweep_args(const gkm_ctx* c, int p, int d, int v)
+gkm::SweepArgs ens_sweep_args(const gkm_ctx* c, int p, int d, int v, int most)
 {
     gkm::SweepArgs a{};
     a.W = c->W[p];
@@ -1173,10 +1174,47 @@ gkm::SweepArgs ens_sweep_args(const gkm_ctx* c, int p, int d, int v)
     a.half_idx = 0.5 * a.inv_dx;
     a.g = gkm::gas_const(c->gas);
     a.tile = v;
-    a.seg = gkm::sweep_seg_len(d, c->nc, v, 0, c->cfg.precision == GKM_MIXED);
+    a.seg = gkm::sweep_seg_most(d, c->nc, v, most, c->cfg.precision == GKM_MIXED);
     a.nseg = gkm::sweep_nseg(c->nc, a.seg);
     a.mode = d;
     return a;
+}
+
+// Chunks per workgroup of an ensemble's sweep: the limit whose workgroups, taken
+// longest first by whichever of the device's slots is free, end first.  A
+// workgroup costs its chunks and about 1.3 more (the lead-in chunk and its
+// loads).  Whole lines leave the slots idle behind the longest members unless
+// there are several rounds of them.
+int ens_most_chunks(const gkm_ensemble* e, int d, int v)
+{
+    const bool mixed = e->mem[0]->cfg.precision == GKM_MIXED;
+    int best = 1 << 20;
+    double best_end = 0.0;
+    for (const int most : {1 << 20, 24, 16, 12, 8, 6, 4, 3, 2, 1}) {
+        std::vector<std::pair<double, int>> items;  // cost, workgroups
+        for (const gkm_ctx* c : e->mem) {
+            const int seg = gkm::sweep_seg_most(d, c->nc, v, most, mixed);
+            items.push_back({gkm::sweep_chunks(d, v, seg, mixed) + 1.3, gkm::sweep_blocks(d, c->nc, v, seg, mixed)});
+        }
+        std::sort(items.begin(), items.end(), [](auto& x, auto& y) { return x.first > y.first; });
+        std::map<double, int> slots{{0.0, e->mem[0]->slots}};  // slots by the time they come free
+        double end = 0.0;
+        for (const auto& it : items)
+            for (int left = it.second; left > 0;) {
+                const auto first = slots.begin();
+                const int k = std::min(left, first->second);
+                const double t = first->first + it.first;
+                if ((first->second -= k) == 0) slots.erase(first);
+                slots[t] += k;
+                end = std::max(end, t);
+                left -= k;
+            }
+        if (best_end == 0.0 || end < best_end) {
+            best_end = end;
+            best = most;
+        }
+    }
+    return best;
 }
 
 // upload the argument tables for tiles t[3]
@@ -1200,17 +1238,18 @@ int ens_build(gkm_ensemble* e, const int t[3])
         // pencils out in this order (64-member workload: 6.62 -> 6.42 ms per
         // step); the per-phase launches measured the same either way
         const bool mixed = e->mem[0]->cfg.precision == GKM_MIXED;  // members share the precision
+        const int most = ens_most_chunks(e, d, t[d]);
         std::vector<int> order(n);
         std::vector<int> seg(n);
         for (int m = 0; m < n; m++) {
             order[m] = m;
-            seg[m] = ens_sweep_args(e->mem[m], 0, d, t[d]).seg;
+            seg[m] = ens_sweep_args(e->mem[m], 0, d, t[d], most).seg;
         }
         std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return seg[x] > seg[y]; });
         for (int k = 0; k < n; k++) {
             const int m = order[k];
             first[(size_t)d * (n + 1) + k] = acc;
-            for (int p = 0; p < 2; p++) args[((size_t)p * 3 + d) * n + k] = ens_sweep_args(e->mem[m], p, d, t[d]);
+            for (int p = 0; p < 2; p++) args[((size_t)p * 3 + d) * n + k] = ens_sweep_args(e->mem[m], p, d, t[d], most);
             const gkm::SweepArgs& a = args[(size_t)d * n + k];
             acc += gkm::sweep_blocks(d, a.nc, t[d], a.seg, mixed);
             exact = exact && gkm::sweep_exact(d, t[d], a.nc, a.seg, mixed);

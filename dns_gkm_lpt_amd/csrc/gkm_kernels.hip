@@ -216,17 +216,20 @@ int sweep_seg_len(int dir, int nc, int tile, int slots, bool mixed)
         }
         return best;
     }
-    // members of an ensemble (their workgroups add up): the whole line when
-    // that already gives >= 1024 workgroups (4 per CU), otherwise halve while
-    // segments stay >= 8 chunks and >= 64 faces long.
-    const int min_seg = 8 * CN > 64 ? 8 * CN : 64;
-    int seg = lchunks * CN;
-    while (pencils * cdiv(nc, seg) < 1024) {
-        const int half = cdiv(seg / CN, 2) * CN;
-        if (half >= seg || half < min_seg) break;
-        seg = half;
-    }
-    return seg;
+    return lchunks * CN;  // an ensemble's members: whole lines, or sweep_seg_most
+}
+
+int sweep_seg_most(int dir, int nc, int tile, int most, bool mixed)
+{
+    // at most `most` chunks per workgroup, in equal parts where the tile divides
+    // the line (the segment then divides the grid too: sweep_exact)
+    if (!sweep_tile_ok(dir, tile, nc) || most < 1) return 0;
+    const int CN = tile_shape(dir, tile, mixed)[0];
+    const int lchunks = cdiv(nc, CN);
+    int parts = cdiv(lchunks, most);
+    if (nc % CN == 0)
+        while (lchunks % parts) parts++;
+    return cdiv(lchunks, parts) * CN;
 }
 
 template <int DIR, int V>
@@ -285,6 +288,8 @@ int sweep_blocks(int dir, int nc, int tile, int seg, bool mixed)
     const int* t = tile_shape(dir, tile, mixed);
     return cdiv(nc, t[1]) * cdiv(nc, t[2]) * cdiv(nc, seg);
 }
+
+int sweep_chunks(int dir, int tile, int seg, bool mixed) { return seg / tile_shape(dir, tile, mixed)[0]; }
 
 bool sweep_exact(int dir, int tile, int nc, int seg, bool mixed)
 {

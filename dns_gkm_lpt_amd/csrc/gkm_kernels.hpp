@@ -71,6 +71,7 @@ struct Tile {
 hipError_t launch_sweep(int dir, const SweepArgs& a, bool mixed, hipStream_t s);
 // blocks of one grid's sweep launch for a tile variant and segment length
 int sweep_blocks(int dir, int nc, int tile, int seg, bool mixed);
+int sweep_chunks(int dir, int tile, int seg, bool mixed);  // chunks of a segment
 // one launch sweeping every member of an ensemble: members[m] (device array) with
 // blocks [first[m], first[m+1]) of nblk = first[nmem]; one tile variant for all.
 // exact: the tile and segment divide every member's grid (sweep_exact);
@@ -83,6 +84,8 @@ bool sweep_exact(int dir, int tile, int nc, int seg, bool mixed);
 // faces per workgroup chosen for a grid: slots = concurrent workgroups of the
 // device for a single grid, 0 for the members of an ensemble
 int sweep_seg_len(int dir, int nc, int tile, int slots, bool mixed);
+// the same for at most `most` chunks per workgroup
+int sweep_seg_most(int dir, int nc, int tile, int most, bool mixed);
 // any nc in [16, 1024] has a tile variant per direction; a variant fits nc when
 // CN + 3 <= nc and CA, CB <= nc
 bool sweep_grid_ok(int nc);
