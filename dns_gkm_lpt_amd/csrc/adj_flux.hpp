@@ -1,5 +1,7 @@
 // adj_flux.hpp -- reverse-mode derivative of the GKS face flux with respect to
-// all 50 of its inputs (no reference counterpart).
+// all 50 of its inputs (no reference counterpart).  The kernels run it by two lanes
+// per face (adj_pair.hpp) from the same building blocks; face_flux_vjp is the
+// one-lane form the host checks hold both to.
 //
 // face_flux_vjp gives xbar[k] = sum_q Fbar[q] dF_q/dx_k for face_flux (the FP64
 // flux gks_flux_tf<double, double> of gkm_flux.hpp, which restates
@@ -237,8 +239,8 @@ struct SideFwd {
     double sy[5], sz[5], b[5], f[5];
 };
 
-template <int side>
-__host__ __device__ __forceinline__ void side_fwd(const Maxw<double>& S, double h0, double h1, const double* x,
+template <int side, typename X>
+__host__ __device__ __forceinline__ void side_fwd(const Maxw<double>& S, double h0, double h1, const X& x,
                                                   const Maxw<double>& E, const TimeCoefs<double>& tc, const FluxK& k,
                                                   SideFwd& s)
 {
@@ -295,12 +297,12 @@ struct CoefBar {
 // (Beb, Fsb, byeb, bzeb) to the side's parameters (Sb), E's tangential
 // velocity, the side's two half-space moments h0, h1, the six-slope inputs of
 // this side (xbar[20 + 5 (2 d + side) + q]) and the time coefficients.
-template <int side>
-__host__ __device__ __noinline__ void side_rev(const Maxw<double>& S, double h0, double h1, const double* x,
+template <int side, typename X, typename XB>
+__host__ __device__ __forceinline__ void side_rev(const Maxw<double>& S, double h0, double h1, const X& x,
                                          const Maxw<double>& E, const TimeCoefs<double>& tc, const FluxK& k,
                                          const double Beb[5], const double Fsb[5], const double byeb[5],
                                          const double bzeb[5], MaxwBar& Sb, MaxwBar& Eb, double& h0b, double& h1b,
-                                         CoefBar& cb, double* xbar)
+                                         CoefBar& cb, XB&& xbar)
 {
     SideFwd s;
     side_fwd<side>(S, h0, h1, x, E, tc, k, s);
@@ -418,7 +420,7 @@ __host__ __device__ __noinline__ void side_rev(const Maxw<double>& S, double h0,
         for (int q = 0; q < 5; q++) Dl[q] = x[20 + 5 * (2 * d + side) + q] * s.iden;
         tunshift_vjp(Dl, S.v, S.w, mb, Sb.v, Sb.w);
         for (int q = 0; q < 5; q++) {
-            xbar[20 + 5 * (2 * d + side) + q] = s.iden * mb[q];
+            xbar(20 + 5 * (2 * d + side) + q, s.iden * mb[q]);
             idenb += x[20 + 5 * (2 * d + side) + q] * mb[q];
         }
     }
@@ -690,8 +692,9 @@ __host__ __device__ inline void face_flux_vjp(const double x[50], double dt, dou
     Eb.den += tc.gm2 * cBEb + tc.p2 * cFEb;
     // the side blocks
     double hlb[4] = {0, 0, 0, 0}, hrb[4] = {0, 0, 0, 0};
-    side_rev<0>(L, hl[0], hl[1], x, E, tc, k, Beb, Fsb, byeb, bzeb, Lb, Eb, hlb[0], hlb[1], cb, xbar);
-    side_rev<1>(R, hr[0], hr[1], x, E, tc, k, Beb, Fsb, byeb, bzeb, Rb, Eb, hrb[0], hrb[1], cb, xbar);
+    auto put = [&](int i, double v) { xbar[i] = v; };
+    side_rev<0>(L, hl[0], hl[1], x, E, tc, k, Beb, Fsb, byeb, bzeb, Lb, Eb, hlb[0], hlb[1], cb, put);
+    side_rev<1>(R, hr[0], hr[1], x, E, tc, k, Beb, Fsb, byeb, bzeb, Rb, Eb, hrb[0], hrb[1], cb, put);
     // Be's start: tunshift(Bz), Bz = gm1 den_e tshift(m1) + gm3 We
     {
         double Bzb[5];

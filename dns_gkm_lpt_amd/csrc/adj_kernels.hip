@@ -26,7 +26,7 @@
 // kernels (x: n = x, a = y, b = z; y: n = y, a = x, b = z; z: n = z, a = x, b = y).
 #include "adj_kernels.hpp"
 
-#include "adj_flux.hpp"
+#include "adj_pair.hpp"
 #include "adj_math.hpp"
 #include "gkm_dual.hpp"
 #include "gkm_flux.hpp"
@@ -176,29 +176,70 @@ __global__ __launch_bounds__(256, 2) void tl_update_kernel(const double* __restr
 // ---------------------------------------------------------------------------
 // Xbar[k][f] = sum_q Fbar_q dF_q / dx_k for the 50 flux inputs of face f, with
 // Fbar = -(1/dx) (lam(cell n) - lam(cell n+1)); stored by input group and lab slot.
+// Two lanes per face (adj_pair.hpp): neighbouring lanes take its two sides.
 template <int DIR>
 __global__ __launch_bounds__(256, 1) void flux_adj_kernel(const double* __restrict__ W, const double* __restrict__ WS,
                                                        const double* __restrict__ lam, long plane, int nc,
                                                        Gas<double> g, double dt, double dx,
                                                        double* __restrict__ Xbar)
 {
-    const long f = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (f >= plane) return;
+    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const int side = (int)(t & 1);
+    // lanes past the last face repeat it: the exchange needs every lane
+    const bool live = (t >> 1) < plane;
+    const long f = live ? t >> 1 : plane - 1;
     int n, a, b;
     coords_of<DIR>(f, nc, n, a, b);
     const long fr = cell_at<DIR>(wrap(n + 1, nc), a, b, nc);
-    const double inv_dx = 1.0 / dx;
-    double Fbar[5];
+    const long fam = cell_at<DIR>(n, wrap(a - 1, nc), b, nc), fap = cell_at<DIR>(n, wrap(a + 1, nc), b, nc);
+    const long fbm = cell_at<DIR>(n, a, wrap(b - 1, nc), nc), fbp = cell_at<DIR>(n, a, wrap(b + 1, nc), nc);
+    const long cell = side ? fr : f;
+    // the lane's first and second tangential direction
+    const long t0m = side ? fbm : fam, t0p = side ? fbp : fap, t1m = side ? fam : fbm, t1p = side ? fap : fbp;
+    const double two_idx = 2.0 / dx, half_idx = 0.5 / dx, inv_dx = 1.0 / dx;
+    // slot q of the lane's frame: lab variable var(q), sign(q) on states and tangential slopes
+    auto var = [&](int q) { return side && (q == 2 || q == 3) ? phys<DIR>(5 - q) : phys<DIR>(q); };
+    auto sign = [&](int q) { return side && q == 1 ? -1.0 : 1.0; };
+    __shared__ double set[AdjPark::kDoubles * 256];
+    const AdjPark pk{set + threadIdx.x, 256};
+    double Fbar[5], C[5];
+#pragma unroll
     for (int q = 0; q < 5; q++) {
-        const int p = phys<DIR>(q);
+        const int p = var(q);
+        const double m = sign(q);
+        const double* ws = WS + (long)(5 * side + p) * plane;
+        const double s = m * ws[f];
+        C[q] = m * W[p * plane + cell];
+        pk(AdjPark::kC + q) = C[q];
+        pk(AdjPark::kS + q) = s;
+        pk(AdjPark::kN + q) = (s - C[q]) * two_idx;
+        pk(AdjPark::kT + q) = m * ((ws[t0p] - ws[t0m]) * half_idx);
+        pk(AdjPark::kT + 5 + q) = m * ((ws[t1p] - ws[t1m]) * half_idx);
+        // the flux of lane 1's frame: -F0, F1, -F3, -F2, -F4
         Fbar[q] = -inv_dx * (lam[p * plane + f] - lam[p * plane + fr]);
+        if (side && q != 1) Fbar[q] = -Fbar[q];
     }
-    auto get = [&](int arr, int v, long idx) { return arr == 0 ? W[v * plane + idx] : WS[v * plane + idx]; };
-    double x[50];
-    gather_inputs<DIR, double>(n, a, b, nc, plane, dx, get, x);
-    double xbar[50];
-    face_flux_vjp(x, dt, dx, g, Fbar, xbar);
-    for (int k = 0; k < 50; k++) Xbar[(long)(5 * (k / 5) + phys<DIR>(k % 5)) * plane + f] = xbar[k];
+    // the collision time is the left cell's
+    double tau = collision_time<double>(C, g);
+    const double other = PairSwap{}(tau);
+    tau = side ? other : tau;
+    pk.fence();
+    // groups: cell, WENO state, normal slope (D0 / D1), slopes along a (D2 / D3) and b (D4 / D5)
+    const double taub = face_flux_vjp_pair(pk, tau, dt, dx, g, Fbar, PairSwap{}, [&](int i, double v) {
+        const int q = i % 5, grp = i / 10;
+        const int at = 10 * grp + 5 * side + (side ? (grp == 3 ? 10 : (grp == 4 ? -10 : 0)) : 0);
+        if (live) Xbar[(long)(at + var(q)) * plane + f] = (grp == 2 && side ? -sign(q) : sign(q)) * v;
+    });
+    // the cell again, for its collision time's derivative
+    double dtau[5];
+    pk.fence();
+#pragma unroll
+    for (int q = 0; q < 5; q++) C[q] = sign(q) * W[var(q) * plane + cell];
+    collision_time_vjp(C, g, dtau);
+    if (live)
+#pragma unroll
+        for (int q = 0; q < 5; q++)
+            Xbar[(long)(5 * side + var(q)) * plane + f] = sign(q) * (pk(AdjPark::kC + q) + (side ? 0.0 : taub * dtau[q]));
 }
 
 // adjoints of the WENO states (WSbar, 10 per face) and of the face's two cells
@@ -348,7 +389,8 @@ hipError_t adj_dir(const double* W, const double* lam, long plane, int nc, const
     hipLaunchKernelGGL(weno_faces_kernel<DIR>, dim3(nb), dim3(256), 0, st, W, nullptr, plane, nc, g, s.WS, nullptr);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(flux_adj_kernel<DIR>, dim3(nb), dim3(256), 0, st, W, s.WS, lam, plane, nc, g, dt, dx, s.Xbar);
+    hipLaunchKernelGGL(flux_adj_kernel<DIR>, dim3(blocks_of(2 * plane)), dim3(256), 0, st, W, s.WS, lam, plane, nc, g, dt,
+                       dx, s.Xbar);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     hipLaunchKernelGGL(adj_assemble_kernel<DIR>, dim3(nb), dim3(256), 0, st, s.Xbar, plane, nc, dx, s.WSbar, s.CL, s.CR);
     if ((e = hipGetLastError()) != hipSuccess) return e;

@@ -82,7 +82,7 @@ __host__ __device__ __forceinline__ void gks_flux_pair(const IN& in, double tau,
     }
     {   // pressure-jump term of the collision time (GKMflux.cpp:156-157)
         const T pa = T(2) * S.den * S.i2l, pb = sw(pa);  // rho / lambda of the two sides
-        tau = tau + dt * g_div(fabs(pa - pb), fabs(pa + pb));
+        tau = tau + dt * g_div(::fabs(pa - pb), ::fabs(pa + pb));
     }
     // half-space u table of the side, entries 0 and 1 (gkm_flux.hpp)
     T h0, h1;
