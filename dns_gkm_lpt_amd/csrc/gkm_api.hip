@@ -48,7 +48,7 @@ struct gkm_ctx {
     int* dflag = nullptr;          // in dscal[3]: non-physical-state flag, ticket of the step's CFL
     double* hscal = nullptr;       // pinned copy of dscal
     double* partial = nullptr;     // CFL block maxima
-    double* faces = nullptr;       // face fluxes of the three directions (small FP64 grids)
+    double* faces = nullptr;       // face fluxes of the three directions (small grids)
     double* hist = nullptr;        // behind dscal: dt of the last kHist steps of gkm_run
     bool have_state = false;
     int tile[3] = {0, 0, 0};       // sweep tile variant per direction
@@ -134,13 +134,19 @@ gkm::SweepArgs sweep_args(const gkm_ctx* c, int dir, int mode)
 }
 
 // Two launches instead of three sweeps (gkm::launch_small_step) where the grid
-// is small and nothing asks for the sweeps one by one; the results are the same.
-bool small_step(const gkm_ctx* c) { return c->faces && !c->timing && !c->compensate; }
+// is small and nothing asks for the sweeps one by one; the results are those of
+// the sweeps in their first tile variants.  Mixed variants round differently
+// (FP32 contractions), so a mixed context with another one keeps its sweeps.
+bool small_step(const gkm_ctx* c)
+{
+    const bool first = !c->tile[0] && !c->tile[1] && !c->tile[2];
+    return c->faces && !c->timing && (first || c->cfg.precision != GKM_MIXED);
+}
 
 int eulerian_step(gkm_ctx* c)
 {
     if (small_step(c)) {
-        HIPCHK(c, gkm::launch_small_step(sweep_args(c, 0, 0), c->faces, nullptr, c->stream));
+        HIPCHK(c, gkm::launch_small_step(sweep_args(c, 0, 0), c->faces, nullptr, c->slots, c->cfg.precision == GKM_MIXED, c->stream));
         c->cur = 1 - c->cur;
         c->lpt.valid = false;
         return GKM_OK;
@@ -224,7 +230,7 @@ int gkm_create(const gkm_config* cfg, gkm_ctx** out)
     const bool mixed = cfg->precision == GKM_MIXED;
     const size_t state = 5 * (size_t)c->plane, staged = 5 * (size_t)c->padded;
     // face fluxes of the two-launch step: the y and z directions' behind dW's 5 planes
-    const size_t faces = !mixed && gkm::small_step_ok(nc) ? 2 * state : 0;
+    const size_t faces = gkm::small_step_ok(nc, mixed) ? 2 * state : 0;
     const size_t carry = mixed ? (5 * (size_t)gkm::carry_plane(nc) + 1) / 2 : 0;  // floats, in doubles
     auto even = [](size_t n) { return (n + 31) & ~size_t(31); };               // 256 B
     const size_t sizes[] = {even(state), even(state), even(state + faces), even(staged), even(kScal + kHist),
@@ -413,7 +419,7 @@ int gkm_run(gkm_ctx* c, int nsteps, double* dt_hist)
             // the history's slot of step n + 1 may be one not yet fetched: fetch first
             if (dt_hist && (n + 1) % kHist == 0 && n + 1 < nsteps) HIPCHK(c, fetch(n + 1));
             const gkm::StepCfl next{c->gas.gam, c->cfg.cfl, c->partial, c->dscal, c->dscal + 1, hist(n + 1), c->dflag, c->dflag + 1};
-            HIPCHK(c, gkm::launch_small_step(sweep_args(c, 0, 0), c->faces, &next, c->stream));
+            HIPCHK(c, gkm::launch_small_step(sweep_args(c, 0, 0), c->faces, &next, c->slots, c->cfg.precision == GKM_MIXED, c->stream));
             c->cur = 1 - c->cur;
             c->lpt.valid = false;
         } else {
@@ -614,6 +620,21 @@ int gkm_autotune(gkm_ctx* c, int reps, int tile[3], double ms[9])
     int rc = cfl_on_device(c);
     if (rc) return rc;
     const bool mixed = c->cfg.precision == GKM_MIXED;
+    // average time of a launch after one warm-up
+    auto average = [&](auto launch, double* avg) -> int {
+        float el = 0.f;
+        for (int r = -1; r < reps; r++) {
+            if (r == 0) HIPCHK(c, hipEventRecord(c->ev[0], c->stream));
+            const hipError_t e = launch();
+            if (e != hipSuccess) return fail(c, GKM_EHIP, std::string("kernel launch: ") + hipGetErrorString(e));
+        }
+        HIPCHK(c, hipEventRecord(c->ev[1], c->stream));
+        HIPCHK(c, hipEventSynchronize(c->ev[1]));
+        HIPCHK(c, hipEventElapsedTime(&el, c->ev[0], c->ev[1]));
+        *avg = el / reps;
+        return GKM_OK;
+    };
+    double sweeps = 0.0;  // the picks together
     for (int dir = 0; dir < 3; dir++) {
         double best = 0.0;
         int best_v = c->tile[dir];
@@ -627,18 +648,9 @@ int gkm_autotune(gkm_ctx* c, int reps, int tile[3], double ms[9])
             a.seg = gkm::sweep_seg_len(dir, c->nc, v, c->slots, mixed);
             a.nseg = gkm::sweep_nseg(c->nc, a.seg);
             // dW is scratch and Wout is the next state's buffer: the resident state is not changed
-            hipError_t e = gkm::launch_sweep(dir, a, mixed, c->stream);  // warm-up
-            if (e != hipSuccess) return fail(c, GKM_EHIP, std::string("kernel launch: ") + hipGetErrorString(e));
-            HIPCHK(c, hipEventRecord(c->ev[0], c->stream));
-            for (int r = 0; r < reps; r++) {
-                e = gkm::launch_sweep(dir, a, mixed, c->stream);
-                if (e != hipSuccess) return fail(c, GKM_EHIP, std::string("kernel launch: ") + hipGetErrorString(e));
-            }
-            HIPCHK(c, hipEventRecord(c->ev[1], c->stream));
-            HIPCHK(c, hipEventSynchronize(c->ev[1]));
-            float el = 0.f;
-            HIPCHK(c, hipEventElapsedTime(&el, c->ev[0], c->ev[1]));
-            const double avg = el / reps;
+            double avg = 0.0;
+            rc = average([&] { return gkm::launch_sweep(dir, a, mixed, c->stream); }, &avg);
+            if (rc) return rc;
             if (ms) ms[3 * dir + v] = avg;
             if (best == 0.0 || avg < best) {
                 best = avg;
@@ -646,6 +658,16 @@ int gkm_autotune(gkm_ctx* c, int reps, int tile[3], double ms[9])
             }
         }
         c->tile[dir] = best_v;
+        sweeps += best;
+    }
+    if (c->faces && mixed) {
+        // the two-launch step goes with the first variants: keep them where it is faster
+        double avg = 0.0;
+        rc = average([&] { return gkm::launch_small_step(sweep_args(c, 0, 0), c->faces, nullptr, c->slots, true, c->stream); },
+                     &avg);
+        if (rc) return rc;
+        if (avg < sweeps)
+            for (int d = 0; d < 3; d++) c->tile[d] = 0;
     }
     if (tile)
         for (int d = 0; d < 3; d++) tile[d] = c->tile[d];

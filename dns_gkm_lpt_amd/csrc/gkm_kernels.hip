@@ -43,38 +43,43 @@ __global__ __launch_bounds__(256, 2) void ens_sweep_kernel(const SweepArgs* __re
 static int cdiv(int a, int b) { return (a + b - 1) / b; }
 
 // ---------------------------------------------------------------------------
-// FP64 step of a small grid in two launches.  A 32^3 sweep is 256 workgroups of
-// two chunks, one of them the lead-in: three sweeps in turn leave half the chip
-// idle, do every face twice and pay three launches.  Here one launch computes
-// the face fluxes of all three directions (independent of each other), one chunk
-// per workgroup and no lead-in, and a second one the update (the sweeps'
-// expressions in their order: equal to them bit for bit) and, in a free-running
-// loop, the CFL maximum of the new state; its last workgroup forms the next dt.
+// Step of a small grid in two launches.  A 32^3 sweep is 256 workgroups of two
+// chunks, one of them the lead-in: three sweeps in turn leave half the chip idle,
+// do every face twice and pay three launches.  Here one launch computes the face
+// fluxes of all three directions (independent of each other) with no lead-in,
+// and a second one the update (the sweeps' expressions in their order: equal to
+// them bit for bit) and, in a free-running loop, the CFL maximum of the new
+// state; its last workgroup forms the next dt.  On a grid that no tile divides
+// the last pencils and segments move back into the grid, where the sweeps' reach
+// past it and mask (100^3 mixed, us per step: 647 -> 418).
 // ---------------------------------------------------------------------------
 struct FaceArgs {
     SweepArgs dir[3];
     int first[4];  // blocks [first[d], first[d+1]) sweep direction d
 };
-template <bool GEN>
+template <bool MIX>
 __global__ __launch_bounds__(256, 2) void faces_kernel(FaceArgs a)
 {
-    __shared__ double lds[max3(sweep_lds_doubles<0, 0, false>(), sweep_lds_doubles<1, 0, false>(), sweep_lds_doubles<2, 0, false>())];
+    __shared__ double lds[max3(sweep_lds_doubles<0, 0, MIX>(), sweep_lds_doubles<1, 0, MIX>(), sweep_lds_doubles<2, 0, MIX>())];
     const int b = blockIdx.x;
-    if (b < a.first[1]) sweep_body_pair<0, 0, true, GEN, true>(a.dir[0], b, a.first[1], true, lds);
-    else if (b < a.first[2]) sweep_body_pair<1, 0, true, GEN, true>(a.dir[1], b - a.first[1], a.first[2] - a.first[1], true, lds);
-    else sweep_body_pair<2, 0, true, GEN, true>(a.dir[2], b - a.first[2], a.first[3] - a.first[2], true, lds);
+    if (b < a.first[1]) sweep_body<0, MIX, 0, true, false, 0, true>(a.dir[0], b, a.first[1], true, lds);
+    else if (b < a.first[2]) sweep_body<1, MIX, 0, true, false, 0, true>(a.dir[1], b - a.first[1], a.first[2] - a.first[1], true, lds);
+    else sweep_body<2, MIX, 0, true, false, 0, true>(a.dir[2], b - a.first[2], a.first[3] - a.first[2], true, lds);
 }
 
 struct UpdateArgs {
     const double* W;
     double* Wout;
     const double* F;  // 3 directions x 5 planes
+    const float* cmp_in;  // compensated update (SweepArgs): the carried errors
+    float* cmp_out;
     long plane;
     int nc;
     double inv_dx, gam, cfl, dx;
     double *partial, *dt, *vmax, *hist;  // partial = nullptr: no CFL
     int *bad, *ticket;
 };
+template <bool CMP>
 __global__ __launch_bounds__(256) void step_update_kernel(UpdateArgs a)
 {
     const int nc = a.nc;
@@ -91,7 +96,16 @@ __global__ __launch_bounds__(256) void step_update_kernel(UpdateArgs a)
             const double *Fx = a.F + q * a.plane, *Fy = Fx + 5 * a.plane, *Fz = Fy + 5 * a.plane;
             const double dW = (Fx[c] - Fx[cx]) + (Fy[c] - Fy[cy]);
             const double dF = Fz[c] - Fz[cz];
-            t[q] = a.W[q * a.plane + c] - a.inv_dx * (dW + dF);
+            if constexpr (CMP) {  // TwoSum, as in sweep_body
+                const long co = q * carry_plane(nc) + carry_index(y, x, z, nc);
+                const double w = a.W[q * a.plane + c];
+                const double d = (double)a.cmp_in[co] - a.inv_dx * (dW + dF);
+                t[q] = w + d;
+                const double dv = t[q] - w;
+                a.cmp_out[co] = (float)((w - (t[q] - dv)) + (d - dv));
+            } else {
+                t[q] = a.W[q * a.plane + c] - a.inv_dx * (dW + dF);
+            }
             a.Wout[q * a.plane + c] = t[q];
         }
         if (a.partial) cfl_cell(t[0], t[1], t[2], t[3], t[4], a.gam, m, bad);
@@ -116,37 +130,76 @@ __global__ __launch_bounds__(256) void step_update_kernel(UpdateArgs a)
     cfl_reduce(a.partial, gridDim.x, a.cfl, a.dx, a.dt, a.vmax, a.bad, a.hist);
 }
 
-bool small_step_ok(int nc)
+static const int* tile_shape(int dir, int tile, bool mixed) { return mixed ? kTiles[dir][tile] : kTilesPair[dir][tile]; }
+
+bool small_step_ok(int nc, bool mixed)
 {
-    bool ok = nc >= 16 && nc <= kSmallNc;
+    bool ok = nc >= 16 && !(mixed && nc % 2) && nc <= (mixed ? kSmallNcMixed : kSmallNc);
     for (int d = 0; d < 3; d++) {
-        const int* t = kTilesPair[d][0];
+        const int* t = tile_shape(d, 0, mixed);
         ok = ok && t[0] + 3 <= nc && t[1] <= nc && t[2] <= nc;
     }
     return ok;
 }
 
-hipError_t launch_small_step(const SweepArgs& a, double* F, const StepCfl* cfl, hipStream_t s)
+// segments of at most `most` chunks of CN faces: in equal parts where CN divides
+// the line (the segment then divides the grid too: sweep_exact)
+static int equal_parts(int nc, int CN, int most)
 {
-    if (!small_step_ok(a.nc) || !F || a.cmp_out) return hipErrorInvalidValue;
+    const int lchunks = cdiv(nc, CN);
+    int parts = cdiv(lchunks, most);
+    if (nc % CN == 0)
+        while (lchunks % parts) parts++;
+    return cdiv(lchunks, parts) * CN;
+}
+
+// Faces per workgroup of faces_kernel along the sweep axis.  A workgroup's chunks
+// pay one start (FP64: the ring's window, half a chunk; mixed: a quarter) and the
+// launch ends a quarter of a workgroup's time after the slots run dry, so longer segments
+// pay on larger grids only (us per step at 1 / 2 / 4 / 8 chunks, FP64: 32^3 29 /
+// 32 / 35 / 51, 64^3 135 / 125 / 122 / 123, 128^3 898 / 805 / 773 / 765; mixed:
+// 32^3 31 / 34 / 49 / 82, 128^3 813 / 793 / 762 / 767).
+static int faces_seg_len(int dir, int nc, int slots, bool mixed)
+{
+    const int* t = tile_shape(dir, 0, mixed);
+    const long pencils = (long)cdiv(nc, t[1]) * cdiv(nc, t[2]);
+    const double start = mixed ? 0.25 : 0.5;
+    int best = t[0];
+    double cost = -1.0;
+    for (int k = 1; k <= 8; k++) {
+        const int seg = equal_parts(nc, t[0], k);
+        if (seg > nc) break;
+        const double chunks = seg / t[0] + start;
+        const double c = (double)(pencils * sweep_nseg(nc, seg)) / slots * chunks + 0.25 * chunks;
+        if (cost < 0.0 || c < cost) {
+            cost = c;
+            best = seg;
+        }
+    }
+    return best;
+}
+
+hipError_t launch_small_step(const SweepArgs& a, double* F, const StepCfl* cfl, int slots, bool mixed, hipStream_t s)
+{
+    if (!small_step_ok(a.nc, mixed) || !F || (a.cmp_out != nullptr) != (a.cmp_in != nullptr) || (a.cmp_out && !mixed))
+        return hipErrorInvalidValue;
     FaceArgs f{};
-    bool gen = false;
     for (int d = 0; d < 3; d++) {
         f.dir[d] = a;
         f.dir[d].tile = 0;
         f.dir[d].mode = 0;
         f.dir[d].dW = F + (long)d * 5 * a.plane;
-        const int* t = kTilesPair[d][0];
-        f.dir[d].seg = t[0];  // one chunk per workgroup
-        f.dir[d].nseg = sweep_nseg(a.nc, t[0]);
+        const int* t = tile_shape(d, 0, mixed);
+        f.dir[d].seg = faces_seg_len(d, a.nc, slots, mixed);
+        f.dir[d].nseg = sweep_nseg(a.nc, f.dir[d].seg);
         f.first[d + 1] = f.first[d] + cdiv(a.nc, t[1]) * cdiv(a.nc, t[2]) * f.dir[d].nseg;
-        gen = gen || a.nc % t[0] || a.nc % t[1] || a.nc % t[2];
     }
-    if (gen) hipLaunchKernelGGL(faces_kernel<true>, dim3(f.first[3]), dim3(256), 0, s, f);
-    else hipLaunchKernelGGL(faces_kernel<false>, dim3(f.first[3]), dim3(256), 0, s, f);
+    const dim3 grid(f.first[3]), block(256);
+    if (mixed) hipLaunchKernelGGL(faces_kernel<true>, grid, block, 0, s, f);
+    else hipLaunchKernelGGL(faces_kernel<false>, grid, block, 0, s, f);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    UpdateArgs u{a.W, a.Wout, F, a.plane, a.nc, a.inv_dx, 0.0, 0.0, a.dx, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
+    UpdateArgs u{a.W, a.Wout, F, a.cmp_in, a.cmp_out, a.plane, a.nc, a.inv_dx, 0.0, 0.0, a.dx, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
     if (cfl) {
         u.gam = cfl->gam;
         u.cfl = cfl->cfl;
@@ -160,7 +213,8 @@ hipError_t launch_small_step(const SweepArgs& a, double* F, const StepCfl* cfl, 
     // with the CFL one maximum and one ticket per block: two blocks per CU
     const long all = (a.plane + 255) / 256, blocks = cfl && all > 512 ? 512 : all;
     static_assert(512 <= kCflBlocks, "a partial maximum per block");
-    hipLaunchKernelGGL(step_update_kernel, dim3((unsigned)blocks), dim3(256), 0, s, u);
+    if (a.cmp_out) hipLaunchKernelGGL(step_update_kernel<true>, dim3((unsigned)blocks), block, 0, s, u);
+    else hipLaunchKernelGGL(step_update_kernel<false>, dim3((unsigned)blocks), block, 0, s, u);
     return hipGetLastError();
 }
 
@@ -187,8 +241,6 @@ bool sweep_grid_ok(int nc)
 {
     return nc >= 16 && sweep_first_tile(0, nc) >= 0 && sweep_first_tile(1, nc) >= 0 && sweep_first_tile(2, nc) >= 0;
 }
-
-static const int* tile_shape(int dir, int tile, bool mixed) { return mixed ? kTiles[dir][tile] : kTilesPair[dir][tile]; }
 
 int sweep_seg_len(int dir, int nc, int tile, int slots, bool mixed)
 {
@@ -221,15 +273,8 @@ int sweep_seg_len(int dir, int nc, int tile, int slots, bool mixed)
 
 int sweep_seg_most(int dir, int nc, int tile, int most, bool mixed)
 {
-    // at most `most` chunks per workgroup, in equal parts where the tile divides
-    // the line (the segment then divides the grid too: sweep_exact)
     if (!sweep_tile_ok(dir, tile, nc) || most < 1) return 0;
-    const int CN = tile_shape(dir, tile, mixed)[0];
-    const int lchunks = cdiv(nc, CN);
-    int parts = cdiv(lchunks, most);
-    if (nc % CN == 0)
-        while (lchunks % parts) parts++;
-    return cdiv(lchunks, parts) * CN;
+    return equal_parts(nc, tile_shape(dir, tile, mixed)[0], most);
 }
 
 template <int DIR, int V>

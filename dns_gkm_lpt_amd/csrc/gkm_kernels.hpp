@@ -103,20 +103,27 @@ hipError_t launch_cfl(const double* W, long plane, double gam, double cfl, doubl
 // *p = v in stream order (a scalar the caller need not keep)
 hipError_t launch_set_scalar(double* p, double v, hipStream_t s);
 
-// FP64 step of a small grid in two launches: the face fluxes of the three
-// directions, then the update and, with cfl, the dt of the new state.  F holds
-// 15 plane doubles.  Equal to the three sweeps bit for bit.  us per step with
-// dt, this / the sweeps and the CFL pass: 16^3 16 / 44, 32^3 29 / 57, 64^3 123 /
-// 160, 80^3 229 / 266, 96^3 381 / 411, 128^3 907 / 764 (the fluxes' round trip
-// through memory outweighs the lead-in chunks).
-constexpr int kSmallNc = 96;
-bool small_step_ok(int nc);
+// Step of a small grid in two launches: the face fluxes of the three
+// directions, then the update (compensated with cmp_out) and, with cfl, the dt of
+// the new state.  F holds 15 plane doubles, slots as in sweep_seg_len.  Equal to
+// the three sweeps with their first tile variants bit for bit.  us per step with
+// dt, this / the sweeps and the CFL pass, FP64: 32^3 29 / 49, 64^3 125 / 151, 96^3
+// 345 / 427, 128^3 770 / 790, 160^3 1527 / 1660, 176^3 2079 / 2090, 200^3 3057 /
+// 2907, 256^3 6470 / 5997; mixed: 32^3 30 / 72, 64^3 119 / 166, 96^3 343 / 466, 128^3
+// 765 / 856, 192^3 2635 / 2963, 240^3 5153 / 5806, 256^3 6290 / 6410, 384^3 21470 /
+// 21330.  Each line lies where the fluxes' round trip through memory (and the
+// 10 planes more it holds) begins to outweigh the lead-in chunks and the three
+// launches' ends.  Mixed: even grids only, since the x and y sweeps reconstruct
+// faces in pairs whose two members round differently, and a segment moved back
+// by an odd number of faces would change the pairs.
+constexpr int kSmallNc = 160, kSmallNcMixed = 256;
+bool small_step_ok(int nc, bool mixed);
 struct StepCfl {
     double gam, cfl;
     double *partial, *dt, *vmax, *hist;  // hist may be nullptr
     int *bad, *ticket;                   // ticket: 0 before the first launch, left 0
 };
-hipError_t launch_small_step(const SweepArgs& a, double* F, const StepCfl* cfl, hipStream_t s);
+hipError_t launch_small_step(const SweepArgs& a, double* F, const StepCfl* cfl, int slots, bool mixed, hipStream_t s);
 // ensemble CFL: one dt per member (partial holds nmem * kEnsCflBlocks doubles)
 struct CflArgs {
     const double* W;

@@ -1,7 +1,7 @@
 // gkm_noalloc.hip -- gkm_step_noalloc: one Eulerian step on caller-owned device
 // buffers with no device allocation (declared in include/dnsgkm.h).
 //
-// The step's scratch -- the face fluxes of the three directions (FP64, 15 nc^3
+// The step's scratch -- the face fluxes of the three directions (15 nc^3
 // doubles; gkm::launch_small_step) or the flux-difference accumulator of the x
 // and y sweeps (5 nc^3), and the device dt they read -- lives in the
 // file-scope array `scratch` below, sized for nc <= kNoallocMaxNc.  Each GPU
@@ -111,8 +111,8 @@ extern "C" int gkm_step_noalloc(const gkm_config* cfg, const double* W, double* 
         a.seg = gkm::sweep_seg_len(dir, nc, a.tile, slots, mixed);
         a.nseg = gkm::sweep_nseg(nc, a.seg);
         a.mode = dir;  // x: dW = dF, y: dW += dF, z: Wout = W - (dW + dF)/dx
-        if (dir == 0 && !mixed && gkm::small_step_ok(nc)) {
-            e = gkm::launch_small_step(a, sc, nullptr, s);
+        if (dir == 0 && gkm::small_step_ok(nc, mixed)) {
+            e = gkm::launch_small_step(a, sc, nullptr, slots, mixed, s);
             if (e != hipSuccess) return put_msg(msg, msglen, GKM_EHIP, std::string("step launch: ") + hipGetErrorString(e));
             break;
         }

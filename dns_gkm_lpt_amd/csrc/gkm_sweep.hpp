@@ -128,8 +128,10 @@ constexpr int sweep_lds_max()
 template <bool MIX>
 constexpr int kSweepLdsMax = max3(sweep_lds_max<0, MIX>(), sweep_lds_max<1, MIX>(), sweep_lds_max<2, MIX>());
 
-// workgroup -> pencil corner (a0, b0) and segment s of one grid (member)
-template <int DIR, int CA, int CB, bool GEN>
+// workgroup -> pencil corner (a0, b0) and segment s of one grid (member).
+// FACES: a pencil that would reach past the grid is moved back into it; it takes
+// some lines of its neighbour a second time, to the same values.
+template <int DIR, int CA, int CB, bool GEN, bool FACES = false>
 __device__ __forceinline__ void sweep_pencil(const SweepArgs& p, int bid, int nblk, bool remap, int& a0, int& b0, int& s)
 {
     const int nc = p.nc;
@@ -138,7 +140,7 @@ __device__ __forceinline__ void sweep_pencil(const SweepArgs& p, int bid, int nb
     if (remap && (nblk & 7) == 0) bid = (bid & 7) * (nblk >> 3) + (bid >> 3);
     s = bid % p.nseg;
     const int pencil = bid / p.nseg;
-    const int npb = GEN ? (nc + CB - 1) / CB : nc / CB;  // pencils across b; with GEN the last may reach past nc
+    const int npb = GEN || FACES ? (nc + CB - 1) / CB : nc / CB;  // pencils across b; with GEN the last may reach past nc
     // z sweep on an exact grid: pencils in 8 x 8 patches, so that the ~64
     // workgroups an XCD runs at once cover a square of lines whose tangential
     // edge lines are mostly interior lines of the same patch, read once into
@@ -146,7 +148,7 @@ __device__ __forceinline__ void sweep_pencil(const SweepArgs& p, int bid, int nb
     // 512^3: z sweep 19.55 -> 19.22 ms mixed, 25.44 -> 24.79 ms FP64).  The
     // x and y sweeps keep the row order, which measured faster for them.
     int pa, pb;
-    if (DIR == 2 && !GEN && (npb & 7) == 0 && ((nc / CA) & 7) == 0) {
+    if (DIR == 2 && !GEN && !FACES && (npb & 7) == 0 && ((nc / CA) & 7) == 0) {
         const int t = pencil >> 6, w = pencil & 63, tpb = npb >> 3;
         pa = (t / tpb) * 8 + (w >> 3);
         pb = (t % tpb) * 8 + (w & 7);
@@ -156,6 +158,10 @@ __device__ __forceinline__ void sweep_pencil(const SweepArgs& p, int bid, int nb
     }
     a0 = pa * CA;
     b0 = pb * CB;
+    if (FACES) {
+        a0 = a0 < nc - CA ? a0 : nc - CA;
+        b0 = b0 < nc - CB ? b0 : nc - CB;
+    }
 }
 
 // thread -> face of the chunk: the fastest index is the one contiguous in
@@ -329,13 +335,13 @@ __device__ __forceinline__ void sweep_body_pair(const SweepArgs& p, int bid, int
     const long plane = p.plane;
     const double* __restrict__ W = p.W;
     int a0, b0, s;
-    sweep_pencil<DIR, CA, CB, GEN>(p, bid, nblk, remap, a0, b0, s);
+    sweep_pencil<DIR, CA, CB, GEN, FACES>(p, bid, nblk, remap, a0, b0, s);
 
     const int tid = threadIdx.x;
     const double dt = *p.dt;
     const double dx = p.dx;
     const int nchunk = p.seg / CN;
-    const int seg0 = s * p.seg;
+    const int seg0 = FACES && s * p.seg > nc - p.seg ? nc - p.seg : s * p.seg;
     const int seg_end = seg0 + p.seg < nc ? seg0 + p.seg : nc;
 
     // the thread's line and cell (loads, WENO)
@@ -508,11 +514,12 @@ __device__ __forceinline__ void sweep_body_pair(const SweepArgs& p, int bid, int
 // general form's extra live values made the mixed x and y sweeps spill).
 // CMP (the z sweep's update): -1 compensated when p.cmp_out is set, 0 plain,
 // 1 compensated (the fixed forms leave the other update out of the kernel).
-template <int DIR, bool MIX, int V, bool EXT = false, bool GEN = true, int CMP = -1>
+// FACES as in sweep_body_pair.
+template <int DIR, bool MIX, int V, bool EXT = false, bool GEN = true, int CMP = -1, bool FACES = false>
 __device__ __forceinline__ void sweep_body(const SweepArgs& p, int bid, int nblk, bool remap, double* lds = nullptr)
 {
     if constexpr (!MIX) {
-        sweep_body_pair<DIR, V, EXT, GEN>(p, bid, nblk, remap, lds);
+        sweep_body_pair<DIR, V, EXT, GEN, FACES>(p, bid, nblk, remap, lds);
         return;
     } else {
     constexpr int CN = Tile<DIR, V, true>::CN, CA = Tile<DIR, V, true>::CA, CB = Tile<DIR, V, true>::CB;
@@ -535,7 +542,7 @@ __device__ __forceinline__ void sweep_body(const SweepArgs& p, int bid, int nblk
     const double* __restrict__ W = p.W;
 
     int a0, b0, s;
-    sweep_pencil<DIR, CA, CB, GEN>(p, bid, nblk, remap, a0, b0, s);
+    sweep_pencil<DIR, CA, CB, GEN, FACES>(p, bid, nblk, remap, a0, b0, s);
 
     const int tid = threadIdx.x;
     int tn, ta, tb;
@@ -548,7 +555,7 @@ __device__ __forceinline__ void sweep_body(const SweepArgs& p, int bid, int nblk
     const double dt = *p.dt;
     const double dx = p.dx;
     const int nchunk = p.seg / CN;
-    const int seg0 = s * p.seg;
+    const int seg0 = FACES && s * p.seg > nc - p.seg ? nc - p.seg : s * p.seg;
     const int seg_end = seg0 + p.seg < nc ? seg0 + p.seg : nc;
 
     SweepIn<DIR, CN, L> in;
@@ -564,7 +571,7 @@ __device__ __forceinline__ void sweep_body(const SweepArgs& p, int bid, int nblk
     in.two_idx = p.two_idx;
     in.half_idx = p.half_idx;
 
-    for (int c = -1; c < nchunk; ++c) {
+    for (int c = FACES ? 0 : -1; c < nchunk; ++c) {
         const int n0 = seg0 + c * CN;  // first face of the chunk (may be < 0 for the lead-in)
 
         weno_chunk<DIR, CN, CA, CB, NT>(p, n0, a0, b0, tid, sW);
@@ -596,6 +603,15 @@ __device__ __forceinline__ void sweep_body(const SweepArgs& p, int bid, int nblk
             }
             double F[5];
             gks_flux_tf<double, float>(in, tau, dt, dx, p.g, F);
+            if constexpr (FACES) {
+                if (upd) {
+                    const long idx = cell_index<DIR>(n0 + tn, a0 + ta, b0 + tb, nc);
+#pragma unroll
+                    for (int q = 0; q < 5; q++) p.dW[in.phys(q) * plane + idx] = F[q];
+                }
+                __syncthreads();  // the next chunk's WENO rewrites sW
+                continue;
+            }
 #pragma unroll
             for (int q = 0; q < 5; q++) sF[sf_at<DIR, CN, CA * CB>(in.phys(q), tn + 1, lc)] = F[q];
         }

@@ -119,7 +119,8 @@ int gkm_set_sweep_tiles(gkm_ctx *ctx, const int tile[3]);
 int gkm_get_sweep_tiles(const gkm_ctx *ctx, int tile[3]);
 /* Time every tile variant of every sweep on the resident state (reps timed
  * launches each after one warm-up, the CFL dt of the state) and keep the
- * fastest per direction.  The resident state is not changed.  tile (may be
+ * fastest per direction -- or variant 0 in all three where a GKM_MIXED step of
+ * this grid in two launches, which goes with them, is faster.  The resident state is not changed.  tile (may be
  * NULL) receives the choice, ms (may be NULL, 9 doubles) the average launch
  * time of variant v of direction d at [3 d + v]. */
 int gkm_autotune(gkm_ctx *ctx, int reps, int tile[3], double ms[9]);

@@ -49,3 +49,41 @@ def test_small_step_reports_a_nonphysical_state():
         with pytest.raises(gl.GkmError) as e:
             c.run(2)
         assert e.value.code == 4
+
+
+@pytest.mark.parametrize("compensate", [True, False])
+@pytest.mark.parametrize("nc", [18, 20, 21, 32, 46, 100, 126, 128, 256])
+def test_mixed_small_step_equals_sweeps(nc, compensate):
+    """Mixed: first variants; state, carry and dt history bit for bit."""
+    W, P, _ = make_case(nc, seed=nc)
+    out = []
+    for timed in (False, True):
+        with gl.Context(nc, P, precision=gl.GKM_MIXED) as c:
+            c.set_compensation(compensate)
+            c.timing(timed)
+            c.upload(W)
+            dts = c.run(3, record_dt=True)
+            c.step(float(dts[-1]))
+            out.append((dts, c.cfl_dt(), c.download()) + ((c.download_carry(),) if compensate else ()))
+    for a, b in zip(*out):
+        np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("nc", [112, 127, 160, 161])
+def test_several_chunks_a_workgroup(nc):
+    """Segments of more than one chunk, ragged and moved back into the grid."""
+    test_small_step_equals_sweeps(nc)
+
+
+@pytest.mark.parametrize("nc", [32, 50])
+def test_mixed_context_with_other_tiles_keeps_its_sweeps(nc):
+    W, P, _ = make_case(nc, seed=1)
+    out = []
+    for timed in (False, True):
+        with gl.Context(nc, P, precision=gl.GKM_MIXED) as c:
+            c.set_tiles((2, 1, 2))
+            c.timing(timed)
+            c.upload(W)
+            c.run(3)
+            out.append(c.download())
+    np.testing.assert_array_equal(out[0], out[1])
