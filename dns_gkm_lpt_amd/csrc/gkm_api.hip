@@ -1110,9 +1110,9 @@ int lpt_coupled_step(gkm_ctx* c, double dt)
 
 // ---------------------------------------------------------------------------
 // Ensemble: independent members (own grid size, gas, IC, dt) stepped together.
-// Per step one launch computes every member's CFL dt (two kernels), and one
-// launch per direction sweeps every member (ens_sweep_kernel), so a step is
-// five launches whatever the number of members; a step from each buffer
+// Per step two launches compute every member's CFL dt, and the Eulerian step of
+// every member is two launches (launch_ens_small_step; three sweeps where a
+// member's grid has no two-launch step), whatever the number of members; a step from each buffer
 // parity is captured once into a HIP graph and replayed.  Each member is a
 // gkm_ctx, so its state goes in and out through gkm_upload_state /
 // gkm_download_state / gkm_stats_compute.  No reference counterpart.
@@ -1126,6 +1126,12 @@ struct gkm_ensemble {
     int tile[3] = {0, 0, 0};
     gkm::SweepArgs* dargs = nullptr;  // [parity][direction][member]
     int* dfirst = nullptr;            // [direction][member + 1] first block of each member
+    // the two-launch step (gkm::launch_ens_small_step), where every member has one
+    gkm::SweepArgs* dface = nullptr;  // [parity][direction][member]
+    gkm::UpdateArgs* dupd = nullptr;  // [parity][member]
+    int* dsfirst = nullptr;           // [3 member + 1] blocks of dface, [member + 1] of dupd
+    int nfblk = 0, nublk = 0;
+    bool small = false;
     int nblk[3] = {0, 0, 0};
     bool exact[3] = {false, false, false};  // per direction: tile and segment divide every member's grid
     bool compensated = false;               // every member's z sweep takes the compensated update
@@ -1281,6 +1287,44 @@ int ens_build(gkm_ensemble* e, const int t[3])
         e->exact[d] = exact;
     }
     e->compensated = ncomp == n;
+    // two launches where every member's step has them (small_step)
+    e->small = true;
+    double cells = 0.0;
+    for (int d = 0; d < 3; d++) e->tile[d] = t[d];
+    for (const gkm_ctx* c : e->mem) {
+        e->small = e->small && c->faces && (!e->mixed || (!t[0] && !t[1] && !t[2]));
+        cells += (double)c->plane;
+    }
+    if (e->small) {
+        std::vector<int> order(n), sfirst((size_t)4 * n + 2);
+        for (int m = 0; m < n; m++) order[m] = m;
+        // the largest members first: the launch ends on short workgroups
+        std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return e->mem[x]->nc > e->mem[y]->nc; });
+        std::vector<gkm::SweepArgs> face((size_t)6 * n);
+        std::vector<gkm::UpdateArgs> upd((size_t)2 * n);
+        int acc = 0, uacc = 0;
+        for (int d = 0; d < 3; d++)
+            for (int k = 0; k < n; k++) {
+                gkm_ctx* c = e->mem[order[k]];
+                for (int p = 0; p < 2; p++) {
+                    const gkm::SweepArgs a = ens_sweep_args(c, p, d, t[d], 1);
+                    face[((size_t)p * 3 + d) * n + k] = gkm::faces_args(a, c->faces, d, c->slots, (double)c->plane / cells, e->mixed);
+                    upd[(size_t)p * n + k] = gkm::update_args(a, c->faces);
+                }
+                sfirst[(size_t)d * n + k] = acc;
+                acc += gkm::faces_blocks(d, face[(size_t)d * n + k], e->mixed);
+                if (d == 0) {
+                    sfirst[(size_t)3 * n + 1 + k] = uacc;
+                    uacc += gkm::update_blocks(upd[k]);
+                }
+            }
+        sfirst[(size_t)3 * n] = e->nfblk = acc;
+        sfirst[(size_t)4 * n + 1] = e->nublk = uacc;
+        EHIPCHK(e, hipMemcpyAsync(e->dface, face.data(), sizeof(gkm::SweepArgs) * face.size(), hipMemcpyHostToDevice, e->stream));
+        EHIPCHK(e, hipMemcpyAsync(e->dupd, upd.data(), sizeof(gkm::UpdateArgs) * upd.size(), hipMemcpyHostToDevice, e->stream));
+        EHIPCHK(e, hipMemcpyAsync(e->dsfirst, sfirst.data(), sizeof(int) * sfirst.size(), hipMemcpyHostToDevice, e->stream));
+        EHIPCHK(e, hipStreamSynchronize(e->stream));  // the host vectors go out of scope
+    }
     std::vector<gkm::CflArgs> cfl((size_t)2 * n);
     for (int p = 0; p < 2; p++)
         for (int m = 0; m < n; m++) {
@@ -1294,7 +1338,6 @@ int ens_build(gkm_ensemble* e, const int t[3])
     EHIPCHK(e, hipMemcpyAsync(e->dcfl, cfl.data(), sizeof(gkm::CflArgs) * cfl.size(), hipMemcpyHostToDevice,
                               e->stream));
     EHIPCHK(e, hipStreamSynchronize(e->stream));  // the host vectors go out of scope
-    for (int d = 0; d < 3; d++) e->tile[d] = t[d];
     drop_graphs(e);
     return GKM_OK;
 }
@@ -1338,6 +1381,13 @@ gkm::PersistStep persist_args(const gkm_ensemble* e, int p)
     return a;
 }
 
+// the Eulerian part of a step from parity p in two launches
+hipError_t ens_small_step(gkm_ensemble* e, int p)
+{
+    return gkm::launch_ens_small_step(e->dface + (size_t)p * 3 * e->n, e->dsfirst, e->nfblk, e->dupd + (size_t)p * e->n,
+                                      e->dsfirst + 3 * e->n + 1, e->nublk, e->n, e->mixed, e->compensated, e->stream);
+}
+
 // capturing: the launches go into a HIP graph (the persistent step is then an
 // ordinary launch; eager persistent steps are cooperative launches)
 hipError_t ens_step(gkm_ensemble* e, int p, bool capturing)
@@ -1348,7 +1398,9 @@ hipError_t ens_step(gkm_ensemble* e, int p, bool capturing)
     hipError_t r = hipSuccess;
     if (np) r = lpt::launch_ens_sample(e->dpart + (size_t)(2 * p) * np, e->dpfirst, np, e->pblk, e->stream);
     if (r == hipSuccess) r = gkm::launch_ens_cfl(e->dcfl + (size_t)p * n, n, e->partial, e->stream);
-    for (int d = 0; d < 3 && r == hipSuccess; d++)
+    if (e->small && r == hipSuccess)
+        r = ens_small_step(e, p);
+    for (int d = 0; d < 3 && !e->small && r == hipSuccess; d++)
         r = gkm::launch_ens_sweep(d, e->tile[d], e->dargs + ((size_t)p * 3 + d) * n, e->dfirst + (size_t)d * (n + 1),
                                   n, e->nblk[d], e->mixed, e->exact[d], e->compensated, e->stream);
     if (np && r == hipSuccess)
@@ -1513,6 +1565,9 @@ int gkm_ensemble_create(int n, const gkm_config* cfgs, gkm_ensemble** out)
     EHIPCHK(e, hipEventCreate(&e->ev[1]));
     if (hipMalloc(&e->dargs, sizeof(gkm::SweepArgs) * 6 * (size_t)n) != hipSuccess ||
         hipMalloc(&e->dfirst, sizeof(int) * 3 * (size_t)(n + 1)) != hipSuccess ||
+        hipMalloc(&e->dface, sizeof(gkm::SweepArgs) * 6 * (size_t)n) != hipSuccess ||
+        hipMalloc(&e->dupd, sizeof(gkm::UpdateArgs) * 2 * (size_t)n) != hipSuccess ||
+        hipMalloc(&e->dsfirst, sizeof(int) * (4 * (size_t)n + 2)) != hipSuccess ||
         hipMalloc(&e->dcfl, sizeof(gkm::CflArgs) * 2 * (size_t)n) != hipSuccess ||
         hipMalloc(&e->partial, sizeof(double) * gkm::kEnsCflBlocks * (size_t)n) != hipSuccess)
         return efail(e, GKM_ENOMEM, "hipMalloc ensemble tables");
@@ -1537,6 +1592,9 @@ void gkm_ensemble_destroy(gkm_ensemble* e)
     for (gkm_ctx* c : e->mem) gkm_destroy(c);
     (void)hipFree(e->dargs);
     (void)hipFree(e->dfirst);
+    (void)hipFree(e->dface);
+    (void)hipFree(e->dupd);
+    (void)hipFree(e->dsfirst);
     (void)hipFree(e->dcfl);
     (void)hipFree(e->partial);
     for (void* ptr : {(void*)e->dpart, (void*)e->dpfirst, (void*)e->dz, (void*)e->dzfirst, (void*)e->dline,
@@ -1574,6 +1632,19 @@ int gkm_ensemble_autotune(gkm_ensemble* e, int reps, int tile[3], double ms[9])
     if (rc) return rc;
     const int n = e->n;
     EHIPCHK(e, gkm::launch_ens_cfl(e->dcfl + (size_t)p * n, n, e->partial, e->stream));  // every member's dt
+    // average time of a launch after one warm-up
+    auto average = [&](auto launch, double* avg) -> int {
+        float el = 0.f;
+        EHIPCHK(e, launch());
+        EHIPCHK(e, hipEventRecord(e->ev[0], e->stream));
+        for (int r = 0; r < reps; r++) EHIPCHK(e, launch());
+        EHIPCHK(e, hipEventRecord(e->ev[1], e->stream));
+        EHIPCHK(e, hipEventSynchronize(e->ev[1]));
+        EHIPCHK(e, hipEventElapsedTime(&el, e->ev[0], e->ev[1]));
+        *avg = el / reps;
+        return GKM_OK;
+    };
+    double sweeps = 0.0;  // the picks together
     int best[3];
     for (int d = 0; d < 3; d++) {
         double best_ms = 0.0;
@@ -1591,18 +1662,12 @@ int gkm_ensemble_autotune(gkm_ensemble* e, int reps, int tile[3], double ms[9])
             rc = ens_build(e, t);
             if (rc) return rc;
             // dW is scratch and Wout the next state's buffer: the members' states are not changed
-            auto launch = [&] {
+            double avg = 0.0;
+            rc = average([&] {
                 return gkm::launch_ens_sweep(d, v, e->dargs + ((size_t)p * 3 + d) * n, e->dfirst + (size_t)d * (n + 1),
                                              n, e->nblk[d], e->mixed, e->exact[d], e->compensated, e->stream);
-            };
-            EHIPCHK(e, launch());
-            EHIPCHK(e, hipEventRecord(e->ev[0], e->stream));
-            for (int r = 0; r < reps; r++) EHIPCHK(e, launch());
-            EHIPCHK(e, hipEventRecord(e->ev[1], e->stream));
-            EHIPCHK(e, hipEventSynchronize(e->ev[1]));
-            float el = 0.f;
-            EHIPCHK(e, hipEventElapsedTime(&el, e->ev[0], e->ev[1]));
-            const double avg = el / reps;
+            }, &avg);
+            if (rc) return rc;
             if (ms) ms[3 * d + v] = avg;
             if (first || avg < best_ms) {
                 best_ms = avg;
@@ -1614,6 +1679,22 @@ int gkm_ensemble_autotune(gkm_ensemble* e, int reps, int tile[3], double ms[9])
         t[d] = best[d];
         rc = ens_build(e, t);
         if (rc) return rc;
+        sweeps += best_ms;
+    }
+    if (e->mixed && !e->small) {
+        // the two-launch step goes with the first variants: keep them where it is faster
+        const int t[3] = {e->tile[0], e->tile[1], e->tile[2]}, zero[3] = {0, 0, 0};
+        bool ok = true;
+        for (gkm_ctx* c : e->mem) ok = ok && c->faces;
+        if (ok) {
+            double avg = 0.0;
+            rc = ens_build(e, zero);
+            if (rc) return rc;
+            rc = average([&] { return ens_small_step(e, p); }, &avg);
+            if (rc) return rc;
+            if (avg >= sweeps) rc = ens_build(e, t);
+            if (rc) return rc;
+        }
     }
     if (tile)
         for (int d = 0; d < 3; d++) tile[d] = e->tile[d];

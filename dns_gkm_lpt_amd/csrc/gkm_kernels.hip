@@ -18,6 +18,18 @@ __global__ __launch_bounds__(256, 2) void sweep_kernel(SweepArgs p)
     sweep_body<DIR, MIX, V, false, GEN, CMP>(p, blockIdx.x, gridDim.x, true);
 }
 
+// the entry a block belongs to: first[k] <= g < first[k + 1], 0 <= k < n
+__device__ __forceinline__ int entry_of(const int* __restrict__ first, int n, int g)
+{
+    int lo = 0, hi = n;  // first[lo] <= g < first[hi]
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (first[mid] <= g) lo = mid;
+        else hi = mid;
+    }
+    return lo;
+}
+
 // One launch for the sweeps of every member of an ensemble: member m owns the
 // blocks [first[m], first[m+1]) of the grid, in launch order.  Unlike the
 // single-grid sweep there is no XCD-grouped reorder: members' workgroups
@@ -29,15 +41,9 @@ template <int DIR, bool MIX, int V, bool GEN, int CMP>
 __global__ __launch_bounds__(256, 2) void ens_sweep_kernel(const SweepArgs* __restrict__ members,
                                                           const int* __restrict__ first, int nmem)
 {
-    const int g = blockIdx.x;
-    int lo = 0, hi = nmem;  // first[lo] <= g < first[hi]
-    while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (first[mid] <= g) lo = mid;
-        else hi = mid;
-    }
-    const SweepArgs p = members[lo];
-    sweep_body<DIR, MIX, V, false, GEN, CMP>(p, g - first[lo], first[lo + 1] - first[lo], false);
+    const int m = entry_of(first, nmem, blockIdx.x);
+    const SweepArgs p = members[m];
+    sweep_body<DIR, MIX, V, false, GEN, CMP>(p, blockIdx.x - first[m], first[m + 1] - first[m], false);
 }
 
 static int cdiv(int a, int b) { return (a + b - 1) / b; }
@@ -67,47 +73,44 @@ __global__ __launch_bounds__(256, 2) void faces_kernel(FaceArgs a)
     else sweep_body<2, MIX, 0, true, false, 0, true>(a.dir[2], b - a.first[2], a.first[3] - a.first[2], true, lds);
 }
 
-struct UpdateArgs {
-    const double* W;
-    double* Wout;
-    const double* F;  // 3 directions x 5 planes
-    const float* cmp_in;  // compensated update (SweepArgs): the carried errors
-    float* cmp_out;
-    long plane;
-    int nc;
-    double inv_dx, gam, cfl, dx;
-    double *partial, *dt, *vmax, *hist;  // partial = nullptr: no CFL
-    int *bad, *ticket;
-};
+// cell c of the next state, into t and memory
+template <bool CMP>
+__device__ __forceinline__ void update_cell(const UpdateArgs& a, long c, double t[5])
+{
+    const int nc = a.nc;
+    // plane < 2^31 (small_step_ok); a 64-bit division is some 100 instructions
+    const unsigned row = (unsigned)c / (unsigned)nc;
+    const int z = (int)((unsigned)c - row * nc), y = (int)(row / (unsigned)nc), x = (int)(row - (unsigned)y * nc);
+    const long cx = x ? c - nc : c + (long)(nc - 1) * nc;
+    const long cy = y ? c - (long)nc * nc : c + (long)(nc - 1) * nc * nc;
+    const long cz = z ? c - 1 : c + nc - 1;
+#pragma unroll
+    for (int q = 0; q < 5; q++) {
+        const double *Fx = a.F + q * a.plane, *Fy = Fx + 5 * a.plane, *Fz = Fy + 5 * a.plane;
+        const double dW = (Fx[c] - Fx[cx]) + (Fy[c] - Fy[cy]);
+        const double dF = Fz[c] - Fz[cz];
+        if constexpr (CMP) {  // TwoSum, as in sweep_body
+            const long co = q * carry_plane(nc) + carry_index(y, x, z, nc);
+            const double w = a.W[q * a.plane + c];
+            const double d = (double)a.cmp_in[co] - a.inv_dx * (dW + dF);
+            t[q] = w + d;
+            const double dv = t[q] - w;
+            a.cmp_out[co] = (float)((w - (t[q] - dv)) + (d - dv));
+        } else {
+            t[q] = a.W[q * a.plane + c] - a.inv_dx * (dW + dF);
+        }
+        a.Wout[q * a.plane + c] = t[q];
+    }
+}
+
 template <bool CMP>
 __global__ __launch_bounds__(256) void step_update_kernel(UpdateArgs a)
 {
-    const int nc = a.nc;
     double m = 0.0;
     bool bad = false;
     for (long c = (long)blockIdx.x * 256 + threadIdx.x; c < a.plane; c += (long)gridDim.x * 256) {
-        const int z = (int)(c % nc), x = (int)((c / nc) % nc), y = (int)(c / ((long)nc * nc));
-        const long cx = x ? c - nc : c + (long)(nc - 1) * nc;
-        const long cy = y ? c - (long)nc * nc : c + (long)(nc - 1) * nc * nc;
-        const long cz = z ? c - 1 : c + nc - 1;
         double t[5];
-#pragma unroll
-        for (int q = 0; q < 5; q++) {
-            const double *Fx = a.F + q * a.plane, *Fy = Fx + 5 * a.plane, *Fz = Fy + 5 * a.plane;
-            const double dW = (Fx[c] - Fx[cx]) + (Fy[c] - Fy[cy]);
-            const double dF = Fz[c] - Fz[cz];
-            if constexpr (CMP) {  // TwoSum, as in sweep_body
-                const long co = q * carry_plane(nc) + carry_index(y, x, z, nc);
-                const double w = a.W[q * a.plane + c];
-                const double d = (double)a.cmp_in[co] - a.inv_dx * (dW + dF);
-                t[q] = w + d;
-                const double dv = t[q] - w;
-                a.cmp_out[co] = (float)((w - (t[q] - dv)) + (d - dv));
-            } else {
-                t[q] = a.W[q * a.plane + c] - a.inv_dx * (dW + dF);
-            }
-            a.Wout[q * a.plane + c] = t[q];
-        }
+        update_cell<CMP>(a, c, t);
         if (a.partial) cfl_cell(t[0], t[1], t[2], t[3], t[4], a.gam, m, bad);
     }
     if (!a.partial) return;
@@ -128,6 +131,50 @@ __global__ __launch_bounds__(256) void step_update_kernel(UpdateArgs a)
     if (!last) return;
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     cfl_reduce(a.partial, gridDim.x, a.cfl, a.dx, a.dt, a.vmax, a.bad, a.hist);
+}
+
+// The same two launches for every member of an ensemble: entry d n + m of
+// members is member m's faces of direction d, with the blocks [first[k],
+// first[k + 1]).  Against the three ens_sweep launches every lead-in chunk and
+// two of the launches' ends are gone (8 x 32^3, 8 x 48^3 and 4 x 64^3 mixed with
+// 8192 tracers each, us a step: sweeps 1009 -> faces 745 + update 96, all 1264 ->
+// 1095).
+template <bool MIX>
+__global__ __launch_bounds__(256, 2) void ens_faces_kernel(const SweepArgs* __restrict__ members,
+                                                          const int* __restrict__ first, int nmem)
+{
+    __shared__ double lds[max3(sweep_lds_doubles<0, 0, MIX>(), sweep_lds_doubles<1, 0, MIX>(), sweep_lds_doubles<2, 0, MIX>())];
+    const int k = entry_of(first, 3 * nmem, blockIdx.x);
+    const SweepArgs p = members[k];
+    const int b = blockIdx.x - first[k], nblk = first[k + 1] - first[k];
+    if (k < nmem) sweep_body<0, MIX, 0, true, false, 0, true>(p, b, nblk, false, lds);
+    else if (k < 2 * nmem) sweep_body<1, MIX, 0, true, false, 0, true>(p, b, nblk, false, lds);
+    else sweep_body<2, MIX, 0, true, false, 0, true>(p, b, nblk, false, lds);
+}
+
+template <bool CMP>
+__global__ __launch_bounds__(256) void ens_update_kernel(const UpdateArgs* __restrict__ members,
+                                                        const int* __restrict__ first, int nmem)
+{
+    const int m = entry_of(first, nmem, blockIdx.x);
+    const UpdateArgs a = members[m];
+    const long c = (long)(blockIdx.x - first[m]) * 256 + threadIdx.x;
+    double t[5];
+    if (c < a.plane) update_cell<CMP>(a, c, t);
+}
+
+hipError_t launch_ens_small_step(const SweepArgs* faces, const int* ffirst, int nfblk, const UpdateArgs* upd,
+                                 const int* ufirst, int nublk, int nmem, bool mixed, bool compensated, hipStream_t s)
+{
+    if (nmem <= 0 || nfblk <= 0 || nublk <= 0 || (compensated && !mixed)) return hipErrorInvalidValue;
+    const dim3 fg((unsigned)nfblk), ug((unsigned)nublk), block(256);
+    if (mixed) hipLaunchKernelGGL(ens_faces_kernel<true>, fg, block, 0, s, faces, ffirst, nmem);
+    else hipLaunchKernelGGL(ens_faces_kernel<false>, fg, block, 0, s, faces, ffirst, nmem);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    if (compensated) hipLaunchKernelGGL(ens_update_kernel<true>, ug, block, 0, s, upd, ufirst, nmem);
+    else hipLaunchKernelGGL(ens_update_kernel<false>, ug, block, 0, s, upd, ufirst, nmem);
+    return hipGetLastError();
 }
 
 static const int* tile_shape(int dir, int tile, bool mixed) { return mixed ? kTiles[dir][tile] : kTilesPair[dir][tile]; }
@@ -158,8 +205,9 @@ static int equal_parts(int nc, int CN, int most)
 // launch ends a quarter of a workgroup's time after the slots run dry, so longer segments
 // pay on larger grids only (us per step at 1 / 2 / 4 / 8 chunks, FP64: 32^3 29 /
 // 32 / 35 / 51, 64^3 135 / 125 / 122 / 123, 128^3 898 / 805 / 773 / 765; mixed:
-// 32^3 31 / 34 / 49 / 82, 128^3 813 / 793 / 762 / 767).
-static int faces_seg_len(int dir, int nc, int slots, bool mixed)
+// 32^3 31 / 34 / 49 / 82, 128^3 813 / 793 / 762 / 767).  A member of an
+// ensemble answers for its share of the launch's end.
+static int faces_seg_len(int dir, int nc, int slots, double share, bool mixed)
 {
     const int* t = tile_shape(dir, 0, mixed);
     const long pencils = (long)cdiv(nc, t[1]) * cdiv(nc, t[2]);
@@ -170,7 +218,7 @@ static int faces_seg_len(int dir, int nc, int slots, bool mixed)
         const int seg = equal_parts(nc, t[0], k);
         if (seg > nc) break;
         const double chunks = seg / t[0] + start;
-        const double c = (double)(pencils * sweep_nseg(nc, seg)) / slots * chunks + 0.25 * chunks;
+        const double c = (double)(pencils * sweep_nseg(nc, seg)) / slots * chunks + 0.25 * share * chunks;
         if (cost < 0.0 || c < cost) {
             cost = c;
             best = seg;
@@ -179,27 +227,43 @@ static int faces_seg_len(int dir, int nc, int slots, bool mixed)
     return best;
 }
 
+SweepArgs faces_args(const SweepArgs& a, double* F, int dir, int slots, double share, bool mixed)
+{
+    SweepArgs f = a;
+    f.tile = 0;
+    f.mode = 0;
+    f.dW = F + (long)dir * 5 * a.plane;
+    f.seg = faces_seg_len(dir, a.nc, slots, share, mixed);
+    f.nseg = sweep_nseg(a.nc, f.seg);
+    return f;
+}
+
+int faces_blocks(int dir, const SweepArgs& f, bool mixed)
+{
+    const int* t = tile_shape(dir, 0, mixed);
+    return cdiv(f.nc, t[1]) * cdiv(f.nc, t[2]) * f.nseg;
+}
+
+UpdateArgs update_args(const SweepArgs& a, const double* F)
+{
+    return {a.W, a.Wout, F, a.cmp_in, a.cmp_out, a.plane, a.nc, a.inv_dx, 0.0, 0.0, a.dx, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
+}
+
 hipError_t launch_small_step(const SweepArgs& a, double* F, const StepCfl* cfl, int slots, bool mixed, hipStream_t s)
 {
     if (!small_step_ok(a.nc, mixed) || !F || (a.cmp_out != nullptr) != (a.cmp_in != nullptr) || (a.cmp_out && !mixed))
         return hipErrorInvalidValue;
     FaceArgs f{};
     for (int d = 0; d < 3; d++) {
-        f.dir[d] = a;
-        f.dir[d].tile = 0;
-        f.dir[d].mode = 0;
-        f.dir[d].dW = F + (long)d * 5 * a.plane;
-        const int* t = tile_shape(d, 0, mixed);
-        f.dir[d].seg = faces_seg_len(d, a.nc, slots, mixed);
-        f.dir[d].nseg = sweep_nseg(a.nc, f.dir[d].seg);
-        f.first[d + 1] = f.first[d] + cdiv(a.nc, t[1]) * cdiv(a.nc, t[2]) * f.dir[d].nseg;
+        f.dir[d] = faces_args(a, F, d, slots, 1.0, mixed);
+        f.first[d + 1] = f.first[d] + faces_blocks(d, f.dir[d], mixed);
     }
     const dim3 grid(f.first[3]), block(256);
     if (mixed) hipLaunchKernelGGL(faces_kernel<true>, grid, block, 0, s, f);
     else hipLaunchKernelGGL(faces_kernel<false>, grid, block, 0, s, f);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    UpdateArgs u{a.W, a.Wout, F, a.cmp_in, a.cmp_out, a.plane, a.nc, a.inv_dx, 0.0, 0.0, a.dx, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
+    UpdateArgs u = update_args(a, F);
     if (cfl) {
         u.gam = cfl->gam;
         u.cfl = cfl->cfl;

@@ -124,6 +124,31 @@ struct StepCfl {
     int *bad, *ticket;                   // ticket: 0 before the first launch, left 0
 };
 hipError_t launch_small_step(const SweepArgs& a, double* F, const StepCfl* cfl, int slots, bool mixed, hipStream_t s);
+
+// The update of the two-launch step.
+struct UpdateArgs {
+    const double* W;
+    double* Wout;
+    const double* F;  // 3 directions x 5 planes
+    const float* cmp_in;  // compensated update (SweepArgs): the carried errors
+    float* cmp_out;
+    long plane;
+    int nc;
+    double inv_dx, gam, cfl, dx;
+    double *partial, *dt, *vmax, *hist;  // partial = nullptr: no CFL
+    int *bad, *ticket;
+};
+// Its parts for a member of an ensemble: a is the member's sweep arguments, F its
+// face fluxes, share its part of the ensemble's cells.
+SweepArgs faces_args(const SweepArgs& a, double* F, int dir, int slots, double share, bool mixed);
+int faces_blocks(int dir, const SweepArgs& f, bool mixed);
+UpdateArgs update_args(const SweepArgs& a, const double* F);
+inline int update_blocks(const UpdateArgs& u) { return (int)((u.plane + 255) / 256); }
+// faces: 3 nmem entries (direction by direction) with blocks [ffirst[k], ffirst[k +
+// 1]) of nfblk; upd: nmem entries with [ufirst[m], ufirst[m + 1]) of nublk
+hipError_t launch_ens_small_step(const SweepArgs* faces, const int* ffirst, int nfblk, const UpdateArgs* upd,
+                                 const int* ufirst, int nublk, int nmem, bool mixed, bool compensated, hipStream_t s);
+
 // ensemble CFL: one dt per member (partial holds nmem * kEnsCflBlocks doubles)
 struct CflArgs {
     const double* W;
