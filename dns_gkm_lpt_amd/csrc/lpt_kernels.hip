@@ -164,31 +164,55 @@ hipError_t launch_prefilter_velocity(const double* W, long plane, double gam, co
 // weights are (1, 4, 1)/6 for the value and (1, -2, 1) delta^-2 for the second
 // derivative, so the Laplacian is a 27-point stencil on the coefficients.
 // The result lands at the knot positions of the coefficient box `lap`.
-__global__ void lap_knots_kernel(const double* __restrict__ c, Geom g, double* __restrict__ lap)
+// A thread walks kMarch knots of a column along the slowest axis and keeps the
+// two in-plane sums of three coefficient planes: 9 loads a knot where a knot by
+// itself takes 27, and no index divisions inside.  What is left is the box read
+// and written once (240^3: 177 -> 93 us,
+// 2.5 TB/s; 128^3: 28 -> 18).
+constexpr int kMarch = 16;
+__global__ __launch_bounds__(256) void lap_knots_kernel(const double* __restrict__ c, Geom g, double* __restrict__ lap)
 {
-    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long nt = g.nt, N = g.N;
-    if (t >= nt * nt * nt) return;
-    const int a = (int)(t / (nt * nt)), b = (int)((t / nt) % nt), k = (int)(t % nt);
+    const int nt = g.nt;
+    const unsigned col = blockIdx.x * 256u + threadIdx.x;
+    if (col >= (unsigned)nt * (unsigned)nt) return;
+    const long N = g.N;
+    const int b = (int)(col / (unsigned)nt), k = (int)(col - (unsigned)b * nt);
+    const int a0 = blockIdx.y * kMarch, a1 = a0 + kMarch < nt ? a0 + kMarch : nt;
     const double w[3] = {1.0 / 6.0, 4.0 / 6.0, 1.0 / 6.0}, d2[3] = {1.0, -2.0, 1.0};
-    double hyy = 0, hxx = 0, hzz = 0;
-    for (int i = 0; i < 3; i++)
+    const double scale = g.dinv * g.dinv;
+    const double* at = c + ((long)a0 * N + b) * N + k;
+    // plane sums: V weights (1, 4, 1) both ways, H second differences along x and z
+    auto plane = [&](double& V, double& H) {
+        V = H = 0.0;
+#pragma unroll
         for (int j = 0; j < 3; j++) {
-            const double* row = c + ((long)(a + i) * N + (b + j)) * N + k;
+            const double* row = at + j * N;
             const double rv = w[0] * row[0] + w[1] * row[1] + w[2] * row[2];
-            const double r2 = d2[0] * row[0] + d2[1] * row[1] + d2[2] * row[2];
-            hyy += d2[i] * w[j] * rv;
-            hxx += w[i] * d2[j] * rv;
-            hzz += w[i] * w[j] * r2;
+            V += w[j] * rv;
+            H += d2[j] * rv + w[j] * (d2[0] * row[0] + d2[1] * row[1] + d2[2] * row[2]);
         }
-    lap[((long)a * N + b) * N + k] = (hyy + hxx + hzz) * (g.dinv * g.dinv);
+        at += N * N;
+    };
+    double V0, V1, V2, H0, H1, H2;
+    plane(V0, H0);
+    plane(V1, H1);
+    double* out = lap + ((long)a0 * N + b) * N + k;
+#pragma unroll 2
+    for (int a = a0; a < a1; a++, out += N * N) {
+        plane(V2, H2);
+        *out = ((d2[0] * V0 + d2[1] * V1 + d2[2] * V2) + (w[0] * H0 + w[1] * H1 + w[2] * H2)) * scale;
+        V0 = V1;
+        V1 = V2;
+        H0 = H1;
+        H1 = H2;
+    }
 }
 
 hipError_t launch_lap_spline(const double* c, const Geom& g, const double* pivots, double* lap, hipStream_t s)
 {
     if (c == lap || g.nt != g.nc + 6 || g.N != g.nt + 2 || !z_chunks(g.nt)) return hipErrorInvalidValue;
-    const long n = (long)g.nt * g.nt * g.nt;
-    hipLaunchKernelGGL(lap_knots_kernel, dim3(blocks_for(n, 256)), dim3(256), 0, s, c, g, lap);
+    const dim3 grid(blocks_for((long)g.nt * g.nt, 256), blocks_for(g.nt, kMarch));
+    hipLaunchKernelGGL(lap_knots_kernel, grid, dim3(256), 0, s, c, g, lap);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     e = with_chunks(z_chunks(g.nt), [&](auto k) {
@@ -249,81 +273,90 @@ hipError_t launch_sample(long np, const double* pos, const double* const cu[3], 
 // Particle (ParticleTrack.h:21-22): DEN, U[3], P, gradD[3], gradU[3], gradV[3],
 // gradW[3], gradP[3], lapU, lapV, lapW, hessP[9], gradLapU[3], gradLapV[3],
 // gradLapW[3]; vectors over (y, x, z), hessP row-major over (y, x, z).
-__global__ __launch_bounds__(256) void props_kernel(long np, const double* __restrict__ pos, const int* __restrict__ tag,
-                                                    const double* const* __restrict__ cs, Geom g,
-                                                    double* __restrict__ out)
+// A quad of lanes per tracer and field (sample_quad's way of reading a stencil),
+// field after field: a thread per tracer left 1-4 waves per SIMD waiting on their
+// gathers one field after the other (10^5 tracers at
+// 240^3, where they touch most of the eight fields' 950 MB: 347 -> 215 us; 2^18 at
+// 128^3: 318 -> 172).
+__global__ __launch_bounds__(256) void props_kernel(long np, unsigned bpf, const double* __restrict__ pos,
+                                                    const int* __restrict__ tag, const double* const* __restrict__ cs,
+                                                    Geom g, double* __restrict__ out)
 {
-    const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const int f = (int)(blockIdx.x / bpf);
+    const long t = (long)(blockIdx.x - f * bpf) * blockDim.x + threadIdx.x;
+    const long p = t >> 2;
+    const int lane = (int)(t & 3);
     if (p >= np) return;
-    if (g.drop && isnan(pos[3 * p])) {  // dropped tracer: a row of NaN
-        for (int k = 0; k < kPropWidth; k++) out[(long)tag[p] * kPropWidth + k] = __builtin_nan("");
-        return;
-    }
-    const Loc Ly = locate(pos[3 * p + 0], g, true);
-    const Loc Lx = locate(pos[3 * p + 1], g, true);
-    const Loc Lz = locate(pos[3 * p + 2], g, true);
-    // second-derivative weights of the cubic B-spline
-    double hy[4], hx[4], hz[4];
-    {
-        const double d2 = g.dinv * g.dinv;
-        const Loc* L3[3] = {&Ly, &Lx, &Lz};
-        double* H3[3] = {hy, hx, hz};
-#pragma unroll
-        for (int a = 0; a < 3; a++) {
-            const double t = L3[a]->t;
-            H3[a][0] = (1 - t) * d2;
-            H3[a][1] = (3 * t - 2) * d2;
-            H3[a][2] = (1 - 3 * t) * d2;
-            H3[a][3] = t * d2;
-        }
-    }
-    const long N = g.N;
-    double* o = out + (long)tag[p] * kPropWidth;
     // output slots of value and gradient per field
-    const int vslot[8] = {0, 1, 2, 3, 4, 20, 21, 22};
-    const int gslot[8] = {5, 8, 11, 14, 17, 32, 35, 38};
-    for (int f = 0; f < 8; f++) {
-        double v = 0, gy = 0, gx = 0, gz = 0, hyy = 0, hyx = 0, hyz = 0, hxx = 0, hxz = 0, hzz = 0;
-        const double* cf = cs[f];
-        for (int a = 0; a < 4; a++)
-            for (int b = 0; b < 4; b++) {
-                const double* row = cf + ((Ly.i + a) * N + (Lx.i + b)) * N + Lz.i;
-                double rv = 0, rd = 0, rh = 0;
+    const int vslot = f < 5 ? f : f + 15, gslot = f < 5 ? 5 + 3 * f : 17 + 3 * f;
+    double* o = out + (long)tag[p] * kPropWidth;
+    double r[4], h[9];  // value and gradient (y, x, z), Hessian
+    if (g.drop && isnan(pos[3 * p])) {  // dropped tracer: a row of NaN
 #pragma unroll
-                for (int c = 0; c < 4; c++) {
-                    rv += Lz.w[c] * row[c];
-                    rd += Lz.d[c] * row[c];
-                    rh += hz[c] * row[c];
-                }
-                const double wab = Ly.w[a] * Lx.w[b];
-                v += wab * rv;
-                gz += wab * rd;
-                gy += Ly.d[a] * Lx.w[b] * rv;
-                gx += Ly.w[a] * Lx.d[b] * rv;
-                if (f == 4) {
-                    hyy += hy[a] * Lx.w[b] * rv;
-                    hxx += Ly.w[a] * hx[b] * rv;
-                    hzz += wab * rh;
-                    hyx += Ly.d[a] * Lx.d[b] * rv;
-                    hyz += Ly.d[a] * Lx.w[b] * rd;
-                    hxz += Ly.w[a] * Lx.d[b] * rd;
-                }
-            }
-        o[vslot[f]] = v;
-        o[gslot[f] + 0] = gy;
-        o[gslot[f] + 1] = gx;
-        o[gslot[f] + 2] = gz;
+        for (int k = 0; k < 4; k++) r[k] = __builtin_nan("");
+#pragma unroll
+        for (int k = 0; k < 9; k++) h[k] = __builtin_nan("");
+    } else {
+        const Loc Ly = locate(pos[3 * p + 0], g, true);
+        const Loc Lx = locate(pos[3 * p + 1], g, true);
+        const Loc Lz = locate(pos[3 * p + 2], g, true);
+        const double wz = pick4(Lz.w, lane), dz = pick4(Lz.d, lane);
+        const long N = g.N;
+        const double* cf = cs[f] + ((long)Ly.i * N + Lx.i) * N + Lz.i + lane;
+        // second-derivative weights of the cubic B-spline
+        auto second = [&](double t, double q[4]) {
+            const double d2 = g.dinv * g.dinv;
+            q[0] = (1 - t) * d2;
+            q[1] = (3 * t - 2) * d2;
+            q[2] = (1 - 3 * t) * d2;
+            q[3] = t * d2;
+        };
+        // this lane's column of the sums: value, d/dy, d/dx and, for the pressure, the second ones
+        double P = 0, Py = 0, Px = 0, Pyy = 0, Pxx = 0, Pyx = 0;
+        double hy[4], hx[4];
         if (f == 4) {
-            o[23] = hyy;
-            o[24] = hyx;
-            o[25] = hyz;
-            o[26] = hyx;
-            o[27] = hxx;
-            o[28] = hxz;
-            o[29] = hyz;
-            o[30] = hxz;
-            o[31] = hzz;
+            second(Ly.t, hy);
+            second(Lx.t, hx);
         }
+#pragma unroll
+        for (int a = 0; a < 4; a++) {
+            double s = 0, sx = 0, sxx = 0;
+#pragma unroll
+            for (int b = 0; b < 4; b++) {
+                const double c = cf[((long)a * N + b) * N];
+                s += Lx.w[b] * c;
+                sx += Lx.d[b] * c;
+                if (f == 4) sxx += hx[b] * c;
+            }
+            P += Ly.w[a] * s;
+            Py += Ly.d[a] * s;
+            Px += Ly.w[a] * sx;
+            if (f == 4) {
+                Pyy += hy[a] * s;
+                Pxx += Ly.w[a] * sxx;
+                Pyx += Ly.d[a] * sx;
+            }
+        }
+        r[0] = quad_sum(wz * P);
+        r[1] = quad_sum(wz * Py);
+        r[2] = quad_sum(wz * Px);
+        r[3] = quad_sum(dz * P);
+        if (f == 4) {
+            double hz[4];
+            second(Lz.t, hz);
+            h[0] = quad_sum(wz * Pyy);
+            h[1] = h[3] = quad_sum(wz * Pyx);
+            h[2] = h[6] = quad_sum(dz * Py);
+            h[4] = quad_sum(wz * Pxx);
+            h[5] = h[7] = quad_sum(dz * Px);
+            h[8] = quad_sum(pick4(hz, lane) * P);
+        }
+    }
+    o[lane == 0 ? vslot : gslot + lane - 1] = pick4(r, lane);
+    if (f == 4) {
+        o[23 + lane] = pick4(h, lane);
+        o[27 + lane] = pick4(h + 4, lane);
+        if (lane == 0) o[31] = h[8];
     }
 }
 
@@ -331,7 +364,8 @@ hipError_t launch_props(long np, const double* pos, const int* tag, const double
                         double* out, hipStream_t s)
 {
     if (np <= 0) return hipSuccess;
-    hipLaunchKernelGGL(props_kernel, dim3(blocks_for(np, 256)), dim3(256), 0, s, np, pos, tag, cs_dev, g, out);
+    const unsigned bpf = blocks_for(4 * np, 256);
+    hipLaunchKernelGGL(props_kernel, dim3(8 * bpf), dim3(256), 0, s, np, bpf, pos, tag, cs_dev, g, out);
     return hipGetLastError();
 }
 
@@ -475,41 +509,79 @@ __global__ __launch_bounds__(256) void stats_kernel(const double* __restrict__ W
     const double w0 = 1.0 / 6.0, w1 = 4.0 / 6.0;
     const double d = 0.5 * g.dinv;
     const double* cs[3] = {cu, cv, cw};
-    for (long c = (long)blockIdx.x * blockDim.x + threadIdx.x; c < plane; c += (long)gridDim.x * blockDim.x) {
-        const int k = (int)(c % nc), i = (int)((c / nc) % nc), j = (int)(c / ((long)nc * nc));
-        const double den = W[c], ir = 1.0 / den;
-        const double uu = W[plane + c] * ir, vv = W[2 * plane + c] * ir, ww = W[3 * plane + c] * ir;
-        const double Vsqr = uu * uu + vv * vv + ww * ww;
-        const double P = (den * (sp.gam - 1)) * (W[4 * plane + c] * ir - 0.5 * Vsqr);
-        const double T = P / (sp.R * den);
+    // A block takes 256 columns along y, kMarch cells of them at a time, and a
+    // thread keeps three planes' in-plane sums of each field: 27 coefficient loads
+    // a cell where a cell by itself takes 81.  With two or three waves per SIMD
+    // the time was the loads' latency, once for the coefficients and once for the
+    // state (240^3: 548 us, marching alone 562); the next cell's loads before this
+    // one's arithmetic: 304 us, 128^3 81 -> 47.
+    const unsigned cols = (unsigned)nc * (unsigned)nc, cblk = (cols + 255) / 256;
+    const unsigned items = cblk * (unsigned)((nc + kMarch - 1) / kMarch);
+    for (unsigned it = blockIdx.x; it < items; it += gridDim.x) {
+    const unsigned sg = it / cblk, col = (it - sg * cblk) * 256 + threadIdx.x;
+    if (col >= cols) continue;
+    const int i = (int)(col / (unsigned)nc), k = (int)(col - (unsigned)i * nc);
+    const int j0 = (int)sg * kMarch, j1 = j0 + kMarch < nc ? j0 + kMarch : nc;
+    // knot (j+3, i+3, k+3): coefficient block starts at (j+3, i+3, k+3) with t = 0
+    long at = ((long)(j0 + 3) * N + (i + 3)) * N + (k + 3);
+    struct Plane {
+        double v, gx, gz;
+    } pl[3][3];  // [plane][field]
+    double raw[3][9], w[5];
+    auto load = [&] {
+#pragma unroll
+        for (int f = 0; f < 3; f++)
+#pragma unroll
+            for (int b = 0; b < 9; b++) raw[f][b] = cs[f][at + (b / 3) * N + b % 3];
+        at += N * N;
+    };
+    auto sums = [&](Plane q[3]) {
+#pragma unroll
+        for (int f = 0; f < 3; f++) {
+            double rv[3], rd[3];
+#pragma unroll
+            for (int b = 0; b < 3; b++) {
+                rv[b] = w0 * (raw[f][3 * b] + raw[f][3 * b + 2]) + w1 * raw[f][3 * b + 1];
+                rd[b] = d * (raw[f][3 * b + 2] - raw[f][3 * b]);
+            }
+            q[f].v = w0 * (rv[0] + rv[2]) + w1 * rv[1];
+            q[f].gx = d * (rv[2] - rv[0]);
+            q[f].gz = w0 * (rd[0] + rd[2]) + w1 * rd[1];
+        }
+    };
+    auto cell = [&](int j) {
+#pragma unroll
+        for (int q = 0; q < 5; q++) w[q] = W[q * plane + (long)j * cols + col];
+    };
+    load();
+    sums(pl[0]);
+    load();
+    sums(pl[1]);
+    load();
+    cell(j0);
+    for (int j = j0; j < j1; j++) {
+        sums(pl[2]);
+        const double den = w[0], m1 = w[1], m2 = w[2], m3 = w[3], en = w[4];
+        // the next cell's loads pass behind this one's arithmetic (one plane past
+        // the last cell's is still in the box)
+        load();
+        cell(j + 1 < j1 ? j + 1 : j);
+        __builtin_amdgcn_sched_barrier(0);
         double val[3], gr[3][3];  // gr[f] = d/dy, d/dx, d/dz
 #pragma unroll
         for (int f = 0; f < 3; f++) {
-            // knot (j+3, i+3, k+3): coefficient block starts at (j+3, i+3, k+3) with t = 0
-            const double* base = cs[f] + ((long)(j + 3) * N + (i + 3)) * N + (k + 3);
-            double v = 0, gy = 0, gx = 0, gz = 0;
-#pragma unroll
-            for (int a = 0; a < 3; a++) {
-                const double wa = a == 1 ? w1 : w0;
-                const double da = a == 0 ? -d : (a == 2 ? d : 0.0);
-#pragma unroll
-                for (int b = 0; b < 3; b++) {
-                    const double wb = b == 1 ? w1 : w0;
-                    const double db = b == 0 ? -d : (b == 2 ? d : 0.0);
-                    const double* row = base + (a * N + b) * N;
-                    const double rv = w0 * row[0] + w1 * row[1] + w0 * row[2];
-                    const double rd = d * (row[2] - row[0]);
-                    v += wa * wb * rv;
-                    gz += wa * wb * rd;
-                    gy += da * wb * rv;
-                    gx += wa * db * rv;
-                }
-            }
-            val[f] = v;
-            gr[f][0] = gy;
-            gr[f][1] = gx;
-            gr[f][2] = gz;
+            val[f] = w0 * (pl[0][f].v + pl[2][f].v) + w1 * pl[1][f].v;
+            gr[f][0] = d * (pl[2][f].v - pl[0][f].v);
+            gr[f][1] = w0 * (pl[0][f].gx + pl[2][f].gx) + w1 * pl[1][f].gx;
+            gr[f][2] = w0 * (pl[0][f].gz + pl[2][f].gz) + w1 * pl[1][f].gz;
+            pl[0][f] = pl[1][f];
+            pl[1][f] = pl[2][f];
         }
+        const double ir = 1.0 / den;
+        const double uu = m1 * ir, vv = m2 * ir, ww = m3 * ir;
+        const double Vsqr = uu * uu + vv * vv + ww * ww;
+        const double P = (den * (sp.gam - 1)) * (en * ir - 0.5 * Vsqr);
+        const double T = P / (sp.R * den);
         const double dudx = gr[0][1], dudy = gr[0][0], dudz = gr[0][2];
         const double dvdx = gr[1][1], dvdy = gr[1][0], dvdz = gr[1][2];
         const double dwdx = gr[2][1], dwdy = gr[2][0], dwdz = gr[2][2];
@@ -533,6 +605,7 @@ __global__ __launch_bounds__(256) void stats_kernel(const double* __restrict__ W
         acc[13] += P;
         acc[14] += T;
         acc[15] += ir;
+    }
     }
     block_sum<16>(acc, red + 32 * blockIdx.x);
 }
