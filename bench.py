@@ -63,12 +63,15 @@ MEASURED_TRAFFIC_GIB = {
     ("mixed", 1, 2, 512): (17.22, 5.00),
     ("mixed", 2, 0, 512): (23.18, 7.50),
     ("mixed", 2, 2, 512): (53.09, 7.85),
-    ("fp64", 0, 0, 512): (52.88, 21.27),
-    ("fp64", 0, 2, 512): (65.76, 17.07),
-    ("fp64", 1, 0, 512): (56.53, 16.70),
-    ("fp64", 1, 2, 512): (65.35, 18.61),
-    ("fp64", 2, 0, 512): (59.67, 19.91),
-    ("fp64", 2, 2, 512): (85.34, 19.45),
+    ("fp64", 0, 0, 512): (7.04, 5.39),
+    ("fp64", 0, 1, 512): (6.68, 5.00),
+    ("fp64", 0, 2, 512): (7.60, 5.00),
+    ("fp64", 1, 0, 512): (12.30, 5.54),
+    ("fp64", 1, 1, 512): (11.34, 5.00),
+    ("fp64", 1, 2, 512): (12.60, 5.00),
+    ("fp64", 2, 0, 512): (15.02, 6.43),
+    ("fp64", 2, 1, 512): (39.67, 6.24),
+    ("fp64", 2, 2, 512): (44.07, 5.35),
 }
 # rocprofv3 VALUBusy (% of time the VALU issues) of each sweep launch, keyed
 # like MEASURED_TRAFFIC_GIB; commands and table in profiles/sweep_valu_512.md.
@@ -79,12 +82,15 @@ MEASURED_VALU_BUSY = {
     ("mixed", 1, 2, 512): 68.1,
     ("mixed", 2, 0, 512): 71.7,
     ("mixed", 2, 2, 512): 65.7,
-    ("fp64", 0, 0, 512): 57.6,
-    ("fp64", 0, 2, 512): 52.3,
-    ("fp64", 1, 0, 512): 52.4,
-    ("fp64", 1, 2, 512): 47.7,
-    ("fp64", 2, 0, 512): 54.7,
-    ("fp64", 2, 2, 512): 51.4,
+    ("fp64", 0, 0, 512): 78.7,
+    ("fp64", 0, 1, 512): 78.7,
+    ("fp64", 0, 2, 512): 86.7,
+    ("fp64", 1, 0, 512): 78.1,
+    ("fp64", 1, 1, 512): 74.0,
+    ("fp64", 1, 2, 512): 80.8,
+    ("fp64", 2, 0, 512): 82.7,
+    ("fp64", 2, 1, 512): 78.7,
+    ("fp64", 2, 2, 512): 83.1,
 }
 KERNEL_NAMES = {0: "sweep_kernel<0> (x)", 1: "sweep_kernel<1> (y)", 2: "sweep_kernel<2> (z, with update)",
                 3: "cfl reduction", 4: "spline prefilter (u, v, w)", 5: "particle sample + Heun",

@@ -1681,8 +1681,10 @@ int gkm_ensemble_autotune(gkm_ensemble* e, int reps, int tile[3], double ms[9])
         if (rc) return rc;
         sweeps += best_ms;
     }
-    if (e->mixed && !e->small) {
-        // the two-launch step goes with the first variants: keep them where it is faster
+    if (e->mixed && !e->small && !e->persistent) {
+        // the two-launch step goes with the first variants: keep them where it is
+        // faster (the persistent step sweeps: 64 members, 6.54 ms with them, 6.2 with
+        // the fastest)
         const int t[3] = {e->tile[0], e->tile[1], e->tile[2]}, zero[3] = {0, 0, 0};
         bool ok = true;
         for (gkm_ctx* c : e->mem) ok = ok && c->faces;

@@ -206,7 +206,8 @@ gkm_ctx *gkm_ensemble_member(gkm_ensemble *e, int m);
 /* one tile variant per direction for all members; gkm_ensemble_autotune times
  * every variant of every direction on the members' current states (which it
  * does not change) and keeps the fastest, or variant 0 throughout where the
- * two-launch step is faster, as gkm_autotune; so does ms (may be NULL) */
+ * two-launch step is faster, as gkm_autotune (not in persistent mode, which
+ * sweeps); ms (may be NULL) as gkm_autotune */
 int gkm_ensemble_set_tiles(gkm_ensemble *e, const int tile[3]);
 int gkm_ensemble_autotune(gkm_ensemble *e, int reps, int tile[3], double ms[9]);
 /* nsteps steps of every member, each with dt from its own CFL condition */
