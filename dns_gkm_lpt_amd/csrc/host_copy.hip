@@ -34,6 +34,18 @@ int usable_cpus()
     return 1;
 }
 
+// memory the runtime knows (pinned, managed, on a device): the device reaches it
+// itself, and host code may not
+bool known_to_runtime(const void* p)
+{
+    hipPointerAttribute_t a{};
+    if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return a.type != hipMemoryTypeUnregistered;
+}
+
 struct Chunk {
     char *host, *dev;
     size_t bytes;
@@ -89,6 +101,8 @@ hipError_t HostPipe::run(const CopySeg* seg, int n, hipStream_t s, bool to_host)
     size_t total = 0;
     for (int i = 0; i < n; i++) total += seg[i].bytes;
     if (total < kPipeMin) return plain(seg, n, s, to_host);
+    for (int i = 0; i < n; i++)
+        if (known_to_runtime(seg[i].host)) return plain(seg, n, s, to_host);
     const int nthr = (int)std::min<size_t>(std::min(usable_cpus(), 8), total / (size_t(2) << 20) + 1);
     if (nthr < 2 || !ready(total)) return plain(seg, n, s, to_host);
 

@@ -1,6 +1,7 @@
 """Copies of whole arrays through the pinned ring (csrc/host_copy.hip): sizes
 below and just above the 32 MB at which it starts, tails that fill no slice, several
 segments, several contexts at once.  Bytes have to arrive as they are."""
+import ctypes
 import threading
 
 import numpy as np
@@ -61,3 +62,18 @@ def test_tracer_arrays_in_parts():
         props = c.lpt_properties()
     for a, b in ((U, props[:, 1:4]), (gU, props[:, 8:11]), (gV, props[:, 11:14]), (gW, props[:, 14:17])):
         assert np.max(np.abs(a - b)) <= 1e-12 * np.max(np.abs(b))
+
+
+@pytest.mark.parametrize("nc", [64, 101])
+def test_pinned_memory_goes_straight(nc):
+    """Memory the runtime knows takes the plain copy on both sides of the 32 MB."""
+    W = random_state(nc, nc)
+    with gl.Context(nc, PAR) as c:
+        hip = ctypes.CDLL("libamdhip64.so.7")  # the runtime the library loaded
+        p = ctypes.c_void_p()
+        assert hip.hipHostMalloc(ctypes.byref(p), ctypes.c_size_t(W.nbytes), 0) == 0
+        pinned = np.ctypeslib.as_array(ctypes.cast(p, ctypes.POINTER(ctypes.c_double)), W.shape)
+        pinned[:] = W
+        c.upload(pinned)
+        np.testing.assert_array_equal(c.download(), W)
+        assert hip.hipHostFree(p) == 0
