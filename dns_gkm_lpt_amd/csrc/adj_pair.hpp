@@ -124,7 +124,7 @@ __host__ __device__ __forceinline__ double face_flux_vjp_pair(const AdjPark& pk,
     {
         double W[5];
         unpark(AdjPark::kS, W);
-        maxw_init(S, W, g);
+        pair_maxw(S, W, g);
     }
     const double pa = 2.0 * S.den * S.i2l, pb = sw(pa);  // rho / lambda of the two sides
     const double taue = tau0 + dt * g_div(::fabs(pa - pb), ::fabs(pa + pb));
@@ -136,7 +136,7 @@ __host__ __device__ __forceinline__ double face_flux_vjp_pair(const AdjPark& pk,
         f_sqrt_inv(S.lam, s, is);
         const double z = s * S.u, e = f_exp(-z * z);
         const double h0 = half_erfc(-z, e);
-        half_tab<4>(S.u, S.i2l, h0, S.u * h0 + 0.5 * isqpi * e * is, h);
+        half_tab<4>(S.u, S.i2l, h0, fma(0.5 * isqpi, e * is, S.u * h0), h);
     };
     half_start();
     // the half Maxwellian's <psi> (equilibrium) and <u psi> (p3 flux)
@@ -160,7 +160,7 @@ __host__ __device__ __forceinline__ double face_flux_vjp_pair(const AdjPark& pk,
     }
     pk.fence();
     Maxw<double> E;
-    maxw_init(E, We, g);
+    pair_maxw(E, We, g);
     const TState<double> sE{E.u, E.i2l, 2.0 * E.lam};
     const double cBE = tc.gm2 * E.den, cFE = tc.p2 * E.den;
     double Be[5] = {0, 0, 0, 0, 0}, Fs[5] = {0, 0, 0, 0, 0}, by[5] = {0, 0, 0, 0, 0};
@@ -183,7 +183,7 @@ __host__ __device__ __forceinline__ double face_flux_vjp_pair(const AdjPark& pk,
     double se, ise;
     f_sqrt_inv(E.lam, se, ise);
     const double ze = se * E.u, ee = f_exp(-ze * ze);
-    const double hp0 = half_erfc(-ze, ee), ge = 0.5 * isqpi * ee * ise;
+    const double hp0 = half_erfc(-ze, ee), ge = 0.5 * isqpi * (ee * ise);
     const double cn = 2.0 * g_rcp(E.den * dx);
     auto normal_fwd = [&](double hh[7], double dn[5], double m[5], double a[5]) {
         half_tab<7>(sE.u, sE.th, hp0, E.u * hp0 + ge, hh);
@@ -330,7 +330,7 @@ __host__ __device__ __forceinline__ double face_flux_vjp_pair(const AdjPark& pk,
         {
             double W[5];
             unpark(AdjPark::kS, W);
-            maxw_init(S, W, g);
+            pair_maxw(S, W, g);
             half_start();
             tc = time_coefs<double>(pk(AdjPark::kTc + 2), dt);
             unpark(AdjPark::kF, Fsb);

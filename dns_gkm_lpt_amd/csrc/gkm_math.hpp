@@ -141,35 +141,41 @@ __host__ __device__ __forceinline__ double g_div<double>(double a, double b)
 // keeps sqrt() and exp(): its FP32 terms turn a last-bit change of an FP64 input
 // into an FP32 rounding, and its results stay what they were.
 //
-// f_sqrt_inv: square root and its inverse together (the flux needs both): the
-// hardware's reciprocal root y, s = x y and h = y/2 refined by one coupled Newton
-// step (both errors squared), s by its residual x - s^2, 1/s by the residual of
-// s (1/s) = 1: 11 VALU instructions (8 for the root alone, 22 for sqrt() with its
-// scaling and special cases) within 1 ulp for normal x > 0; zero, negative,
-// infinite and NaN x give NaN (a state's lambda and temperature are positive
-// and finite, as for g_rcp).
+// f_sqrt_inv: square root and its inverse together (the flux needs both) by
+// Goldschmidt's coupled iteration: the hardware's reciprocal root y, s = x y and
+// h = y/2 refined by one step (both errors squared), s by its residual
+// d = x - s^2, and 1/sqrt(x) = 1/s - d/(2 s^3) by the residual of s (1/s) = 1
+// and by what s leaves of x: 14 VALU instructions (22 for sqrt() alone with its
+// scaling and special cases).  Both are correctly rounded or next to it: largest
+// relative error 1.11e-16 of 4e6 arguments.  (1/s of the rounded s: 1.66e-16,
+// which was the largest single error of the flux's half-space moments.)  Normal
+// x > 0; zero, negative, infinite and NaN x give NaN (a state's lambda and
+// temperature are positive and finite, as for g_rcp).
 // f_exp: exp of the flux's arguments -z^2 and -dt/tau.  x = n ln 2 + r,
 // |r| <= ln 2 / 2 (ln 2 in two parts, n times the first exact), e^r =
 // 1 + r + r^2 q(r) with q of degree 9 interpolating (e^r - 1 - r)/r^2 on
 // Chebyshev points (dns_gkm_lpt_amd/erfcx_fit.py prints the coefficients;
-// 1.7e-17 relative), scaled by 2^n: 19 VALU instructions against 42, 1.4e-16
-// relative.  Arguments below -1000 give 0 as e^-1000 does.
+// 1.7e-17 relative), 1 + r kept in two parts, scaled by 2^n: 22 VALU
+// instructions against exp()'s 42, largest relative error on [-700, 0] 1.30e-16
+// against 1.35e-16 (1.65e-16 with r + r^2 q rounded before the 1 is added).
+// Arguments below -1000 give 0 as e^-1000 does; so does NaN, which the flux has
+// in its other factors then.
 __host__ __device__ __forceinline__ void f_sqrt_inv(double x, double& s, double& is)
 {
 #if defined(__HIP_DEVICE_COMPILE__)
     const double y = __builtin_amdgcn_rsq(x);
+#else
+    // as good a guess as the hardware's, so that host checks run the same steps
+    const double y = (double)(1.0f / ::sqrtf((float)x));
+#endif
     s = x * y;
     double h = 0.5 * y;
     const double e = fma(-h, s, 0.5);
     s = fma(s, e, s);
     h = fma(h, e, h);
     s = fma(fma(-s, s, x), h, s);
-    h += h;
-    is = fma(fma(-s, h, 1.0), h, h);
-#else
-    s = sqrt(x);
-    is = 1.0 / s;
-#endif
+    const double d = fma(-s, s, x), h2 = h + h;
+    is = fma(fma(-d, h * h2, fma(-s, h2, 1.0)), h2, h2);
 }
 __host__ __device__ __forceinline__ double f_exp(double x)
 {
@@ -187,7 +193,8 @@ __host__ __device__ __forceinline__ double f_exp(double x)
     q = fma(q, r, 0.04166666666662413);
     q = fma(q, r, 0.16666666666666669);
     q = fma(q, r, 0.5000000000000001);
-    return ldexp(fma(q * r, r, r) + 1.0, (int)n);
+    const double h = 1.0 + r;
+    return ldexp(h + fma(q * r, r, (1.0 - h) + r), (int)n);
 }
 
 // 0.5 erfc(x) given E = exp(-x^2), which the half-space moments of a

@@ -14,13 +14,12 @@
 //  * Vectors that both sides add to cross over by DPP (no LDS): the mirrored
 //    partner's moment-like vector m is (m0, -m1, m3, m2, m4) here, its flux the
 //    negative of that.  21 values cross per face.
-//  * Terms of the equilibrium state that belong to neither side enter with half
-//    their weight in each lane.
+//  * The time slope's p1 term, which belongs to neither side, enters with half
+//    its weight in each lane; p0 <u psi>_e is added after the exchange.
 //  * gm1 den_e <psi>_e + gm3 We (GKMflux.cpp:185) is zero by the definition of
 //    We (gm3 = -gm1): left out.
 //
-//
-// 1100 VALU instructions per lane against 2030 for a face in one lane, and
+// 1075 VALU instructions per lane against 2030 for a face in one lane, and
 // nothing spilled (215-235 VGPRs in the sweeps).  With the difference form of
 // WENO (gkm_math.hpp) and the ring of cells (gkm_sweep.hpp), 256^3 x / y / z
 // sweep: 2.63 / 2.98 / 3.18 -> 1.88 / 1.91 / 2.01 ms.  Built for three waves per
@@ -56,6 +55,21 @@ __host__ __device__ __forceinline__ void pair_add(double m[5], const double p[5]
     m[4] += sw(p[4]);
 }
 
+// maxw_init for the two-lane forms: 1/(2 lambda) = p/rho from the specific energy
+// alone, without the density's way in and out again (two roundings less in the
+// pressure, which the half-space moments' difference amplifies)
+template <typename G>
+__host__ __device__ __forceinline__ void pair_maxw(Maxw<double>& s, const double W[5], const G& g)
+{
+    s.den = W[0];
+    const double ir = g_rcp(W[0]);
+    s.u = W[1] * ir;
+    s.v = W[2] * ir;
+    s.w = W[3] * ir;
+    s.i2l = gas_gam1(g) * fma(W[4], ir, -0.5 * (s.u * s.u + s.v * s.v + s.w * s.w));
+    s.lam = 0.5 * g_rcp(s.i2l);
+}
+
 // Inputs of one side through an accessor (the lane's frame: slot 1 the normal
 // momentum towards the lane's u > 0, slots 2 and 3 its first and second
 // tangential momentum):
@@ -78,7 +92,7 @@ __host__ __device__ __forceinline__ void gks_flux_pair(const IN& in, double tau,
         T W[5];
 #pragma unroll
         for (int q = 0; q < 5; q++) W[q] = in.S(q);
-        maxw_init(S, W, g);
+        pair_maxw(S, W, g);
     }
     {   // pressure-jump term of the collision time (GKMflux.cpp:156-157)
         const T pa = T(2) * S.den * S.i2l, pb = sw(pa);  // rho / lambda of the two sides
@@ -91,7 +105,7 @@ __host__ __device__ __forceinline__ void gks_flux_pair(const IN& in, double tau,
         f_sqrt_inv(S.lam, s, is);
         const T z = s * S.u, e = f_exp(-z * z);
         h0 = half_erfc(-z, e);
-        h1 = S.u * h0 + T(0.5) * isqpi * e * is;
+        h1 = fma(T(0.5) * isqpi, e * is, S.u * h0);
     }
     T We[5];
     {
@@ -103,7 +117,7 @@ __host__ __device__ __forceinline__ void gks_flux_pair(const IN& in, double tau,
         pair_add(We, m, sw);
     }
     Maxw<T> E;
-    maxw_init(E, We, g);
+    pair_maxw(E, We, g);
     // time-integration coefficients (GKMflux.cpp:162-167, 197-204)
     const T ex = f_exp(-g_div(dt, tau));
     const T om = T(1) - ex;
@@ -214,13 +228,6 @@ __host__ __device__ __forceinline__ void gks_flux_pair(const IN& in, double tau,
 #pragma unroll
         for (int q = 0; q < 5; q++) Fs[q] += m[q];
     }
-    {   // p0 <u psi>_e (GKMflux.cpp:225), half in each lane
-        const T f2 = E.u * E.u + E.i2l, f3 = E.u * f2 + T(2) * E.i2l * E.u;
-        const T c = T(0.5) * p0 * E.den;
-        Fs[0] += c * E.u;
-        Fs[1] += c * f2;
-        Fs[4] += c * (T(0.5) * (f3 + kp2 * E.i2l * E.u));
-    }
     {   // equilibrium state, normal slope of this side (GKMflux.cpp:115-116, 124-125, 170-171, 210-211)
         T s, is;
         f_sqrt_inv(E.lam, s, is);
@@ -228,7 +235,7 @@ __host__ __device__ __forceinline__ void gks_flux_pair(const IN& in, double tau,
         T hp[7];
         {
             const T a0 = half_erfc(-z, e);
-            half_tab<7>(se.u, se.th, a0, E.u * a0 + T(0.5) * isqpi * e * is, hp);
+            half_tab<7>(se.u, se.th, a0, fma(T(0.5) * isqpi, e * is, E.u * a0), hp);
         }
         const T c = T(2) * g_rcp(E.den * dx);
         T a[5], t[5];
@@ -282,6 +289,13 @@ __host__ __device__ __forceinline__ void gks_flux_pair(const IN& in, double tau,
     F[2] -= sw(Fs[3]);
     F[3] -= sw(Fs[2]);
     F[4] -= sw(Fs[4]);
+    {   // p0 <u psi>_e (GKMflux.cpp:225), the largest term: last, so that the others' sums round at their own size
+        const T f2 = E.u * E.u + E.i2l, f3 = E.u * f2 + T(2) * E.i2l * E.u;
+        const T c = p0 * E.den;
+        F[0] += c * E.u;
+        F[1] += c * f2;
+        F[4] += c * (T(0.5) * (f3 + kp2 * E.i2l * E.u));
+    }
     tshift(F, E.v, E.w);
 }
 
