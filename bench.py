@@ -310,7 +310,7 @@ def run_ensemble(gl, steps, warmup):
         for m, c in enumerate(cases):
             e.members[m].upload(c[2])
             e.members[m].lpt_upload(icm.uniform_particles(ntr, seed=c[3]))
-        tiles, _ = e.autotune(reps=2)
+        tiles, tms = e.autotune(reps=2)
         e.run(warmup, graph=True)
         for mode, graph, persistent in (("graph", True, False), ("eager", False, False),
                                         ("persistent", True, True)):
@@ -328,6 +328,7 @@ def run_ensemble(gl, steps, warmup):
                  "spline z pass", "spline x pass", "spline y pass", "Heun"]
         out["persistent_phase_ms"] = dict(zip(names, (round(float(v), 4) for v in e.persistent_profile())))
         out["sweep_tiles"] = list(tiles)
+        out["persistent_sweep_tiles"] = [min((v for v in range(3) if r[v] > 0), key=lambda v: r[v]) for r in tms]
         out["steps"] = steps
     out["value"] = out["member_cell_updates_per_s_graph"]
     out["unit"] = "member cell-updates/s"

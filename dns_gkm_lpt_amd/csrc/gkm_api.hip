@@ -1123,7 +1123,9 @@ struct gkm_ensemble {
     std::vector<gkm_ctx*> mem;
     hipStream_t stream = nullptr;
     hipEvent_t ev[2] = {nullptr, nullptr};
-    int tile[3] = {0, 0, 0};
+    int tile[3] = {0, 0, 0};               // what the tables were built for
+    int step_tile[3] = {0, 0, 0};          // variants for launches per phase, and
+    int persist_tile[3] = {0, 0, 0};       // for the persistent step, which always sweeps
     gkm::SweepArgs* dargs = nullptr;  // [parity][direction][member]
     int* dfirst = nullptr;            // [direction][member + 1] first block of each member
     // the two-launch step (gkm::launch_ens_small_step), where every member has one
@@ -1521,6 +1523,14 @@ int ens_particles_prepare(gkm_ensemble* e, int p)
     return GKM_OK;
 }
 
+// the variants of the mode the ensemble is in
+int ens_choose(gkm_ensemble* e, const int step[3], const int persist[3])
+{
+    std::copy(step, step + 3, e->step_tile);
+    std::copy(persist, persist + 3, e->persist_tile);
+    return ens_build(e, e->persistent ? e->persist_tile : e->step_tile);
+}
+
 int ens_parity(gkm_ensemble* e, int* p)
 {
     for (int m = 0; m < e->n; m++) {
@@ -1581,7 +1591,7 @@ int gkm_ensemble_create(int n, const gkm_config* cfgs, gkm_ensemble** out)
         }
         if (t0[d] < 0) return efail(e, GKM_EINVAL, "no sweep tile fits every member's grid");
     }
-    return ens_build(e, t0);
+    return ens_choose(e, t0, t0);
 }
 
 void gkm_ensemble_destroy(gkm_ensemble* e)
@@ -1621,7 +1631,7 @@ int gkm_ensemble_set_tiles(gkm_ensemble* e, const int tile[3])
         for (gkm_ctx* c : e->mem)
             if (!gkm::sweep_tile_ok(d, tile[d], c->nc))
                 return efail(e, GKM_EINVAL, "tile variant out of range or larger than a member's grid");
-    return ens_build(e, tile);
+    return ens_choose(e, tile, tile);
 }
 
 int gkm_ensemble_autotune(gkm_ensemble* e, int reps, int tile[3], double ms[9])
@@ -1681,23 +1691,23 @@ int gkm_ensemble_autotune(gkm_ensemble* e, int reps, int tile[3], double ms[9])
         if (rc) return rc;
         sweeps += best_ms;
     }
-    if (e->mixed && !e->small && !e->persistent) {
-        // the two-launch step goes with the first variants: keep them where it is
-        // faster (the persistent step sweeps: 64 members, 6.54 ms with them, 6.2 with
-        // the fastest)
-        const int t[3] = {e->tile[0], e->tile[1], e->tile[2]}, zero[3] = {0, 0, 0};
-        bool ok = true;
-        for (gkm_ctx* c : e->mem) ok = ok && c->faces;
-        if (ok) {
-            double avg = 0.0;
-            rc = ens_build(e, zero);
-            if (rc) return rc;
-            rc = average([&] { return ens_small_step(e, p); }, &avg);
-            if (rc) return rc;
-            if (avg >= sweeps) rc = ens_build(e, t);
-            if (rc) return rc;
-        }
+    // the two-launch step goes with the first variants: keep them for it where it
+    // is faster than the fastest sweeps (the persistent step sweeps: 64 members,
+    // 6.54 ms with the first variants, 6.2 with the fastest)
+    int step[3] = {best[0], best[1], best[2]};
+    bool ok = e->mixed && !e->small;
+    for (gkm_ctx* c : e->mem) ok = ok && c->faces;
+    if (ok) {
+        const int zero[3] = {0, 0, 0};
+        double avg = 0.0;
+        rc = ens_build(e, zero);
+        if (rc) return rc;
+        rc = average([&] { return ens_small_step(e, p); }, &avg);
+        if (rc) return rc;
+        if (avg < sweeps) std::copy(zero, zero + 3, step);
     }
+    rc = ens_choose(e, step, best);
+    if (rc) return rc;
     if (tile)
         for (int d = 0; d < 3; d++) tile[d] = e->tile[d];
     return GKM_OK;
@@ -1784,7 +1794,13 @@ int gkm_ensemble_set_persistent(gkm_ensemble* e, int on)
             return efail(e, GKM_ENOMEM, "hipMalloc barrier");
         EHIPCHK(e, hipMemset(e->dbar, 0, gkm::kPersistSyncWords * sizeof(unsigned long long)));
     }
-    if (e->persistent != (on != 0)) drop_graphs(e);
+    if (e->persistent == (on != 0)) return GKM_OK;
+    const int* t = on ? e->persist_tile : e->step_tile;
+    if (!std::equal(t, t + 3, e->tile)) {  // after an autotune
+        const int rc = ens_build(e, t);
+        if (rc) return rc;
+    }
+    drop_graphs(e);
     e->persistent = on != 0;
     return GKM_OK;
 }

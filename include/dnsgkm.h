@@ -206,8 +206,10 @@ gkm_ctx *gkm_ensemble_member(gkm_ensemble *e, int m);
 /* one tile variant per direction for all members; gkm_ensemble_autotune times
  * every variant of every direction on the members' current states (which it
  * does not change) and keeps the fastest, or variant 0 throughout where the
- * two-launch step is faster, as gkm_autotune (not in persistent mode, which
- * sweeps); ms (may be NULL) as gkm_autotune */
+ * two-launch step is faster, as gkm_autotune.  The persistent mode, which always
+ * sweeps, keeps the fastest ones for itself, whichever of autotune and
+ * set_persistent comes first.  tile (may be NULL) receives the choice for the
+ * mode the ensemble is in, ms (may be NULL) as gkm_autotune */
 int gkm_ensemble_set_tiles(gkm_ensemble *e, const int tile[3]);
 int gkm_ensemble_autotune(gkm_ensemble *e, int reps, int tile[3], double ms[9]);
 /* nsteps steps of every member, each with dt from its own CFL condition */
@@ -216,7 +218,7 @@ int gkm_ensemble_run(gkm_ensemble *e, int nsteps, int use_graph);
  * as stay resident; every phase -- CFL, x, y, z sweeps, tracer splines and
  * Heun -- takes its work items from the same tables, phases separated by grid
  * barriers with a bounded wait); results equal the per-phase launches' bit
- * for bit.  A barrier that timed out makes gkm_ensemble_run fail. */
+ * for bit with the same tiles (GKM_FP64: with any).  A barrier that timed out makes gkm_ensemble_run fail. */
 int gkm_ensemble_set_persistent(gkm_ensemble *e, int on);
 /* one persistent step (eager) with the wall-clock time of each phase, as
  * workgroup 0 saw the barriers: *nphases = 5 (CFL maxima + tracer velocities,
