@@ -579,10 +579,12 @@ __device__ __forceinline__ void sweep_body(const SweepArgs& p, int bid, int nblk
 
         // y sweep: the sum so far of the chunk's cells, loaded ahead of the flux,
         // which hides the latency (256^3, 2 x 8 x 16 tile: 2.16 -> 1.98 ms; the z
-        // sweep with its carry has no registers left for it, 2.42 -> 2.58 ms)
+        // sweep with its carry has no registers left for it, 2.42 -> 2.58 ms, nor
+        // has the persistent step's kernel, 5.56 -> 5.71 ms for 64 members)
+        constexpr bool AHEAD = DIR == 1 && !EXT;
         const bool upd = c >= 0 && live && (!GEN || n0 + tn < seg_end);
         double old[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-        if (DIR == 1 && upd && p.mode != 0) {
+        if (AHEAD && upd && p.mode != 0) {
             const long idx = cell_index<DIR>(n0 + tn, a0 + ta, b0 + tb, nc);
 #pragma unroll
             for (int q = 0; q < 5; q++) old[q] = p.dW[q * plane + idx];
@@ -628,7 +630,7 @@ __device__ __forceinline__ void sweep_body(const SweepArgs& p, int bid, int nblk
                 // unless asked for its flux differences alone (mode 0), the z
                 // sweep updates unless asked for its flux differences alone
                 if (DIR == 0 || p.mode == 0) p.dW[o] = dF;
-                else if (DIR == 1) p.dW[o] = old[q] + dF;
+                else if (DIR == 1) p.dW[o] = (AHEAD ? old[q] : p.dW[o]) + dF;
                 else if (CMP == 1 || (CMP < 0 && p.cmp_out)) {
                     // W^{n+1} + e = W^n + (increment + carried error), exactly (TwoSum);
                     // z sweep: n = z, a = x, b = y
