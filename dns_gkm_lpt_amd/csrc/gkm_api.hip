@@ -52,6 +52,7 @@ struct gkm_ctx {
     double* hist = nullptr;        // behind dscal: dt of the last kHist steps of gkm_run
     bool have_state = false;
     int tile[3] = {0, 0, 0};       // sweep tile variant per direction
+    bool two_launch = true;        // false: an autotune found the sweeps faster than the two-launch step
     int slots = 512;               // concurrent sweep workgroups: 2 per CU
     std::string err;
     gkm::HostPipe pipe;            // copies of whole states and tracer arrays to and from the caller's memory
@@ -134,13 +135,14 @@ gkm::SweepArgs sweep_args(const gkm_ctx* c, int dir, int mode)
 }
 
 // Two launches instead of three sweeps (gkm::launch_small_step) where the grid
-// is small and nothing asks for the sweeps one by one; the results are those of
-// the sweeps in their first tile variants.  Mixed variants round differently
-// (FP32 contractions), so a mixed context with another one keeps its sweeps.
+// is small, no autotune found the sweeps faster and nothing asks for them one by
+// one; the results are those of the sweeps in their first tile variants.  Mixed
+// variants round differently (FP32 contractions), so a mixed context with another
+// one keeps its sweeps.
 bool small_step(const gkm_ctx* c)
 {
     const bool first = !c->tile[0] && !c->tile[1] && !c->tile[2];
-    return c->faces && !c->timing && (first || c->cfg.precision != GKM_MIXED);
+    return c->faces && c->two_launch && !c->timing && (first || c->cfg.precision != GKM_MIXED);
 }
 
 int eulerian_step(gkm_ctx* c)
@@ -602,6 +604,7 @@ int gkm_set_sweep_tiles(gkm_ctx* c, const int tile[3])
         if (!gkm::sweep_tile_ok(d, tile[d], c->nc))
             return fail(c, GKM_EINVAL, "tile variant out of range or larger than the grid");
     for (int d = 0; d < 3; d++) c->tile[d] = tile[d];
+    c->two_launch = true;
     return GKM_OK;
 }
 
@@ -660,13 +663,14 @@ int gkm_autotune(gkm_ctx* c, int reps, int tile[3], double ms[9])
         c->tile[dir] = best_v;
         sweeps += best;
     }
-    if (c->faces && mixed) {
-        // the two-launch step goes with the first variants: keep them where it is faster
+    if (c->faces) {
         double avg = 0.0;
-        rc = average([&] { return gkm::launch_small_step(sweep_args(c, 0, 0), c->faces, nullptr, c->slots, true, c->stream); },
+        rc = average([&] { return gkm::launch_small_step(sweep_args(c, 0, 0), c->faces, nullptr, c->slots, mixed, c->stream); },
                      &avg);
         if (rc) return rc;
-        if (avg < sweeps)
+        c->two_launch = avg < sweeps;
+        // the mixed two-launch step goes with the first variants
+        if (mixed && c->two_launch)
             for (int d = 0; d < 3; d++) c->tile[d] = 0;
     }
     if (tile)
@@ -1134,6 +1138,7 @@ struct gkm_ensemble {
     int* dsfirst = nullptr;           // [3 member + 1] blocks of dface, [member + 1] of dupd
     int nfblk = 0, nublk = 0;
     bool small = false;
+    bool two_launch = true;  // false: an autotune found the sweeps faster
     int nblk[3] = {0, 0, 0};
     bool exact[3] = {false, false, false};  // per direction: tile and segment divide every member's grid
     bool compensated = false;               // every member's z sweep takes the compensated update
@@ -1294,7 +1299,7 @@ int ens_build(gkm_ensemble* e, const int t[3])
     double cells = 0.0;
     for (int d = 0; d < 3; d++) e->tile[d] = t[d];
     for (const gkm_ctx* c : e->mem) {
-        e->small = e->small && c->faces && (!e->mixed || (!t[0] && !t[1] && !t[2]));
+        e->small = e->small && e->two_launch && c->faces && (!e->mixed || (!t[0] && !t[1] && !t[2]));
         cells += (double)c->plane;
     }
     if (e->small) {
@@ -1631,6 +1636,7 @@ int gkm_ensemble_set_tiles(gkm_ensemble* e, const int tile[3])
         for (gkm_ctx* c : e->mem)
             if (!gkm::sweep_tile_ok(d, tile[d], c->nc))
                 return efail(e, GKM_EINVAL, "tile variant out of range or larger than a member's grid");
+    e->two_launch = true;
     return ens_choose(e, tile, tile);
 }
 
@@ -1691,20 +1697,22 @@ int gkm_ensemble_autotune(gkm_ensemble* e, int reps, int tile[3], double ms[9])
         if (rc) return rc;
         sweeps += best_ms;
     }
-    // the two-launch step goes with the first variants: keep them for it where it
-    // is faster than the fastest sweeps (the persistent step sweeps: 64 members,
-    // 6.54 ms with the first variants, 6.2 with the fastest)
+    // the two-launch step where it is faster than the fastest sweeps, in mixed
+    // precision with the first variants, which it goes with (the persistent step
+    // sweeps)
     int step[3] = {best[0], best[1], best[2]};
-    bool ok = e->mixed && !e->small;
+    bool ok = true;
     for (gkm_ctx* c : e->mem) ok = ok && c->faces;
     if (ok) {
         const int zero[3] = {0, 0, 0};
         double avg = 0.0;
-        rc = ens_build(e, zero);
+        e->two_launch = true;
+        rc = ens_build(e, e->mixed ? zero : best);
         if (rc) return rc;
         rc = average([&] { return ens_small_step(e, p); }, &avg);
         if (rc) return rc;
-        if (avg < sweeps) std::copy(zero, zero + 3, step);
+        e->two_launch = avg < sweeps;
+        if (e->mixed && e->two_launch) std::copy(zero, zero + 3, step);
     }
     rc = ens_choose(e, step, best);
     if (rc) return rc;

@@ -112,17 +112,23 @@ int gkm_run(gkm_ctx *ctx, int nsteps, double *dt_hist);
  * A per-direction parity hook for derivsX/Y/Z (update.cpp:214-503). */
 int gkm_sweep_flux_diff(gkm_ctx *ctx, int dir, double dt, double *out);
 /* Sweep tile shape per direction (x, y, z): variant 0..2 of
- * {faces along the sweep axis} x {tangential lines} per workgroup; results do
- * not depend on it.  No reference counterpart (the reference's CUDA path
- * fixes its block shapes in GPUupdate.cu:119-202). */
+ * {faces along the sweep axis} x {tangential lines} per workgroup.  GKM_FP64
+ * results do not depend on it; GKM_MIXED variants differ by the rounding of
+ * their FP32 terms.  The shapes are those of the sweeps.  GKM_FP64 grids up to
+ * 160^3 step in two launches (all faces, then the update) whatever the tiles,
+ * unless gkm_autotune found the sweeps faster; GKM_MIXED grids of even nc up to
+ * 256 do so with variant 0 in all three directions, whose results they give.
+ * Setting tiles forgets what an autotune found.  No reference counterpart (the
+ * reference's CUDA path fixes its block shapes in GPUupdate.cu:119-202). */
 int gkm_set_sweep_tiles(gkm_ctx *ctx, const int tile[3]);
 int gkm_get_sweep_tiles(const gkm_ctx *ctx, int tile[3]);
 /* Time every tile variant of every sweep on the resident state (reps timed
- * launches each after one warm-up, the CFL dt of the state) and keep the
- * fastest per direction -- or variant 0 in all three where a GKM_MIXED step of
- * this grid in two launches, which goes with them, is faster.  The resident state is not changed.  tile (may be
- * NULL) receives the choice, ms (may be NULL, 9 doubles) the average launch
- * time of variant v of direction d at [3 d + v]. */
+ * launches each after one warm-up, the CFL dt of the state) and the two-launch
+ * step where the grid has one, and keep what is faster: the fastest sweeps, or
+ * the two-launch step (GKM_MIXED: then with variant 0 in all three directions).
+ * The resident state is not changed.  tile (may be NULL) receives the choice, ms
+ * (may be NULL, 9 doubles) the average launch time of variant v of direction d at
+ * [3 d + v]. */
 int gkm_autotune(gkm_ctx *ctx, int reps, int tile[3], double ms[9]);
 /* Wait for all work on the context's stream. */
 int gkm_sync(gkm_ctx *ctx);
@@ -205,11 +211,11 @@ const char *gkm_ensemble_last_error(const gkm_ensemble *e);
 gkm_ctx *gkm_ensemble_member(gkm_ensemble *e, int m);
 /* one tile variant per direction for all members; gkm_ensemble_autotune times
  * every variant of every direction on the members' current states (which it
- * does not change) and keeps the fastest, or variant 0 throughout where the
- * two-launch step is faster, as gkm_autotune.  The persistent mode, which always
- * sweeps, keeps the fastest ones for itself, whichever of autotune and
- * set_persistent comes first.  tile (may be NULL) receives the choice for the
- * mode the ensemble is in, ms (may be NULL) as gkm_autotune */
+ * does not change) and the two-launch step, and keeps what is faster, as
+ * gkm_autotune.  The persistent mode, which always sweeps, keeps the fastest
+ * sweeps for itself, whichever of autotune and set_persistent comes first.  tile
+ * (may be NULL) receives the choice for the mode the ensemble is in, ms (may be
+ * NULL) as gkm_autotune */
 int gkm_ensemble_set_tiles(gkm_ensemble *e, const int tile[3]);
 int gkm_ensemble_autotune(gkm_ensemble *e, int reps, int tile[3], double ms[9]);
 /* nsteps steps of every member, each with dt from its own CFL condition */
