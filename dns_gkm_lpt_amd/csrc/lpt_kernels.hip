@@ -278,12 +278,12 @@ hipError_t launch_sample(long np, const double* pos, const double* const cu[3], 
 // gathers one field after the other (10^5 tracers at
 // 240^3, where they touch most of the eight fields' 950 MB: 347 -> 215 us; 2^18 at
 // 128^3: 318 -> 172).
-__global__ __launch_bounds__(256) void props_kernel(long np, unsigned bpf, const double* __restrict__ pos,
-                                                    const int* __restrict__ tag, const double* const* __restrict__ cs,
-                                                    Geom g, double* __restrict__ out)
+__global__ __launch_bounds__(256) void props_kernel(long np, const double* __restrict__ pos, const int* __restrict__ tag,
+                                                    const double* const* __restrict__ cs, Geom g,
+                                                    double* __restrict__ out)
 {
-    const int f = (int)(blockIdx.x / bpf);
-    const long t = (long)(blockIdx.x - f * bpf) * blockDim.x + threadIdx.x;
+    const int f = blockIdx.z;
+    const long t = thread_at(blockIdx.x, blockIdx.y, threadIdx.x);
     const long p = t >> 2;
     const int lane = (int)(t & 3);
     if (p >= np) return;
@@ -364,8 +364,7 @@ hipError_t launch_props(long np, const double* pos, const int* tag, const double
                         double* out, hipStream_t s)
 {
     if (np <= 0) return hipSuccess;
-    const unsigned bpf = blocks_for(4 * np, 256);
-    hipLaunchKernelGGL(props_kernel, dim3(8 * bpf), dim3(256), 0, s, np, bpf, pos, tag, cs_dev, g, out);
+    hipLaunchKernelGGL(props_kernel, thread_grid(4 * np, 8), dim3(256), 0, s, np, pos, tag, cs_dev, g, out);
     return hipGetLastError();
 }
 

@@ -60,6 +60,17 @@ hipError_t launch_prefilter_velocity(const double* W, long plane, double gam, co
                                      double* const coef[3], hipStream_t s);
 // spline of the Laplacian of spline c (knot values, then prefilter in place)
 hipError_t launch_lap_spline(const double* c, const Geom& g, const double* pivots, double* lap, hipStream_t s);
+// Blocks of 256 for n threads, up to 2^23 of them along x and the others along y: the
+// runtime counts the threads along one axis in 32 bits and runs 2^24 + 8 blocks of
+// 256 as 8, with no error.  thread_at: a thread's place among them, n or more for
+// those of the last row's blocks that are not needed.
+constexpr long kGridX = 1L << 23;
+inline dim3 thread_grid(long n, unsigned z = 1)
+{
+    const long b = (n + 255) / 256;
+    return b <= kGridX ? dim3((unsigned)b, 1, z) : dim3((unsigned)kGridX, (unsigned)((b + kGridX - 1) / kGridX), z);
+}
+__host__ __device__ inline long thread_at(unsigned x, unsigned y, unsigned t) { return ((long)y * kGridX + x) * 256 + t; }
 // full particle properties, kPropWidth doubles per particle written to row tag[p];
 // cs_dev is a device array of the 8 spline pointers {rho, u, v, w, p, lap u, lap v, lap w}
 constexpr int kPropWidth = 41;

@@ -58,7 +58,7 @@ __global__ void gather_kernel(long np, const int* __restrict__ perm, const doubl
 __global__ void scatter_kernel(long np, const int* __restrict__ tag, const double* __restrict__ src, int width, int part,
                                double* __restrict__ dst)
 {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long i = thread_at(blockIdx.x, blockIdx.y, threadIdx.x);
     if (i >= np * width) return;
     const long p = i / width;
     const int c = (int)(i - p * width);
@@ -105,7 +105,7 @@ hipError_t scatter_to_tags(long np, const int* tag, const double* src, int width
 {
     if (np <= 0) return hipSuccess;
     if (width < 1 || part < 1 || width % part) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(scatter_kernel, dim3(nblocks(np * width)), dim3(256), 0, st, np, tag, src, width, part, dst);
+    hipLaunchKernelGGL(scatter_kernel, thread_grid(np * width), dim3(256), 0, st, np, tag, src, width, part, dst);
     return hipGetLastError();
 }
 
