@@ -322,6 +322,7 @@ int sweep_seg_len(int dir, int nc, int tile, int slots, bool mixed)
         long best_cost = -1;
         for (int parts = 1;; parts *= 2) {
             const int seg = cdiv(lchunks, parts) * CN;
+            if (seg == nc - 1) continue;  // its last workgroups run past one wrap (sweep_seg_most)
             const long blocks = pencils * cdiv(nc, seg);
             const long cost = (blocks + slots - 1) / slots * (seg / CN + 1);
             if (best_cost < 0 || cost < best_cost) {
@@ -338,7 +339,12 @@ int sweep_seg_len(int dir, int nc, int tile, int slots, bool mixed)
 int sweep_seg_most(int dir, int nc, int tile, int most, bool mixed)
 {
     if (!sweep_tile_ok(dir, tile, nc) || most < 1) return 0;
-    return equal_parts(nc, tile_shape(dir, tile, mixed)[0], most);
+    const int CN = tile_shape(dir, tile, mixed)[0];
+    const int seg = equal_parts(nc, CN, most);
+    // a last segment of one face whose workgroups run on to cell 2 nc, one past
+    // what a single wrap reaches (33^3 in segments of 32, 17^3 in segments of 16):
+    // the next shorter ones
+    return seg == nc - 1 ? equal_parts(nc, CN, seg / CN - 1) : seg;
 }
 
 template <int DIR, int V>
