@@ -168,9 +168,16 @@ int eulerian_step(gkm_ctx* c)
 // a non-physical state
 int read_scalars(gkm_ctx* c)
 {
-    if (!c->hscal && hipHostMalloc(reinterpret_cast<void**>(&c->hscal), sizeof(double) * kScal, hipHostMallocDefault) != hipSuccess) {
-        c->hscal = nullptr;
-        return fail(c, GKM_ENOMEM, "hipHostMalloc scalars");
+    if (!c->hscal) {
+        int was = c->cfg.device;  // the caller may have another device current
+        HIPCHK(c, hipGetDevice(&was));
+        HIPCHK(c, hipSetDevice(c->cfg.device));
+        const hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&c->hscal), sizeof(double) * kScal, hipHostMallocDefault);
+        (void)hipSetDevice(was);
+        if (e != hipSuccess) {
+            c->hscal = nullptr;
+            return fail(c, GKM_ENOMEM, "hipHostMalloc scalars");
+        }
     }
     HIPCHK(c, hipMemcpyAsync(c->hscal, c->dscal, sizeof(double) * kScal, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));

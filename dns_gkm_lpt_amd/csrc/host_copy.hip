@@ -34,6 +34,30 @@ int usable_cpus()
     return 1;
 }
 
+// the device of a stream made current, and the caller's again afterwards
+class OnDeviceOf {
+  public:
+    explicit OnDeviceOf(hipStream_t s)
+    {
+        int dev = -1;
+        ok_ = hipGetDevice(&was_) == hipSuccess && hipStreamGetDevice(s, &dev) == hipSuccess;
+        if (ok_ && dev != was_) {
+            ok_ = hipSetDevice(dev) == hipSuccess;
+            changed_ = ok_;
+        }
+        if (!ok_) (void)hipGetLastError();
+    }
+    ~OnDeviceOf()
+    {
+        if (changed_) (void)hipSetDevice(was_);
+    }
+    bool ok() const { return ok_; }
+
+  private:
+    int was_ = 0;
+    bool ok_ = false, changed_ = false;
+};
+
 // memory the runtime knows (pinned, managed, on a device): the device reaches it
 // itself, and host code may not
 bool known_to_runtime(const void* p)
@@ -64,12 +88,16 @@ void HostPipe::release()
     chunk_ = 0;
 }
 
-// pinned buffers for copies of `bytes` in all; false if there are none to be had
-bool HostPipe::ready(size_t bytes)
+// pinned buffers for copies of `bytes` in all on s's device, whichever is current
+// (an event is recorded on its own device's streams only); false if there are none
+// to be had
+bool HostPipe::ready(size_t bytes, hipStream_t s)
 {
     const size_t want = std::min(kChunk, ((bytes + kDepth - 1) / kDepth + kSlice - 1) / kSlice * kSlice);
     if (chunk_ >= want) return true;
     release();
+    const OnDeviceOf here(s);
+    if (!here.ok()) return false;
     if (hipHostMalloc(reinterpret_cast<void**>(&buf_), kDepth * want, hipHostMallocDefault) != hipSuccess) {
         (void)hipGetLastError();
         buf_ = nullptr;
@@ -104,7 +132,7 @@ hipError_t HostPipe::run(const CopySeg* seg, int n, hipStream_t s, bool to_host)
     for (int i = 0; i < n; i++)
         if (known_to_runtime(seg[i].host)) return plain(seg, n, s, to_host);
     const int nthr = (int)std::min<size_t>(std::min(usable_cpus(), 8), total / (size_t(2) << 20) + 1);
-    if (nthr < 2 || !ready(total)) return plain(seg, n, s, to_host);
+    if (nthr < 2 || !ready(total, s)) return plain(seg, n, s, to_host);
 
     std::vector<Chunk> chunks;
     std::vector<std::thread> threads;

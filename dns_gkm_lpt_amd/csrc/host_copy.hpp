@@ -31,7 +31,7 @@ class HostPipe {
   private:
     hipError_t run(const CopySeg* seg, int n, hipStream_t s, bool to_host);
     hipError_t plain(const CopySeg* seg, int n, hipStream_t s, bool to_host);
-    bool ready(size_t bytes);
+    bool ready(size_t bytes, hipStream_t s);
 
     char* buf_ = nullptr;
     size_t chunk_ = 0;  // bytes of each of the kDepth buffers
