@@ -16,7 +16,10 @@
 
 #include <algorithm>
 #include <atomic>
+#include <condition_variable>
+#include <cstdio>
 #include <cstring>
+#include <mutex>
 #include <thread>
 #include <vector>
 
@@ -26,12 +29,19 @@ namespace {
 
 constexpr size_t kSlice = size_t(1) << 20;
 
+// CPUs the process may use: its affinity, and a container's CPU quota, under which
+// more threads than it pays for only stop each other
 int usable_cpus()
 {
     cpu_set_t set;
     CPU_ZERO(&set);
-    if (sched_getaffinity(0, sizeof(set), &set) == 0) return std::max(1, CPU_COUNT(&set));
-    return 1;
+    int n = sched_getaffinity(0, sizeof(set), &set) == 0 ? CPU_COUNT(&set) : 1;
+    double quota = 0.0, period = 0.0;
+    if (FILE* f = std::fopen("/sys/fs/cgroup/cpu.max", "r")) {  // "max <period>" without a limit
+        if (std::fscanf(f, "%lf %lf", &quota, &period) == 2 && period > 0.0) n = std::min(n, (int)(quota / period));
+        std::fclose(f);
+    }
+    return std::max(1, n);
 }
 
 // the device of a stream made current, and the caller's again afterwards
@@ -133,6 +143,15 @@ hipError_t HostPipe::run(const CopySeg* seg, int n, hipStream_t s, bool to_host)
         if (known_to_runtime(seg[i].host)) return plain(seg, n, s, to_host);
     const int nthr = (int)std::min<size_t>(std::min(usable_cpus(), 8), total / (size_t(2) << 20) + 1);
     if (nthr < 2 || !ready(total, s)) return plain(seg, n, s, to_host);
+    // The threads' waits spin, which is for the times between two chunks only: while
+    // the stream's earlier work runs, they sleep (down: until the first chunk has
+    // arrived) or are not there yet (up).
+    if (!to_host) {
+        const hipError_t before = hipStreamSynchronize(s);
+        if (before != hipSuccess) return before;
+    }
+    std::mutex gate_mutex;
+    std::condition_variable gate;
 
     std::vector<Chunk> chunks;
     std::vector<std::thread> threads;
@@ -163,6 +182,10 @@ hipError_t HostPipe::run(const CopySeg* seg, int n, hipStream_t s, bool to_host)
         left[i % kDepth].fetch_sub(1, std::memory_order_release);
     };
     auto worker = [&] {
+        {
+            std::unique_lock<std::mutex> hold(gate_mutex);
+            gate.wait(hold, [&] { return filled.load(std::memory_order_relaxed) > 0 || stop.load(std::memory_order_relaxed); });
+        }
         for (;;) {
             const int k = next.fetch_add(1, std::memory_order_relaxed);
             if (k >= nch * per) return;
@@ -182,6 +205,10 @@ hipError_t HostPipe::run(const CopySeg* seg, int n, hipStream_t s, bool to_host)
     }
     if (threads.empty()) return plain(seg, n, s, to_host);
 
+    auto open_gate = [&] {
+        { std::lock_guard<std::mutex> hold(gate_mutex); }
+        gate.notify_all();
+    };
     // buffer b's last chunk moved on by the threads
     auto drained = [&](int b) {
         while (left[b].load(std::memory_order_acquire) > 0) std::this_thread::yield();
@@ -201,6 +228,7 @@ hipError_t HostPipe::run(const CopySeg* seg, int n, hipStream_t s, bool to_host)
             if (e == hipSuccess) {
                 left[i % kDepth].store(per, std::memory_order_relaxed);
                 filled.store(i + 1, std::memory_order_release);
+                if (i == 0) open_gate();
             }
         }
     } else {
@@ -211,6 +239,7 @@ hipError_t HostPipe::run(const CopySeg* seg, int n, hipStream_t s, bool to_host)
                 if (open >= kDepth) e = hipEventSynchronize(ev_[open % kDepth]);
                 left[open % kDepth].store(per, std::memory_order_relaxed);
                 filled.store(open + 1, std::memory_order_release);
+                if (open == 0) open_gate();
             }
             if (e != hipSuccess) break;
             const int b = i % kDepth;
@@ -220,6 +249,7 @@ hipError_t HostPipe::run(const CopySeg* seg, int n, hipStream_t s, bool to_host)
         }
     }
     if (e != hipSuccess) stop.store(true, std::memory_order_relaxed);
+    open_gate();
     for (auto& t : threads) t.join();
     const hipError_t es = hipStreamSynchronize(s);
     return e != hipSuccess ? e : es;

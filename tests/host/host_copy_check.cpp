@@ -1,8 +1,9 @@
 // csrc/host_copy.hip on the host, over the fake runtime of fake_hip: bytes of copies
 // both ways (below and above the ring's threshold, tails, several segments), a stream
-// of another device than the current one, and a copy that fails.  Exit status 1 and a
-// line per failure.
+// of another device than the current one, a copy that fails, and the CPU time spent
+// while the stream's earlier work runs.  Exit status 1 and a line per failure.
 #include <cstdio>
+#include <ctime>
 #include <random>
 #include <vector>
 
@@ -15,6 +16,12 @@ static void expect(bool ok, const char* what)
         std::printf("FAILED: %s\n", what);
         bad = 1;
     }
+}
+static double cpu_seconds()
+{
+    timespec t;
+    clock_gettime(CLOCK_PROCESS_CPUTIME_ID, &t);
+    return (double)t.tv_sec + 1e-9 * (double)t.tv_nsec;
 }
 
 int main()
@@ -55,6 +62,19 @@ int main()
         fake::fail_at = fake::copies + at;
         expect(p.to_device(&seg, 1, &s) != hipSuccess, "a failing copy up is reported");
         fake::fail_at = -1;
+        p.release();
+    }
+    for (bool down : {true, false}) {
+        gkm::HostPipe p;
+        expect(p.to_host(&seg, 1, &s) == hipSuccess, "a first copy");
+        const int ring = fake::pinned;
+        s.busy = 0.5;
+        const double t = cpu_seconds();
+        expect((down ? p.to_host(&seg, 1, &s) : p.to_device(&seg, 1, &s)) == hipSuccess, "a copy behind other work");
+        const double used = cpu_seconds() - t;
+        std::printf("%s behind 0.5 s of other work: %.3f s of CPU\n", down ? "down" : "up", used);
+        expect(used < 0.25, "no CPU time while the stream's earlier work runs");
+        expect(fake::pinned == ring, "the ring is kept");
         p.release();
     }
     std::printf("%s\n", bad ? "wrong" : "all right");

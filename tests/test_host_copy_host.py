@@ -1,6 +1,8 @@
 """The ring of pinned buffers that large host copies go through (csrc/host_copy.hip),
 on the host over a fake runtime (tests/host/fake_hip): bytes, a stream of another
-device than the current one, failing copies."""
+device than the current one, failing copies, and no CPU time spent while the
+stream's earlier work runs (0.5 s of it; the copy itself takes some 0.05 s of CPU,
+eight threads spinning through it take 2 s or all the CPUs there are)."""
 import os
 import shutil
 import subprocess
