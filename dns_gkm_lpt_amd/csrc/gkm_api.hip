@@ -32,7 +32,7 @@ struct gkm_ctx {
     double dx = 0.0;
     gkm::Gas<double> gas{};
     hipStream_t stream = nullptr;
-    double* slab = nullptr;  // holds W, dW, faces, stage, dscal, hist, partial and a mixed context's cmp
+    double* slab = nullptr;  // holds W, dW, stage, faces over both, dscal, hist, partial and a mixed context's cmp
     double* W[2] = {nullptr, nullptr};
     int cur = 0;
     double* dW = nullptr;
@@ -48,7 +48,7 @@ struct gkm_ctx {
     int* dflag = nullptr;          // in dscal[3]: non-physical-state flag, ticket of the step's CFL
     double* hscal = nullptr;       // pinned copy of dscal
     double* partial = nullptr;     // CFL block maxima
-    double* faces = nullptr;       // face fluxes of the three directions (small grids)
+    double* faces = nullptr;       // face fluxes of the three directions (small grids), over dW and stage
     double* hist = nullptr;        // behind dscal: dt of the last kHist steps of gkm_run
     bool have_state = false;
     int tile[3] = {0, 0, 0};       // sweep tile variant per direction
@@ -194,11 +194,9 @@ int cfl_on_device(gkm_ctx* c, double* hist = nullptr)
     });
 }
 
-}  // namespace
-
-extern "C" {
-
-int gkm_create(const gkm_config* cfg, gkm_ctx** out)
+// gkm_create; two_launch: with memory for the two-launch step where the grid has
+// one and the memory is there
+int create(const gkm_config* cfg, bool two_launch, gkm_ctx** out)
 {
     if (!cfg || !out) return GKM_EINVAL;
     *out = nullptr;
@@ -238,15 +236,25 @@ int gkm_create(const gkm_config* cfg, gkm_ctx** out)
     // context per call; create at 128^3 0.6-1.2 -> 0.3 ms, at 512^3 1.6 -> 0.7)
     const bool mixed = cfg->precision == GKM_MIXED;
     const size_t state = 5 * (size_t)c->plane, staged = 5 * (size_t)c->padded;
-    // face fluxes of the two-launch step: the y and z directions' behind dW's 5 planes
-    const size_t faces = gkm::small_step_ok(nc, mixed) ? 2 * state : 0;
     const size_t carry = mixed ? (5 * (size_t)gkm::carry_plane(nc) + 1) / 2 : 0;  // floats, in doubles
     auto even = [](size_t n) { return (n + 31) & ~size_t(31); };               // 256 B
-    const size_t sizes[] = {even(state), even(state), even(state + faces), even(staged), even(kScal + kHist),
-                            even(gkm::kCflBlocks), even(carry), even(carry)};
-    size_t total = 0;
-    for (size_t n : sizes) total += n;
-    if (hipMalloc(&c->slab, sizeof(double) * total) != hipSuccess) return fail(c, GKM_ENOMEM, "hipMalloc state");
+    // dW and the staging area behind it.  The face fluxes of the two-launch step, 15
+    // planes, lie over both: no copy is staged while a step runs.
+    const size_t work = even(state) + even(staged), faces = even(3 * state);
+    size_t sizes[] = {even(state), even(state), std::max(work, faces), even(kScal + kHist), even(gkm::kCflBlocks),
+                      even(carry), even(carry)};
+    auto allocate = [&] {
+        size_t total = 0;
+        for (size_t n : sizes) total += n;
+        return hipMalloc(&c->slab, sizeof(double) * total) == hipSuccess;
+    };
+    two_launch = two_launch && gkm::small_step_ok(nc, mixed);
+    if (!two_launch || !allocate()) {
+        (void)hipGetLastError();
+        two_launch = false;
+        sizes[2] = work;
+        if (!allocate()) return fail(c, GKM_ENOMEM, "hipMalloc state");
+    }
     double* at = c->slab;
     auto take = [&](int k) {
         double* p = at;
@@ -256,22 +264,28 @@ int gkm_create(const gkm_config* cfg, gkm_ctx** out)
     c->W[0] = take(0);
     c->W[1] = take(1);
     c->dW = take(2);
-    if (faces) c->faces = c->dW;
-    c->stage = take(3);
-    c->dscal = take(4);
+    if (two_launch) c->faces = c->dW;
+    c->stage = c->dW + even(state);
+    c->dscal = take(3);
     c->dflag = reinterpret_cast<int*>(c->dscal + 3);
     c->hist = c->dscal + kScal;
-    c->partial = take(5);
+    c->partial = take(4);
     HIPCHK(c, hipMemsetAsync(c->dscal, 0, sizeof(double) * kScal, c->stream));
     if (mixed) {
         for (int b = 0; b < 2; b++) {
-            c->cmp[b] = reinterpret_cast<float*>(take(6 + b));
+            c->cmp[b] = reinterpret_cast<float*>(take(5 + b));
             HIPCHK(c, hipMemsetAsync(c->cmp[b], 0, sizeof(float) * 5 * (size_t)gkm::carry_plane(nc), c->stream));
         }
         c->compensate = true;
     }
     return GKM_OK;
 }
+
+}  // namespace
+
+extern "C" {
+
+int gkm_create(const gkm_config* cfg, gkm_ctx** out) { return create(cfg, true, out); }
 
 void gkm_destroy(gkm_ctx* c)
 {
@@ -1554,25 +1568,16 @@ int ens_parity(gkm_ensemble* e, int* p)
     return GKM_OK;
 }
 
-}  // namespace
-
-extern "C" {
-
-int gkm_ensemble_create(int n, const gkm_config* cfgs, gkm_ensemble** out)
+// members, tables and streams of an ensemble (gkm_ensemble_create)
+int ens_make(gkm_ensemble* e, int n, const gkm_config* cfgs, bool two_launch)
 {
-    if (!out) return GKM_EINVAL;
-    *out = nullptr;
-    if (n < 1 || n > 4096 || !cfgs) return GKM_EINVAL;
-    auto* e = new (std::nothrow) gkm_ensemble;
-    if (!e) return GKM_ENOMEM;
-    *out = e;
     e->n = n;
     e->mixed = cfgs[0].precision == GKM_MIXED;
     for (int m = 0; m < n; m++) {
         if (cfgs[m].precision != cfgs[0].precision || cfgs[m].device != cfgs[0].device)
             return efail(e, GKM_EINVAL, "members must share precision and device");
         gkm_ctx* c = nullptr;
-        const int rc = gkm_create(&cfgs[m], &c);
+        const int rc = create(&cfgs[m], two_launch, &c);
         if (rc) {
             const std::string msg = c ? c->err : "gkm_create failed";
             gkm_destroy(c);
@@ -1606,9 +1611,8 @@ int gkm_ensemble_create(int n, const gkm_config* cfgs, gkm_ensemble** out)
     return ens_choose(e, t0, t0);
 }
 
-void gkm_ensemble_destroy(gkm_ensemble* e)
+void ens_release(gkm_ensemble* e)
 {
-    if (!e) return;
     if (e->stream) (void)hipStreamSynchronize(e->stream);
     drop_graphs(e);
     for (gkm_ctx* c : e->mem) gkm_destroy(c);
@@ -1625,6 +1629,34 @@ void gkm_ensemble_destroy(gkm_ensemble* e)
     if (e->ev[0]) (void)hipEventDestroy(e->ev[0]);
     if (e->ev[1]) (void)hipEventDestroy(e->ev[1]);
     if (e->stream) (void)hipStreamDestroy(e->stream);
+}
+
+}  // namespace
+
+extern "C" {
+
+int gkm_ensemble_create(int n, const gkm_config* cfgs, gkm_ensemble** out)
+{
+    if (!out) return GKM_EINVAL;
+    *out = nullptr;
+    if (n < 1 || n > 4096 || !cfgs) return GKM_EINVAL;
+    auto* e = new (std::nothrow) gkm_ensemble;
+    if (!e) return GKM_ENOMEM;
+    *out = e;
+    int rc = ens_make(e, n, cfgs, true);
+    if (rc == GKM_ENOMEM) {  // without the members' memory for the two-launch step
+        ens_release(e);
+        *e = gkm_ensemble{};
+        (void)hipGetLastError();
+        rc = ens_make(e, n, cfgs, false);
+    }
+    return rc;
+}
+
+void gkm_ensemble_destroy(gkm_ensemble* e)
+{
+    if (!e) return;
+    ens_release(e);
     delete e;
 }
 
