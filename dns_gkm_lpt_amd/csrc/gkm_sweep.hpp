@@ -488,7 +488,9 @@ __device__ __forceinline__ void sweep_body_pair(const SweepArgs& p, int bid, int
                 else p.Wout[o] = was[k] - p.inv_dx * (old[k] + dF);
             }
         }
-        // the new cells take the places of the oldest, which only this chunk's WENO read
+        // the new cells take the places of the oldest, which this chunk's WENO and its
+        // flux (window positions 2 to CN + 2) have read: the barrier after the flux
+        // stands between
         if (has && c + 1 < nchunk) store(ring_slot<CN>(h, itn), cell);
         h = ring_slot<CN>(h, CN);
         __syncthreads();
@@ -580,8 +582,10 @@ __device__ __forceinline__ void sweep_body(const SweepArgs& p, int bid, int nblk
         // y sweep: the sum so far of the chunk's cells, loaded ahead of the flux,
         // which hides the latency (256^3, 2 x 8 x 16 tile: 2.16 -> 1.98 ms; the z
         // sweep with its carry has no registers left for it, 2.42 -> 2.58 ms, nor
-        // has the persistent step's kernel, 5.56 -> 5.71 ms for 64 members)
-        constexpr bool AHEAD = DIR == 1 && !EXT;
+        // has the persistent step's kernel, 5.56 -> 5.71 ms for 64 members).  Faces
+        // alone have no sum (mode 0), but are scheduled better with the branch in
+        // than without it (128^3 mixed, 769 against 782 us a step)
+        constexpr bool AHEAD = DIR == 1 && (!EXT || FACES);
         const bool upd = c >= 0 && live && (!GEN || n0 + tn < seg_end);
         double old[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
         if (AHEAD && upd && p.mode != 0) {
