@@ -24,9 +24,11 @@
 // Types: TE carries the prelude (primitive states, collision coefficients), the
 // equilibrium state, and the Euler part of the flux (the p0 and p3 terms, which
 // carry dt times the inviscid flux, and the gm1/gm3 terms of the time slope, which
-// cancel to rounding); TS carries every slope-dependent term.  TE = TS = double is
-// the FP64 path, TE = double / TS = float the mixed path, TE = TS = float the
-// all-FP32 diagnostic path.
+// cancel to rounding); TS carries every slope-dependent term.  TE = double /
+// TS = float is the mixed path, TE = TS = float the all-FP32 diagnostic path.  The
+// FP64 path evaluates the same terms by two lanes per face (gkm_pair.hpp); TE = TS =
+// double, one lane, is the form the host checks hold it to and, with dual numbers,
+// the tangent-linear flux.
 #pragma once
 #include "gkm_math.hpp"
 

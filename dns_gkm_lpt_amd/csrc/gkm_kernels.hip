@@ -3,9 +3,11 @@
 // One fused kernel per sweep direction replaces the reference's derivs*_Kernel,
 // flip_Kernel, flux, flipBack_Kernel and update_Kernel chain
 // (GPUupdate.cu:119-202): WENO states of every face a workgroup needs are
-// built once into LDS, each thread then evaluates one GKS face flux, and the
-// flux differences are formed in LDS and accumulated per cell.  Interface
-// states and fluxes never round-trip HBM.
+// built once into LDS, each thread (mixed precision) or pair of threads (FP64)
+// then evaluates one GKS face flux, and the flux differences are formed in LDS
+// and accumulated per cell.  Interface states never leave LDS, nor do the
+// fluxes of the sweeps.  Small grids step in two launches instead (below), whose
+// 15 planes of fluxes go through memory.
 #include "gkm_kernels.hpp"
 #include "gkm_pair.hpp"
 #include "gkm_sweep.hpp"

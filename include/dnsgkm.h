@@ -140,10 +140,10 @@ int gkm_sync(gkm_ctx *ctx);
  * with the same configuration and default tiles (for GKM_MIXED, with
  * compensation off: this step does the plain FP64 update).  No reference
  * counterpart: for callers that cannot allocate (code under HIP graph
- * capture, serving loops).  Its scratch (the flux-difference accumulator and
- * the device dt) is one file-scope device array per GPU sized for nc <= 64;
- * a larger nc is refused with GKM_EINVAL.  Calls that overlap on one GPU race
- * on that array.  msg (may be NULL) receives an error message of at most
+ * capture, serving loops).  Its scratch (the face fluxes of the three directions,
+ * or the flux-difference accumulator of the sweeps, and the device dt) is one
+ * file-scope device array of 31.5 MB per GPU, sized for nc <= 64; a larger nc is
+ * refused with GKM_EINVAL.  Calls that overlap on one GPU race on that array.  msg (may be NULL) receives an error message of at most
  * msglen bytes. */
 int gkm_step_noalloc(const gkm_config *cfg, const double *W, double *Wout, double dt, void *stream, char *msg,
                      int msglen);
@@ -151,7 +151,9 @@ int gkm_step_noalloc(const gkm_config *cfg, const double *W, double *Wout, doubl
 int gkm_stats_compute(gkm_ctx *ctx, gkm_stats *out);
 
 /* Per-kernel timing with HIP events on the context's stream.  While enabled,
- * every sweep/update launch is bracketed by events; gkm_timing_read returns
+ * steps run as three sweeps, also where they run in two launches otherwise (the
+ * results are the same bit for bit, the time per step is not), and every launch
+ * is bracketed by events and waited for; gkm_timing_read returns
  * accumulated milliseconds and launch counts for slots
  * 0 = x sweep, 1 = y sweep, 2 = z sweep (fused flux difference + update),
  * 3 = CFL reduction, 4 = spline prefilter, 5 = particle sample + Heun step,
@@ -194,9 +196,10 @@ int gkm_adjoint_backward(gkm_ctx *ctx, const double *lamN, double *lam0);
 
 /* ---- Ensemble of independent runs (no reference counterpart) -------------
  * n members, each a full context (own grid size, gas, initial condition,
- * CFL dt), stepped together: per step one launch computes every member's dt
- * and one launch per direction sweeps every member; with use_graph the step
- * is a captured HIP graph (one per buffer parity) replayed nsteps times.
+ * CFL dt), stepped together: per step two launches compute every member's dt,
+ * and two form all their faces and update them (three, one sweep per direction,
+ * where some member's grid or the tiles have no two-launch step); with use_graph
+ * the step is a captured HIP graph (one per buffer parity) replayed nsteps times.
  * Tracers uploaded to a member (lpt_upload on gkm_ensemble_member) advance
  * with it exactly as lpt_coupled_step advances them in a single context.
  * Members must share precision and device.  A member's state goes in and out
@@ -271,7 +274,9 @@ int lpt_properties(gkm_ctx *ctx, double *out);
 /* One coupled step of the Evolve loop (update.cpp:124-170) with the resident
  * state: sample U at x from the current field, advance the field by dt
  * (gkm_step), rebuild the velocity spline, Heun-advance the particles
- * (Particle::updatePosition, ParticleTrack.cpp:48-73). */
+ * (Particle::updatePosition, ParticleTrack.cpp:48-73).  Like gkm_step, this and
+ * lpt_heun return once their work is queued: an error of a kernel shows in a
+ * later call, and a host clock around them needs gkm_sync. */
 int lpt_coupled_step(gkm_ctx *ctx, double dt);
 /* Particle-only Heun step against the current field, using the velocities
  * stored by the last lpt_sample (U at the start of the step). */
