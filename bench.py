@@ -82,15 +82,15 @@ MEASURED_VALU_BUSY = {
     ("mixed", 1, 2, 512): 68.1,
     ("mixed", 2, 0, 512): 71.7,
     ("mixed", 2, 2, 512): 65.7,
-    ("fp64", 0, 0, 512): 78.7,
-    ("fp64", 0, 1, 512): 78.7,
-    ("fp64", 0, 2, 512): 86.7,
-    ("fp64", 1, 0, 512): 78.1,
-    ("fp64", 1, 1, 512): 74.0,
-    ("fp64", 1, 2, 512): 80.8,
-    ("fp64", 2, 0, 512): 82.7,
-    ("fp64", 2, 1, 512): 78.7,
-    ("fp64", 2, 2, 512): 83.1,
+    ("fp64", 0, 0, 512): 80.9,
+    ("fp64", 0, 1, 512): 79.4,
+    ("fp64", 0, 2, 512): 87.3,
+    ("fp64", 1, 0, 512): 77.2,
+    ("fp64", 1, 1, 512): 78.1,
+    ("fp64", 1, 2, 512): 81.8,
+    ("fp64", 2, 0, 512): 83.8,
+    ("fp64", 2, 1, 512): 80.4,
+    ("fp64", 2, 2, 512): 81.5,
 }
 KERNEL_NAMES = {0: "sweep_kernel<0> (x)", 1: "sweep_kernel<1> (y)", 2: "sweep_kernel<2> (z, with update)",
                 3: "cfl reduction", 4: "spline prefilter (u, v, w)", 5: "particle sample + Heun",

@@ -55,8 +55,8 @@ constexpr int kTiles[3][kTileVariants][3] = {
     {{16, 4, 4}, {4, 8, 8}, {8, 8, 4}},
 };
 // FP64 shapes: 128 faces, two threads each (gkm_pair.hpp).  The first of each
-// direction is the fastest or within 1 % of it at 64^3 and 256^3 (256^3: x 1.92-
-// 1.97, y 1.96-2.02, z 2.05-2.21 ms over the three).
+// direction is the fastest or within 1 % of it at 64^3 and 256^3 (256^3: x 1.97-
+// 2.01, y 2.01-2.07, z 2.13-2.32 ms over the three).
 constexpr int kTilesPair[3][kTileVariants][3] = {
     {{2, 8, 8}, {1, 8, 16}, {2, 4, 16}},
     {{2, 8, 8}, {1, 8, 16}, {2, 4, 16}},
@@ -112,7 +112,8 @@ hipError_t launch_set_scalar(double* p, double v, hipStream_t s);
 // 2907, 256^3 6470 / 5997; mixed: 32^3 30 / 72, 64^3 119 / 166, 96^3 343 / 466, 128^3
 // 765 / 856, 192^3 2635 / 2963, 240^3 5153 / 5806, 256^3 6290 / 6410, 384^3 21470 /
 // 21330.  Each line lies where the fluxes' round trip through memory (and the
-// 10 planes more it holds) begins to outweigh the lead-in chunks and the three
+// memory for them: of their 10 planes past dW a context's staging area covers 5.4
+// at 256^3, 7 at 64^3) begins to outweigh the lead-in chunks and the three
 // launches' ends.  Mixed: even grids only, since the x and y sweeps reconstruct
 // faces in pairs whose two members round differently, and a segment moved back
 // by an odd number of faces would change the pairs.

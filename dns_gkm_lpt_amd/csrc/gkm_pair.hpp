@@ -22,7 +22,7 @@
 // 1075 VALU instructions per lane against 2030 for a face in one lane, and
 // nothing spilled (215-235 VGPRs in the sweeps).  With the difference form of
 // WENO (gkm_math.hpp) and the ring of cells (gkm_sweep.hpp), 256^3 x / y / z
-// sweep: 2.63 / 2.98 / 3.18 -> 1.88 / 1.91 / 2.01 ms.  Built for three waves per
+// sweep: 2.63 / 2.98 / 3.18 -> 1.98 / 2.01 / 2.13 ms.  Built for three waves per
 // SIMD (168 VGPRs) it spills 32-40 registers and the sweeps slow by a fifth.
 //
 // The building blocks (rest frames, moments, slopes) are gkm_flux.hpp's.  The

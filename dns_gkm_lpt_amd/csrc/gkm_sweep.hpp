@@ -255,8 +255,7 @@ __device__ __forceinline__ void weno_chunk(const SweepArgs& p, int n0, int a0, i
 // line; they are loaded into registers before the flux of the chunk before and
 // stored in the ring after it, so HBM and L2 latency pass behind the flux.
 // (Reading each stencil from the state array took 30 loads and 6 temperatures
-// per face and line where this takes 5 and 1: 256^3, x / y / z sweep 2.44 / 2.54
-// / 2.56 -> 1.95 / 2.07 / 2.17 ms.)
+// per face and line where this takes 5 and 1, and the 256^3 sweeps a fifth longer.)
 template <int CN>
 constexpr int kRing = CN + 5;
 template <int DIR, int CN, int L>
