@@ -113,7 +113,7 @@ hipError_t launch_set_scalar(double* p, double v, hipStream_t s);
 // 765 / 856, 192^3 2635 / 2963, 240^3 5153 / 5806, 256^3 6290 / 6410, 384^3 21470 /
 // 21330.  Each line lies where the fluxes' round trip through memory (and the
 // memory for them: of their 10 planes past dW a context's staging area covers 5.4
-// at 256^3, 7 at 64^3) begins to outweigh the lead-in chunks and the three
+// at 256^3, 6.5 at 64^3) begins to outweigh the lead-in chunks and the three
 // launches' ends.  Mixed: even grids only, since the x and y sweeps reconstruct
 // faces in pairs whose two members round differently, and a segment moved back
 // by an odd number of faces would change the pairs.

@@ -208,7 +208,9 @@ __host__ __device__ constexpr int pair_slot(int side, int v)
 // a face alone (512^3, 4 x 4 x 16 and 2 x 8 x 16 tiles: x 15.66 -> 14.45 ms,
 // y 17.17 -> 16.42 ms).  The z sweep keeps one face per thread: with pairs,
 // neighbouring lanes read cells two apart along z and it slowed (19.25 ->
-// 20.16 ms).
+// 20.16 ms); its temperatures are formed after all its loads (formed one by one
+// with them, as the pairs' are, the z sweep takes 217 us instead of 209 at 100^3 and
+// 692 instead of 672 at 160^3).
 template <int DIR, int CN, int CA, int CB, int NT>
 __device__ __forceinline__ void weno_chunk(const SweepArgs& p, int n0, int a0, int b0, int tid, double* sW)
 {
@@ -234,12 +236,13 @@ __device__ __forceinline__ void weno_chunk(const SweepArgs& p, int n0, int a0, i
             const long idx = cell_index<DIR>(wrapi(fn - 2 + t, nc), ca, cb, nc);
 #pragma unroll
             for (int q = 0; q < 5; q++) S[t][q] = W[q * plane + idx];
-            Tc[t] = temp_gr<double>(S[t], gR);
+            if (NH == 2) Tc[t] = temp_gr<double>(S[t], gR);
         }
 #pragma unroll
         for (int h = 0; h < NH; h++) {
             double Wl[5], Wr[5];
-            weno5_mixed_t(S + h, Tc + h, p.g, Wl, Wr);
+            if constexpr (NH == 2) weno5_mixed_t(S + h, Tc + h, p.g, Wl, Wr);
+            else weno5_mixed(S, p.g, Wl, Wr);
 #pragma unroll
             for (int q = 0; q < 5; q++) {
                 sW[sw_at<DIR, CN, L>(q, itn + h, il)] = Wl[q];
