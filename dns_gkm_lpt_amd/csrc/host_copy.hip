@@ -131,7 +131,7 @@ hipError_t HostPipe::plain(const CopySeg* seg, int n, hipStream_t s, bool to_hos
                                      : hipMemcpyAsync(seg[i].dev, seg[i].host, seg[i].bytes, hipMemcpyHostToDevice, s);
         if (e != hipSuccess) return e;
     }
-    return hipStreamSynchronize(s);
+    return to_host ? hipStreamSynchronize(s) : hipSuccess;
 }
 
 hipError_t HostPipe::run(const CopySeg* seg, int n, hipStream_t s, bool to_host)

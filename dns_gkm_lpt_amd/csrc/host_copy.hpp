@@ -18,8 +18,9 @@ struct CopySeg {
 // uses them and freed by release().
 class HostPipe {
   public:
-    // enqueue and finish the copies of n segments after the work on s; returns
-    // when the last byte has arrived
+    // the copies of n segments after the work on s.  to_host returns when the last
+    // byte has arrived.  to_device may leave a small copy queued: whoever owns the
+    // memory waits for s before its caller gets it back.
     hipError_t to_host(const CopySeg* seg, int n, hipStream_t s) { return run(seg, n, s, true); }
     hipError_t to_device(const CopySeg* seg, int n, hipStream_t s) { return run(seg, n, s, false); }
     void release();
