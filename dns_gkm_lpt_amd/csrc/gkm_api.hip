@@ -913,22 +913,25 @@ int lpt_upload(gkm_ctx* c, long np, const double* pos)
     const double twopi = 2.0 * (std::atan(1.0) * 4.0);
     for (long p = 0; p < 3 * np; p++)
         if (!(pos[p] >= 0.0 && pos[p] <= twopi)) return fail(c, GKM_EINVAL, "particle position outside [0, 2 pi]");
-    for (void* ptr : {(void*)L.pos, (void*)L.U, (void*)L.G, (void*)L.tag, (void*)L.tag2, (void*)L.pos2, (void*)L.keys,
-                      (void*)L.perm, L.sort_tmp, (void*)L.props})
-        (void)hipFree(ptr);
-    L.pos = L.U = L.G = L.pos2 = L.props = nullptr;
-    L.tag = L.tag2 = L.perm = nullptr;
-    L.keys = nullptr;
-    L.sort_tmp = nullptr;
-    L.sort_tmp_bytes = 0;
-    L.np = np;
     L.sampled = false;
-    if (np == 0) return GKM_OK;
-    if (hipMalloc(&L.pos, sizeof(double) * 3 * np) != hipSuccess || hipMalloc(&L.U, sizeof(double) * 3 * np) != hipSuccess ||
-        hipMalloc(&L.G, sizeof(double) * 9 * np) != hipSuccess || hipMalloc(&L.pos2, sizeof(double) * 9 * np) != hipSuccess ||
-        hipMalloc(&L.tag, sizeof(int) * np) != hipSuccess || hipMalloc(&L.tag2, sizeof(int) * np) != hipSuccess ||
-        hipMalloc(&L.keys, sizeof(unsigned) * 2 * np) != hipSuccess || hipMalloc(&L.perm, sizeof(int) * 2 * np) != hipSuccess)
-        return fail(c, GKM_ENOMEM, "hipMalloc particles");
+    if (np != L.np || np == 0) {  // as many tracers again take the arrays that are there
+        for (void* ptr : {(void*)L.pos, (void*)L.U, (void*)L.G, (void*)L.tag, (void*)L.tag2, (void*)L.pos2, (void*)L.keys,
+                          (void*)L.perm, L.sort_tmp, (void*)L.props})
+            (void)hipFree(ptr);
+        L.pos = L.U = L.G = L.pos2 = L.props = nullptr;
+        L.tag = L.tag2 = L.perm = nullptr;
+        L.keys = nullptr;
+        L.sort_tmp = nullptr;
+        L.sort_tmp_bytes = 0;
+        L.np = 0;
+        if (np == 0) return GKM_OK;
+        if (hipMalloc(&L.pos, sizeof(double) * 3 * np) != hipSuccess || hipMalloc(&L.U, sizeof(double) * 3 * np) != hipSuccess ||
+            hipMalloc(&L.G, sizeof(double) * 9 * np) != hipSuccess || hipMalloc(&L.pos2, sizeof(double) * 9 * np) != hipSuccess ||
+            hipMalloc(&L.tag, sizeof(int) * np) != hipSuccess || hipMalloc(&L.tag2, sizeof(int) * np) != hipSuccess ||
+            hipMalloc(&L.keys, sizeof(unsigned) * 2 * np) != hipSuccess || hipMalloc(&L.perm, sizeof(int) * 2 * np) != hipSuccess)
+            return fail(c, GKM_ENOMEM, "hipMalloc particles");
+        L.np = np;
+    }
     std::vector<int> tags(np);
     for (long p = 0; p < np; p++) tags[p] = (int)p;
     std::vector<double> kept;
