@@ -164,20 +164,20 @@ hipError_t launch_prefilter_velocity(const double* W, long plane, double gam, co
 // weights are (1, 4, 1)/6 for the value and (1, -2, 1) delta^-2 for the second
 // derivative, so the Laplacian is a 27-point stencil on the coefficients.
 // The result lands at the knot positions of the coefficient box `lap`.
-// A thread walks kMarch knots of a column along the slowest axis and keeps the
+// A thread walks `march` knots of a column along the slowest axis and keeps the
 // two in-plane sums of three coefficient planes: 9 loads a knot where a knot by
 // itself takes 27, and no index divisions inside.  What is left is the box read
 // and written once (240^3: 177 -> 93 us,
 // 2.5 TB/s; 128^3: 28 -> 18).
-constexpr int kMarch = 16;
-__global__ __launch_bounds__(256) void lap_knots_kernel(const double* __restrict__ c, Geom g, double* __restrict__ lap)
+__global__ __launch_bounds__(256) void lap_knots_kernel(const double* __restrict__ c, Geom g, int march,
+                                                        double* __restrict__ lap)
 {
     const int nt = g.nt;
     const unsigned col = blockIdx.x * 256u + threadIdx.x;
     if (col >= (unsigned)nt * (unsigned)nt) return;
     const long N = g.N;
     const int b = (int)(col / (unsigned)nt), k = (int)(col - (unsigned)b * nt);
-    const int a0 = blockIdx.y * kMarch, a1 = a0 + kMarch < nt ? a0 + kMarch : nt;
+    const int a0 = blockIdx.y * march, a1 = a0 + march < nt ? a0 + march : nt;
     const double w[3] = {1.0 / 6.0, 4.0 / 6.0, 1.0 / 6.0}, d2[3] = {1.0, -2.0, 1.0};
     const double scale = g.dinv * g.dinv;
     const double* at = c + ((long)a0 * N + b) * N + k;
@@ -208,11 +208,23 @@ __global__ __launch_bounds__(256) void lap_knots_kernel(const double* __restrict
     }
 }
 
+// Cells a thread of the marching kernels walks on a cube of n^3: 16, or as few as
+// leave two workgroups per CU, since on small grids the walk is a chain of loads
+// with most of the chip idle (32^3: statistics 26.9 us with 16, 10.0 with 1; a cell a
+// thread without the walk took 9.5; Laplacian 7.0, 3.0 and 3.1).
+static int march_of(int n)
+{
+    int m = 16;
+    while (m > 1 && (long)blocks_for((long)n * n, 256) * blocks_for(n, m) < 512) m /= 2;
+    return m;
+}
+
 hipError_t launch_lap_spline(const double* c, const Geom& g, const double* pivots, double* lap, hipStream_t s)
 {
     if (c == lap || g.nt != g.nc + 6 || g.N != g.nt + 2 || !z_chunks(g.nt)) return hipErrorInvalidValue;
-    const dim3 grid(blocks_for((long)g.nt * g.nt, 256), blocks_for(g.nt, kMarch));
-    hipLaunchKernelGGL(lap_knots_kernel, grid, dim3(256), 0, s, c, g, lap);
+    const int march = march_of(g.nt);
+    const dim3 grid(blocks_for((long)g.nt * g.nt, 256), blocks_for(g.nt, march));
+    hipLaunchKernelGGL(lap_knots_kernel, grid, dim3(256), 0, s, c, g, march, lap);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     e = with_chunks(z_chunks(g.nt), [&](auto k) {
@@ -497,7 +509,7 @@ __device__ __forceinline__ void block_sum(double (&v)[K], double* out)
 
 __global__ __launch_bounds__(256) void stats_kernel(const double* __restrict__ W, long plane, const double* __restrict__ cu,
                                                     const double* __restrict__ cv, const double* __restrict__ cw, Geom g,
-                                                    StatParams sp, double* __restrict__ red)
+                                                    StatParams sp, int march, double* __restrict__ red)
 {
     // sums: 0 tke, 1 diss, 2 sijsij, 3 enstrophy, 4-6 d2, 7-9 d3, 10-12 d4, 13 P, 14 T, 15 1/rho
     double acc[16];
@@ -508,19 +520,19 @@ __global__ __launch_bounds__(256) void stats_kernel(const double* __restrict__ W
     const double w0 = 1.0 / 6.0, w1 = 4.0 / 6.0;
     const double d = 0.5 * g.dinv;
     const double* cs[3] = {cu, cv, cw};
-    // A block takes 256 columns along y, kMarch cells of them at a time, and a
+    // A block takes 256 columns along y, `march` cells of them at a time, and a
     // thread keeps three planes' in-plane sums of each field: 27 coefficient loads
     // a cell where a cell by itself takes 81.  With two or three waves per SIMD
     // the time was the loads' latency, once for the coefficients and once for the
     // state (240^3: 548 us, marching alone 562); the next cell's loads before this
     // one's arithmetic: 304 us, 128^3 81 -> 47.
     const unsigned cols = (unsigned)nc * (unsigned)nc, cblk = (cols + 255) / 256;
-    const unsigned items = cblk * (unsigned)((nc + kMarch - 1) / kMarch);
+    const unsigned items = cblk * (unsigned)((nc + march - 1) / march);
     for (unsigned it = blockIdx.x; it < items; it += gridDim.x) {
     const unsigned sg = it / cblk, col = (it - sg * cblk) * 256 + threadIdx.x;
     if (col >= cols) continue;
     const int i = (int)(col / (unsigned)nc), k = (int)(col - (unsigned)i * nc);
-    const int j0 = (int)sg * kMarch, j1 = j0 + kMarch < nc ? j0 + kMarch : nc;
+    const int j0 = (int)sg * march, j1 = j0 + march < nc ? j0 + march : nc;
     // knot (j+3, i+3, k+3): coefficient block starts at (j+3, i+3, k+3) with t = 0
     long at = ((long)(j0 + 3) * N + (i + 3)) * N + (k + 3);
     struct Plane {
@@ -628,7 +640,8 @@ __global__ __launch_bounds__(256) void stats2_kernel(const double* __restrict__ 
 hipError_t launch_stats(const double* W, long plane, const double* const cu[3], const Geom& g, const StatParams& sp,
                         double* red, hipStream_t s)
 {
-    hipLaunchKernelGGL(stats_kernel, dim3(kStatBlocks), dim3(256), 0, s, W, plane, cu[0], cu[1], cu[2], g, sp, red);
+    hipLaunchKernelGGL(stats_kernel, dim3(kStatBlocks), dim3(256), 0, s, W, plane, cu[0], cu[1], cu[2], g, sp,
+                       march_of(g.nc), red);
     return hipGetLastError();
 }
 
