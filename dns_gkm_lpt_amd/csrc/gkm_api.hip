@@ -48,6 +48,7 @@ struct gkm_ctx {
     double* dscal = nullptr;       // [0] dt, [1] vmax, [2] dt of lpt_heun, [3] the two ints of dflag
     int* dflag = nullptr;          // in dscal[3]: non-physical-state flag, ticket of the step's CFL
     double* hscal = nullptr;       // pinned copy of dscal
+    double* hred = nullptr;        // pinned copy of the statistics' block sums
     double* partial = nullptr;     // CFL block maxima
     double* faces = nullptr;       // face fluxes of the three directions (small grids), over dW and stage
     double* hist = nullptr;        // behind dscal: dt of the last kHist steps of gkm_run
@@ -166,21 +167,26 @@ int eulerian_step(gkm_ctx* c)
     return GKM_OK;
 }
 
+// *p: n pinned doubles of the context, made on first use
+int pinned(gkm_ctx* c, double** p, size_t n)
+{
+    if (*p) return GKM_OK;
+    int was = c->cfg.device;  // the caller may have another device current
+    HIPCHK(c, hipGetDevice(&was));
+    HIPCHK(c, hipSetDevice(c->cfg.device));
+    const hipError_t e = hipHostMalloc(reinterpret_cast<void**>(p), sizeof(double) * n, hipHostMallocDefault);
+    (void)hipSetDevice(was);
+    if (e == hipSuccess) return GKM_OK;
+    *p = nullptr;
+    return fail(c, GKM_ENOMEM, "hipHostMalloc");
+}
+
 // dscal into hscal once the stream's work is done; an error if the CFL pass saw
 // a non-physical state
 int read_scalars(gkm_ctx* c)
 {
-    if (!c->hscal) {
-        int was = c->cfg.device;  // the caller may have another device current
-        HIPCHK(c, hipGetDevice(&was));
-        HIPCHK(c, hipSetDevice(c->cfg.device));
-        const hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&c->hscal), sizeof(double) * kScal, hipHostMallocDefault);
-        (void)hipSetDevice(was);
-        if (e != hipSuccess) {
-            c->hscal = nullptr;
-            return fail(c, GKM_ENOMEM, "hipHostMalloc scalars");
-        }
-    }
+    const int rc = pinned(c, &c->hscal, kScal);
+    if (rc) return rc;
     HIPCHK(c, hipMemcpyAsync(c->hscal, c->dscal, sizeof(double) * kScal, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     if (*reinterpret_cast<const int*>(c->hscal + 3) && c->cfg.check_state)
@@ -308,6 +314,7 @@ void gkm_destroy(gkm_ctx* c)
     (void)hipFree(c->slab);
     (void)hipFree(c->cmp_own);
     (void)hipHostFree(c->hscal);
+    (void)hipHostFree(c->hred);
     if (c->ev[0]) (void)hipEventDestroy(c->ev[0]);
     if (c->ev[1]) (void)hipEventDestroy(c->ev[1]);
     if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -851,12 +858,14 @@ int ensure_spline(gkm_ctx* c)
 
 int sum_partials(gkm_ctx* c, int stride, int off, int K, double* out)
 {
-    std::vector<double> h((size_t)stride * lpt::kStatBlocks);
-    HIPCHK(c, hipMemcpyAsync(h.data(), c->lpt.red, sizeof(double) * h.size(), hipMemcpyDeviceToHost, c->stream));
+    const int rc = pinned(c, &c->hred, (size_t)32 * lpt::kStatBlocks);
+    if (rc) return rc;
+    HIPCHK(c, hipMemcpyAsync(c->hred, c->lpt.red, sizeof(double) * stride * lpt::kStatBlocks, hipMemcpyDeviceToHost,
+                             c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     for (int k = 0; k < K; k++) {
         double s = 0.0;
-        for (int b = 0; b < lpt::kStatBlocks; b++) s += h[(size_t)b * stride + off + k];
+        for (int b = 0; b < lpt::kStatBlocks; b++) s += c->hred[(size_t)b * stride + off + k];
         out[k] = s;
     }
     return GKM_OK;
