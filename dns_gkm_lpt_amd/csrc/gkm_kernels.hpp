@@ -107,16 +107,17 @@ hipError_t launch_set_scalar(double* p, double v, hipStream_t s);
 // directions, then the update (compensated with cmp_out) and, with cfl, the dt of
 // the new state.  F holds 15 plane doubles, slots as in sweep_seg_len.  Equal to
 // the three sweeps with their first tile variants bit for bit.  us per step with
-// dt, this / the sweeps and the CFL pass, FP64: 32^3 29 / 49, 64^3 125 / 151, 96^3
-// 345 / 427, 128^3 770 / 790, 160^3 1527 / 1660, 176^3 2079 / 2090, 200^3 3057 /
-// 2907, 256^3 6470 / 5997; mixed: 32^3 30 / 72, 64^3 119 / 166, 96^3 343 / 466, 128^3
-// 765 / 856, 192^3 2635 / 2963, 240^3 5153 / 5806, 256^3 6290 / 6410, 384^3 21470 /
-// 21330.  Each line lies where the fluxes' round trip through memory (and the
-// memory for them: of their 10 planes past dW a context's staging area covers 5.4
-// at 256^3, 6.5 at 64^3) begins to outweigh the lead-in chunks and the three
-// launches' ends.  Mixed: even grids only, since the x and y sweeps reconstruct
-// faces in pairs whose two members round differently, and a segment moved back
-// by an odd number of faces would change the pairs.
+// dt, this / those sweeps and the CFL pass, FP64: 32^3 26 / 49, 64^3 112 / 147, 96^3
+// 340 / 430, 128^3 782 / 795, 160^3 1553 / 1657, and from an earlier build 176^3
+// 2079 / 2090, 200^3 3057 / 2907, 256^3 6470 / 5997; mixed: 32^3 29 / 73, 64^3 110 /
+// 164, 96^3 338 / 465, 128^3 758 / 859, 192^3 2614 / 2945, 240^3 5125 / 5788, 256^3
+// 6241 / 6387, and from an earlier build 384^3 21470 / 21330.  Each line lies where
+// the fluxes' round trip through memory (and the memory for them: of their 10
+// planes past dW a context's staging area covers 5.4 at 256^3, 6.5 at 64^3) begins to
+// outweigh the lead-in chunks and the three launches' ends.  Mixed: even grids only,
+// since the x and y sweeps reconstruct faces in pairs whose two members round
+// differently, and a segment moved back by an odd number of faces would change the
+// pairs.
 constexpr int kSmallNc = 160, kSmallNcMixed = 256;
 bool small_step_ok(int nc, bool mixed);
 struct StepCfl {
