@@ -247,7 +247,7 @@ hipError_t launch_lap_spline(const double* c, const Geom& g, const double* pivot
 // at 12.8 / 14.9 GiB.
 __device__ __forceinline__ unsigned xcd_block()
 {
-    const unsigned b = blockIdx.x, nb = gridDim.x;
+    const unsigned b = blockIdx.y * gridDim.x + blockIdx.x, nb = gridDim.x * gridDim.y;  // thread_grid
     return (nb & 7) ? b : (b & 7) * (nb >> 3) + (b >> 3);
 }
 
@@ -273,7 +273,7 @@ hipError_t launch_sample(long np, const double* pos, const double* const cu[3], 
                          hipStream_t s)
 {
     if (np <= 0) return hipSuccess;
-    hipLaunchKernelGGL(sample_kernel, dim3(blocks_for(4 * np, 256)), dim3(256), kSampleLdsCap, s, np, pos, cu[0], cu[1],
+    hipLaunchKernelGGL(sample_kernel, thread_grid(4 * np), dim3(256), kSampleLdsCap, s, np, pos, cu[0], cu[1],
                        cu[2], g, U, G);
     return hipGetLastError();
 }
@@ -392,7 +392,7 @@ hipError_t launch_heun(long np, double* pos, const double* U, const double* cons
                        const double* dt, hipStream_t s)
 {
     if (np <= 0) return hipSuccess;
-    hipLaunchKernelGGL(heun_kernel, dim3(blocks_for(4 * np, 256)), dim3(256), kHeunLdsCap, s, np, pos, U, cn[0], cn[1],
+    hipLaunchKernelGGL(heun_kernel, thread_grid(4 * np), dim3(256), kHeunLdsCap, s, np, pos, U, cn[0], cn[1],
                        cn[2], g, dt);
     return hipGetLastError();
 }

@@ -1,5 +1,5 @@
 """Launch grids of the tracer kernels with several threads per tracer, on the host:
-from one tracer to the 2^31 - 1 an upload accepts, with 4 threads (properties) and 9
+from one tracer to the 2^31 - 1 an upload accepts, with 4 threads (samples, Heun, properties) and 9
 (gradient rows scattered to upload order) each.  One axis of 2^24 blocks of 256 is
 refused by the runtime, and 2^24 + 8 run as 8."""
 import os
