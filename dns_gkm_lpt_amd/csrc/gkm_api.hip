@@ -256,10 +256,10 @@ int create(const gkm_config* cfg, bool two_launch, gkm_ctx** out)
         for (size_t n : sizes) total += n;
         return hipMalloc(&c->slab, sizeof(double) * total) == hipSuccess;
     };
-    two_launch = two_launch && gkm::small_step_ok(nc, mixed);
-    if (!two_launch || !allocate()) {
-        (void)hipGetLastError();
-        two_launch = false;
+    const bool wanted = two_launch && gkm::small_step_ok(nc, mixed);
+    two_launch = wanted && allocate();
+    if (!two_launch) {
+        if (wanted) (void)hipGetLastError();  // of the attempt with the fluxes
         sizes[2] = work;
         if (!allocate()) return fail(c, GKM_ENOMEM, "hipMalloc state");
     }
